@@ -5,7 +5,12 @@
 // of head h attends keys j <= i + (L - S) of KV head h / (Hq/Hkv); with RoPE-Llama both
 // q and k (at position j + k_rope_pos_offset) are rotated in the kernel.
 //
-// Kernel design (one workgroup = 4 wave64s = 128 query rows of one head):
+// Three kernels: the split kernel (attn_split.hpp: few 32-row blocks, head_dim 64, RoPE
+// inside), the pipelined kernel below (head_dim 128, rotated keys, many rows), and this
+// register-staged one for rows that are not 16-byte aligned, which the tests also use as
+// the others' reference.
+//
+// Register-staged kernel (one workgroup = 4 wave64s = 128 query rows of one head):
 //  * Scores are computed transposed, S^T = K . Q^T, with v_mfma_f32_32x32x16_bf16: the
 //    K tile is the A operand (read from LDS), the wave's 32 query rows are the B operand
 //    held in registers for the whole kernel. Each lane then owns one query row and 16
@@ -19,6 +24,7 @@
 //    are loaded together by one thread before the LDS store.
 //  * Causal tiles past the diagonal are skipped; late query tiles are scheduled first.
 #include "attn_pipe.hpp"
+#include "attn_split.hpp"
 #include "common.hpp"
 
 #include <algorithm>
@@ -27,33 +33,9 @@
 
 namespace efm {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
 constexpr int kPfThreads = 256;
 constexpr int kPfQ = 128;   // query rows per workgroup (32 per wave)
 constexpr int kPfKV = 64;   // keys per LDS tile
-
-struct PrefillArgs {
-    const bf16_t* q;
-    const bf16_t* k;
-    const bf16_t* v;
-    bf16_t* o;
-    int S, L, Hq, Hkv;
-    int q_sn, q_sh, k_sn, k_sh, v_sn, v_sh;
-    int o_sn, o_sh;
-    int causal;
-    int rope_q, rope_k;
-    int q_pos_off, k_pos_off;
-    float sm_scale_log2;
-    RopeTable rope;
-};
-
-union Pack8 {
-    bf16x8_t v;
-    uint4 u;
-    uint32_t w[4];
-};
 
 template <int HD>
 __global__ __launch_bounds__(kPfThreads) void prefill_attn_kernel(PrefillArgs a) {
@@ -285,15 +267,6 @@ constexpr int kP2HD = 128;
 constexpr int kP2Row = kP2HD * 2;  // bytes per K / V row in LDS
 constexpr int kP2Tile = kP2KV * kP2Row;
 constexpr int kP2Stage = 2 * kP2Tile;
-constexpr float kP2Lazy = 8.0f;
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
-// Sum of the two bf16 halves of `w` added to acc (fp32).
-__device__ __forceinline__ float add_bf16_pair(uint32_t w, float acc) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w),
-                                           __builtin_bit_cast(bf16x2_t, 0x3f803f80u), acc, false);
-}
 
 // Waves per SIMD the register allocation aims for: 8 / WAVES, but never more than the
 // LDS ring lets reside (S stages of kP2Stage bytes out of 160 KB per CU, four SIMDs).
@@ -619,7 +592,7 @@ __global__ __launch_bounds__(WAVES * 64, pipe_waves_per_eu(WAVES, S)) void prefi
 int validate_attention_ctx(const efm_attention_ctx* c, const char* who);
 
 // EFM_KNOB_PREFILL_REGISTER selects the register-staged kernel (kept as the reference
-// path of the pipelined one in the tests).
+// path of the split and pipelined ones in the tests).
 static bool prefill_pipe_enabled() { return kernel_knob(EFM_KNOB_PREFILL_REGISTER) == 0; }
 
 int prefill_cus() {
@@ -632,6 +605,52 @@ int prefill_cus() {
         cached[dev] = n;
     }
     return cached[dev];
+}
+
+// Whether a head_dim-128 launch over rotated keys splits its keys over waves (attn_split.hpp)
+// or streams shared tiles. The shared stream reads each K / V byte once per 128 or 256 rows
+// and is the faster one once the chip is full; the split pays while 32-row blocks are few.
+// Measured on 256 CUs (us, split / shared; blocks = 32-row blocks of all heads, keys = mean
+// keys a row sees): 24 blocks x 2018 keys 15.8 / 43.1; 192 x 256 8.9 / 15.6; 672 x 672
+// 22.0 / 30.6; 1020 x 1350 43.8 / 58.0; 752 x 3500 70.0 / 75.1; 896 x 8500 183.9 / 181.6;
+// 1536 x 2048 80.6 / 95.5; 1764 x 1000 51.0 / 53.8; 3584 x 2048 170 / 128.
+static bool prefill_split_wins(const PrefillArgs& a, int cus) {
+    const long blocks = (long)((a.S + 31) / 32) * a.Hq;
+    const long keys = a.causal ? a.L - a.S / 2 : a.L;
+    if (blocks <= 3L * cus) return true;
+    if (blocks <= 4L * cus) return keys <= 4096;
+    return blocks <= 7L * cus && keys <= 2048;
+}
+
+// Waves per 32-row block: 8 (one workgroup per CU) while there is a CU for every block and
+// the keys are worth it, else 4 (two per CU), and 2 for many blocks where the chain is short
+// (head_dim 128, rotated keys). Measured (us, 8 / 4 / 2 waves): 24 blocks x 2018 keys 15.8 /
+// 19.2 / 33.5; 224 x 8128 50.8 / 65.8 / 124; 192 x 256 9.3 / 8.9 / 11.8; 384 x 512 16.1 /
+// 14.0 / 19.9; 1316 x 750 51.5 / 36.0 / 33.6; head_dim 64, 308 x 350 9.5 / 7.4 / 9.8;
+// RoPE inside, 384 x 524 29.3 / 25.2 / 36.4, 2632 x 5000 730 / 626 / 660.
+static void prefill_split_launch(const PrefillArgs& a, int hd, int cus, hipStream_t stream) {
+    const int nqt = (a.S + 31) / 32;
+    const long blocks = (long)nqt * a.Hq;
+    const bool eight = blocks <= cus && (2 * blocks <= cus || a.L >= 1024);
+    const dim3 grid = SplitGrid::dims(nqt, a.Hq, a.Hkv);
+    const SplitGrid sg = SplitGrid::of(a.Hq, a.Hkv);
+    auto launch = [&](auto kernel, int waves) {
+        hipLaunchKernelGGL(kernel, grid, dim3(waves * kWave), 0, stream, a, sg, nqt);
+    };
+    if (hd == 128 && a.rope_k) {
+        if (eight) launch(prefill_attn_split_kernel<128, 8, true>, 8);
+        else launch(prefill_attn_split_kernel<128, 4, true>, 4);
+    } else if (hd == 128) {
+        if (eight) launch(prefill_attn_split_kernel<128, 8, false>, 8);
+        else if (blocks <= 5L * cus) launch(prefill_attn_split_kernel<128, 4, false>, 4);
+        else launch(prefill_attn_split_kernel<128, 2, false>, 2);
+    } else if (a.rope_k) {
+        if (eight) launch(prefill_attn_split_kernel<64, 8, true>, 8);
+        else launch(prefill_attn_split_kernel<64, 4, true>, 4);
+    } else {
+        if (eight) launch(prefill_attn_split_kernel<64, 8, false>, 8);
+        else launch(prefill_attn_split_kernel<64, 4, false>, 4);
+    }
 }
 
 }  // namespace efm
@@ -675,16 +694,25 @@ extern "C" int efm_attention_prefill(const efm_attention_ctx* ctx, const void* q
     a.k_pos_off = (int)ctx->k_rope_pos_offset;
     rope_table_fill(&a.rope, hd, ctx->rope_theta, ctx->rope_scale);
     a.sm_scale_log2 = 1.4426950408889634f / sqrtf((float)hd);
-    if (hd == kP2HD && !a.rope_k && prefill_pipe_enabled()) {
+    const int cus = prefill_cus();
+    const int knob = kernel_knob(EFM_KNOB_PREFILL_SHAPE);
+    const bool pipe_ok = hd == kP2HD && !a.rope_k;
+    // the split kernel's tile loads take 16-byte aligned rows and 32-bit offsets inside a
+    // tile, its grid 32-row blocks: anything else stays with the kernels below
+    const bool split_ok = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                            reinterpret_cast<uintptr_t>(v)) & 15u) == 0 &&
+                          std::max(ctx->k_stride_n, ctx->kv_stride_n) < (1u << 24) &&
+                          (long)((qo_len + 31) / 32) * a.Hq < (1L << 22);
+    if (prefill_pipe_enabled() && split_ok && (pipe_ok ? knob == 0 && prefill_split_wins(a, cus) : true)) {
+        prefill_split_launch(a, hd, cus, stream);
+        return check_launch("attention_prefill");
+    }
+    if (pipe_ok && prefill_pipe_enabled()) {
         // 8 waves (256 rows, 4-deep ring, one workgroup per CU) when those workgroups fill
-        // the chip; fewer rows: 4 waves (128 rows) over a 2-deep ring, two workgroups per
-        // CU (twice the workgroups). Measured (causal, no prefix): 12/2 heads S 256 / 512 /
-        // 2048: 10.7 / 15.9 / 46.0 us with 4 waves against 11.4 / 18.2 / 62.8 with the
-        // 2-wave (64-row) kernel and 12.5 / 19.2 / 58.7 with 8 waves; 16/2 S 1344: 31.2
-        // against 42.9 / 38.7; 28/4 S 4096: 151.4 against 237.4 / 146.2. The 2-wave kernel
-        // stays for EFM_KNOB_PREFILL_SHAPE = 2 (2 / 4 / 8 force a shape).
-        const int knob = kernel_knob(EFM_KNOB_PREFILL_SHAPE);
-        const int cus = prefill_cus();
+        // the chip; fewer rows (behind a long prefix; without one the split kernel takes
+        // them): 4 waves (128 rows) over a 2-deep ring, two workgroups per CU. 28/4 heads,
+        // S 4096: 151.4 us with 4 waves, 146.2 with 8. EFM_KNOB_PREFILL_SHAPE = 2 / 4 / 8
+        // forces a shape (2: 64-row workgroups, for the tests).
         const int shape = knob != 0 ? knob : (int)((qo_len + 255) / 256) * a.Hq >= cus ? 8 : 4;
         if (shape == 2) {
             const int nqt = (int)((qo_len + 63) / 64);

@@ -63,9 +63,10 @@ int efm_init(void);
  * one it replaces on the same inputs. value 0 restores the library's own choice.
  *   EFM_KNOB_DECODE_REGISTER   1: decode attention (head_dim 128, rotated cache) runs the
  *                              register-staged kernel instead of the LDS-staged one
- *   EFM_KNOB_PREFILL_REGISTER  1: prefill and Sage attention (head_dim 128) run the
- *                              register-staged kernels instead of the pipelined ones
- *   EFM_KNOB_PREFILL_SHAPE     4 or 8: the pipelined prefill / Sage kernels run with
+ *   EFM_KNOB_PREFILL_REGISTER  1: prefill and Sage attention run the register-staged
+ *                              kernels instead of the split and pipelined ones
+ *   EFM_KNOB_PREFILL_SHAPE     4 or 8: the pipelined prefill / Sage kernels run (for
+ *                              prefill in place of the split kernel too) with
  *                              4-wave (128-row) or 8-wave (256-row) workgroups; 2: the
  *                              prefill kernel runs 2-wave (64-row) workgroups (the Sage
  *                              kernel treats 2 as 4)

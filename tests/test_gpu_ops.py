@@ -1160,6 +1160,75 @@ def test_attention_prefill_pipelined_matches_register_kernel_c4(gpu, knob, shape
         assert_close_bf16(outs[0][r].reshape(1, hq, hd), ref, rtol=2e-2, atol=2e-2, what=f"C4 row {r} vs oracle")
 
 
+SPLIT_CASES = [
+    # hq, hkv, hd, S, L, causal, rope: tile and block edges, one key, one row behind a prefix,
+    # every wave count (8, 4, 2), grids by XCD (1, 2, 4, 8 KV heads) and plain (3)
+    pytest.param(12, 2, 128, 1, 1, 1, "none", id="one_key"),
+    pytest.param(12, 2, 128, 32, 32, 1, "none", id="one_block"),
+    pytest.param(12, 2, 128, 33, 2050, 1, "read", id="eight_waves_rope"),
+    pytest.param(28, 4, 128, 1, 8193, 1, "prerot", id="row_behind_8k"),
+    pytest.param(6, 3, 128, 65, 161, 1, "none", id="plain_grid"),
+    pytest.param(8, 8, 128, 900, 900, 1, "read", id="four_waves_8_kv_heads"),
+    pytest.param(28, 4, 128, 1472, 1475, 1, "prerot", id="two_waves"),
+    pytest.param(12, 2, 128, 130, 97 + 130, 0, "read", id="noncausal_rope"),
+    pytest.param(14, 2, 64, 1, 1, 1, "read", id="hd64_one_key"),
+    pytest.param(14, 2, 64, 31, 95, 1, "none", id="hd64_half_tile"),
+    pytest.param(14, 2, 64, 19, 1531, 1, "prerot", id="hd64_eight_waves"),
+    pytest.param(7, 1, 64, 1200, 1200, 1, "read", id="hd64_four_waves_rope"),
+    pytest.param(16, 8, 64, 97, 128, 0, "none", id="hd64_noncausal"),
+]
+
+
+@pytest.mark.parametrize("hq,hkv,hd,S,L,causal,mode", SPLIT_CASES)
+def test_attention_prefill_split_matches_oracle(gpu, knob, hq, hkv, hd, S, L, causal, mode):
+    """The kernel that splits a 32-row block's keys over the waves of a workgroup, against
+    the oracle and the register-staged kernel, on strided q, k and v (a padded row each)."""
+    torch.manual_seed(S + L + hd)
+    q = torch.randn(S, hq, hd, dtype=torch.bfloat16)
+    k = torch.randn(L, hkv, hd, dtype=torch.bfloat16)
+    v = torch.randn(L, hkv, hd, dtype=torch.bfloat16)
+    octx = O.AttnCtx(hq, hkv, hd, rope=mode != "none", q_rope_pos_offset=L - S)
+    ref = O.attention(q, k, v, torch.arange(S) + (L - S), octx, causal_offset=(L - S) if causal else None)
+    kin = O.rope_llama(k, torch.arange(L), 1.0e6).to(torch.bfloat16) if mode == "prerot" else k
+
+    def padded(t, extra):   # rows of t with `extra` elements of NaN behind each
+        rows = torch.full((t.shape[0], t.shape[1] * hd + extra), float("nan"), dtype=torch.bfloat16)
+        rows[:, : t.shape[1] * hd] = t.reshape(t.shape[0], -1)
+        return rows.to(gpu)
+
+    qg, kg, vg = padded(q, 8), padded(kin, 16), padded(v, 24)
+    ctx = C.make_attention_ctx(hq, hkv, hd, rope=mode != "none", q_rope_pos_offset=L - S,
+                               k_already_prerotated=mode == "prerot", q_stride_n=hq * hd + 8, q_stride_h=hd,
+                               k_stride_n=hkv * hd + 16, k_stride_h=hd, kv_stride_n=hkv * hd + 24, kv_stride_h=hd)
+    outs = []
+    for register in (0, 1):
+        knob(C.EFM_KNOB_PREFILL_REGISTER, register)
+        o = torch.full((S + 1, hq * hd), -7.0, dtype=torch.bfloat16, device=gpu)
+        C.call("efm_attention_prefill", ctx, ptr(qg), ptr(kg), ptr(vg), ptr(o), S, L, causal, stream())
+        torch.cuda.synchronize()
+        assert (o[S] == -7.0).all()
+        outs.append(o[:S].reshape(S, hq, hd))
+    # P is rounded to bf16 before the PV product
+    assert_close_bf16(outs[0], ref, rtol=2e-2, atol=2e-2, what="split vs oracle")
+    assert_close_bf16(outs[0], outs[1], rtol=2e-2, atol=2e-2, what="split vs register-staged")
+
+
+def test_attention_prefill_unaligned_rows(gpu):
+    """head_dim 64 rows at an 8-byte (not 16-byte) aligned address: accepted as before."""
+    torch.manual_seed(5)
+    hq, hkv, hd, S = 14, 2, 64, 70
+    q, k, v = (torch.randn(S, h, hd, dtype=torch.bfloat16) for h in (hq, hkv, hkv))
+    off = [torch.zeros(t.numel() + 4, dtype=torch.bfloat16, device=gpu) for t in (q, k, v)]
+    for d, t in zip(off, (q, k, v)):
+        d[4:] = t.reshape(-1).to(gpu)
+    o = torch.empty(S, hq * hd, dtype=torch.bfloat16, device=gpu)
+    C.call("efm_attention_prefill", C.make_attention_ctx(hq, hkv, hd), *(d.data_ptr() + 8 for d in off), ptr(o), S, S, 1,
+           stream())
+    torch.cuda.synchronize()
+    ref = O.attention_prefill(q, k, v, O.AttnCtx(hq, hkv, hd), causal=True)
+    assert_close_bf16(o.reshape(S, hq, hd), ref, rtol=2e-2, atol=2e-2)
+
+
 def test_attention_prefill_last_row_equals_decode(gpu):
     """The last prefill row equals single-query decode over the same cache (the
     reference's prefill/decode consistency)."""
