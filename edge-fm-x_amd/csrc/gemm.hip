@@ -3,19 +3,22 @@
 // row per token) and B the weights in their [out, in] layout, so both operands are
 // K-contiguous and feed the MFMA lanes with 16-byte loads.
 //
-//  * K % 64 == 0 (every Qwen2.5 projection), two kernels fed by global_load_lds DMA into
+//  * K % 64 == 0 (every Qwen2.5 projection), kernels fed by global_load_lds DMA into
 //    XOR-swizzled LDS rings, operand reads software-pipelined against the MFMAs and a
 //    grouped tile order per XCD:
 //      - the wide kernel: 256 x 256 tiles, one 8-wave workgroup per CU (large M);
 //      - the pipelined kernel: 128 x 128 (128 x 64, 64 x 64) tiles, two 4-wave
 //        workgroups per CU (few tiles), plus its split-K form.
 //    A cost model (rounds of resident workgroups) picks between them.
+//  * The same K, few rows or few tiles: the K-split kernel, whose four waves take a quarter
+//    of K each over 32 x 32 to 64 x 64 tiles.
 //  * Other K: a register-staged kernel with a padded LDS row pitch (40 bf16).
 //  * Epilogues: bf16 (+bias, the cuBLASLt BIAS epilogue), fp32, and SwiGLU, where the
 //    B tile interleaves 32-row blocks of up and gate weights so that each lane holds u
 //    and g of the same output element: out = bf16(silu(bf16(g)) * bf16(u)).
 //  * Every kernel sums each output's keys 16 at a time in increasing order, so results
-//    are bit-identical across kernels and tile shapes (split-K aside).
+//    are bit-identical across kernels and tile shapes (K-split and split-K aside, which add
+//    the sums of contiguous ranges of K in order).
 #include "common.hpp"
 
 #include <algorithm>
@@ -223,16 +226,19 @@ __device__ __forceinline__ void vm_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Waits until at most `slabs` slabs of LPW loads are in flight (the counter holds 63: past
+// that the wait is for fewer).
+constexpr int vm_count(int loads) { return loads < 63 ? loads : 63; }
 template <int LPW>
 __device__ __forceinline__ void vm_wait_slabs(int slabs) {
     switch (slabs) {
         case 0: vm_wait<0>(); break;
-        case 1: vm_wait<1 * LPW>(); break;
-        case 2: vm_wait<2 * LPW>(); break;
-        case 3: vm_wait<3 * LPW>(); break;
-        case 4: vm_wait<4 * LPW>(); break;
-        case 5: vm_wait<5 * LPW>(); break;
-        default: vm_wait<6 * LPW>(); break;
+        case 1: vm_wait<vm_count(1 * LPW)>(); break;
+        case 2: vm_wait<vm_count(2 * LPW)>(); break;
+        case 3: vm_wait<vm_count(3 * LPW)>(); break;
+        case 4: vm_wait<vm_count(4 * LPW)>(); break;
+        case 5: vm_wait<vm_count(5 * LPW)>(); break;
+        default: vm_wait<vm_count(6 * LPW)>(); break;
     }
 }
 
@@ -688,8 +694,217 @@ __global__ __launch_bounds__(WGM * WGN * kWave, 1) void gemm_wide_kernel(const b
     }
 }
 
+// ---------------------------------------------------------------------------------
+// K split over the waves of a workgroup: for launches whose tiles are too few to keep the
+// CUs busy by themselves. The pipelined kernel's four waves share every slab, so one wave
+// runs a single 32 x 32 MFMA tile (64 x 64 workgroup tiles) between two barriers: 512 x
+// 1536 -> 2048 takes 24 slabs at 0.5 us. Here each of KW waves owns a contiguous range of
+// the slabs and the whole 32 TM x 32 TN tile, with an S-deep LDS ring of its own: no
+// barrier until the partial tiles are summed through LDS, in wave order.
+//  * A slab's operand reads are all issued one slab ahead of their MFMAs (two register
+//    sets); its LDS slot is refilled as soon as they have landed.
+//  * The weight rows are the MFMA's first operand, so a lane ends with four consecutive
+//    columns of one row: float4 partials, 16-byte output stores.
+//  * SwiGLU: the tile's first half of weight rows is up, the second gate.
+// ---------------------------------------------------------------------------------
+template <int TM, int TN>
+struct KsplitFrags {
+    bf16x8_t a[kPBK / 16][TM], b[kPBK / 16][TN];
+};
+
+template <int TM, int TN, int KW, int S, int EPI, int WPE>
+__global__ __launch_bounds__(KW * kWave, WPE) void gemm_ksplit_kernel(const bf16_t* __restrict__ A,
+                                                                 const bf16_t* __restrict__ B,
+                                                                 const bf16_t* __restrict__ bias,
+                                                                 void* __restrict__ Cout, int M, int N, int K, int ldc,
+                                                                 int mt, int nt, int vec, int kslices, int slice_slabs) {
+    constexpr int BM = 32 * TM, BN = 32 * TN, KSN = kPBK / 16;
+    constexpr int OC = EPI == GEPI_SWIGLU ? BN / 2 : BN;   // output columns per tile
+    constexpr int STAGE = (BM + BN) * kPRow, RING = S * STAGE;
+    constexpr int LA = BM / 8, LPS = (BM + BN) / 8;        // 1 KB wave loads per slab
+    constexpr int CH = BN / 4;                             // float4 chunks per partial row
+    static_assert(S >= 2 && S * LPS <= 63 && BM * BN * 4 <= RING, "bad K-split shape");
+    __shared__ __align__(1024) unsigned char smem[KW * RING];
+
+    // GEPI_PARTIAL: work unit t covers slice t / (mt * nt) of the slabs
+    const int T = mt * nt * kslices;
+    const int per = (T + 7) / 8;
+    const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (t >= T) return;
+    const int slice = t / (mt * nt);
+    int tm, tn;
+    tile_of(t % (mt * nt), mt, nt, tm, tn);
+    const int m0 = tm * BM, n0 = tn * OC;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+
+    // DMA sources: 32-bit byte offsets (the host keeps both operands under 2 GB); rows past
+    // the matrix repeat its last row (their outputs are not stored)
+    uint32_t voff[LPS];
+    {
+        const int rr = lane >> 3, cs = lane & 7;
+#pragma unroll
+        for (int i = 0; i < LPS; ++i) {
+            const int r = i * 8 + rr;
+            int row;
+            if (i < LA) {
+                row = min(m0 + r, M - 1);
+            } else {
+                const int br = r - BM;
+                const int gate = EPI == GEPI_SWIGLU && br >= OC;
+                row = min(n0 + br - gate * OC, N - 1) + gate * N;
+            }
+            voff[i] = (uint32_t)((row * K + ((cs ^ pipe_swz(r)) << 3)) * 2);
+        }
+    }
+    unsigned char* const ring = smem + wave * RING;
+    const int s0 = slice * slice_slabs, nk = min(K / kPBK - s0, slice_slabs);
+    const int k_begin = s0 + wave * nk / KW, n_slabs = s0 + (wave + 1) * nk / KW - k_begin;
+    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A) + (size_t)k_begin * kPRow;
+    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B) + (size_t)k_begin * kPRow;
+    auto issue = [&](int slab) {
+        const unsigned char* sa = pa + slab * kPRow;
+        const unsigned char* sb = pb + slab * kPRow;
+        unsigned char* dst = ring + (slab % S) * STAGE;
+#pragma unroll
+        for (int i = 0; i < LPS; ++i)
+            __builtin_amdgcn_global_load_lds(static_cast<const void*>((i < LA ? sa : sb) + voff[i]),
+                                             (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, 0);
+    };
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring);
+    const int r32 = lane & 31;
+    uint32_t roff[KSN];   // row r32, chunk of key step ks (32-row blocks differ by an immediate)
+#pragma unroll
+    for (int ks = 0; ks < KSN; ++ks)
+        roff[ks] = lds0 + (uint32_t)(r32 * kPRow + (((ks * 2 + (lane >> 5)) ^ pipe_swz(r32)) << 4));
+    typedef KsplitFrags<TM, TN> Frags;
+    auto read = [&](Frags& f, int slab) {
+        const uint32_t so = (uint32_t)((slab % S) * STAGE);
+#pragma unroll
+        for (int ks = 0; ks < KSN; ++ks) {
+            f.a[ks][0] = ds_read16<0>(roff[ks] + so);
+            if constexpr (TM == 2) f.a[ks][TM - 1] = ds_read16<32 * kPRow>(roff[ks] + so);
+            f.b[ks][0] = ds_read16<BM * kPRow>(roff[ks] + so);
+            if constexpr (TN == 2) f.b[ks][TN - 1] = ds_read16<(BM + 32) * kPRow>(roff[ks] + so);
+        }
+    };
+
+    f32x16_t acc[TN][TM];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
+
+    // slab i: its reads (issued before) have landed in `f`; refill its slot, issue the
+    // reads of slab i + 1 into `g`, and run its MFMAs
+    auto step = [&](int i, Frags& f, Frags& g) {
+        lgkm_wait<0>();
+#pragma unroll
+        for (int ks = 0; ks < KSN; ++ks) {
+#pragma unroll
+            for (int x = 0; x < TM; ++x) asm volatile("" : "+v"(f.a[ks][x]));
+#pragma unroll
+            for (int x = 0; x < TN; ++x) asm volatile("" : "+v"(f.b[ks][x]));
+        }
+        if (i + S < n_slabs) issue(i + S);
+        if (i + 1 < n_slabs) {
+            vm_wait_slabs<LPS>(min(S - 1, n_slabs - 2 - i));
+            asm volatile("" ::: "memory");
+            read(g, i + 1);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KSN; ++ks)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int x = 0; x < TM; ++x)
+                    acc[j][x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[ks][j], f.a[ks][x], acc[j][x], 0, 0, 0);
+    };
+    if (n_slabs > 0) {
+        for (int p = 0; p < min(S, n_slabs); ++p) issue(p);
+        vm_wait_slabs<LPS>(min(S, n_slabs) - 1);
+        asm volatile("" ::: "memory");
+        Frags f, g;
+        read(f, 0);
+        for (int i = 0; i < n_slabs; i += 2) {
+            step(i, f, g);
+            if (i + 1 < n_slabs) step(i + 1, g, f);
+        }
+    }
+
+    // partial tile: float4 chunk c of row m at c ^ swz(m) (distinct bank groups for 16
+    // lanes on 16 rows, and for 16 consecutive chunks)
+    auto swz = [](int m) { return CH >= 16 ? (m & 15) : ((m >> 1) & 7); };
+    float4* part = reinterpret_cast<float4*>(ring);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int x = 0; x < TM; ++x)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int m = x * 32 + r32, c = j * 8 + g * 2 + (lane >> 5);
+                part[m * CH + (c ^ swz(m))] =
+                    make_float4(acc[j][x][g * 4], acc[j][x][g * 4 + 1], acc[j][x][g * 4 + 2], acc[j][x][g * 4 + 3]);
+            }
+    __syncthreads();
+    auto total = [&](int m, int c) {
+        float4 v = reinterpret_cast<const float4*>(smem)[m * CH + (c ^ swz(m))];
+#pragma unroll
+        for (int w = 1; w < KW; ++w) {
+            const float4 u = reinterpret_cast<const float4*>(smem + w * RING)[m * CH + (c ^ swz(m))];
+            v.x += u.x;
+            v.y += u.y;
+            v.z += u.z;
+            v.w += u.w;
+        }
+        return v;
+    };
+    constexpr int OCH = OC / 4;
+    for (int idx = tid; idx < BM * OCH; idx += KW * kWave) {
+        const int m = idx / OCH, c = idx % OCH, row = m0 + m, col = n0 + c * 4;
+        if (row >= M || col >= N) continue;
+        const float4 t0 = total(m, c);
+        float v[4] = {t0.x, t0.y, t0.z, t0.w};
+        if constexpr (EPI == GEPI_SWIGLU) {
+            const float4 t1 = total(m, c + OCH);
+            const float g[4] = {t1.x, t1.y, t1.z, t1.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = silu_f32(round_bf16(g[e])) * round_bf16(v[e]);
+        } else if (bias != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += col + e < N ? bf16_to_f32(bias[col + e]) : 0.f;
+        }
+        const size_t at = (size_t)(EPI == GEPI_PARTIAL ? slice * M + row : row) * ldc + col;
+        if (EPI == GEPI_F32 || EPI == GEPI_PARTIAL) {
+            float* o = reinterpret_cast<float*>(Cout) + at;
+            if (vec) {
+                *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < N) o[e] = v[e];
+            }
+        } else {
+            bf16_t* o = reinterpret_cast<bf16_t*>(Cout) + at;
+            if (vec) {
+                uint2 w;
+                w.x = pack_bf16x2(v[0], v[1]);
+                w.y = pack_bf16x2(v[2], v[3]);
+                *reinterpret_cast<uint2*>(o) = w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < N) o[e] = (bf16_t)f32_to_bf16(v[e]);
+            }
+        }
+    }
+}
+
 // Split-K reduction: out[r, c] = sum over slices s = 0, 1, ... (in that order) of
 // part[s, r, c], + bias[c], as bf16 or fp32. Four columns per thread (N % 4 == 0).
+constexpr int kMaxSlices = 8;
 template <bool F32OUT>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ part, int ksplit, int M,
                                                                  int N, const bf16_t* __restrict__ bias,
@@ -697,14 +912,21 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;   // float4 index
     const size_t plane = (size_t)M * N;
     if (q * 4 >= plane) return;
-    float4 acc = *reinterpret_cast<const float4*>(part + q * 4);
-    for (int sl = 1; sl < ksplit; ++sl) {
-        const float4 v = *reinterpret_cast<const float4*>(part + (size_t)sl * plane + q * 4);
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
-    }
+    // every plane's load in flight at once (kMaxSlices of them; past the plan's slices the
+    // last plane again, not added)
+    float4 v[kMaxSlices];
+#pragma unroll
+    for (int sl = 0; sl < kMaxSlices; ++sl)
+        v[sl] = *reinterpret_cast<const float4*>(part + (size_t)min(sl, ksplit - 1) * plane + q * 4);
+    float4 acc = v[0];
+#pragma unroll
+    for (int sl = 1; sl < kMaxSlices; ++sl)
+        if (sl < ksplit) {
+            acc.x += v[sl].x;
+            acc.y += v[sl].y;
+            acc.z += v[sl].z;
+            acc.w += v[sl].w;
+        }
     const int col = (int)((q * 4) % (size_t)N);
     if (bias != nullptr) {
         acc.x += bf16_to_f32(bias[col + 0]);
@@ -742,11 +964,61 @@ static void gemm_wide_launch(int M, int N, int K, const bf16_t* A, const bf16_t*
                        B, bias, C, M, N, K, ldc, mt, nt);
 }
 
+template <int TM, int TN, int KW, int S, int EPI, int WPE>
+static void gemm_ksplit_launch(int M, int N, int K, const bf16_t* A, const bf16_t* B, const bf16_t* bias, void* C,
+                               int ldc, hipStream_t stream, int kslices = 1, int slice_slabs = 1 << 30) {
+    const int oc = (EPI == GEPI_SWIGLU) ? 16 * TN : 32 * TN;
+    const int mt = (M + 32 * TM - 1) / (32 * TM), nt = (N + oc - 1) / oc;
+    const int grid = 8 * ((mt * nt * kslices + 7) / 8);
+    const int vec = N % 4 == 0 && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
+    hipLaunchKernelGGL((gemm_ksplit_kernel<TM, TN, KW, S, EPI, WPE>), dim3(grid), dim3(KW * kWave), 0, stream, A, B, bias,
+                       C, M, N, K, ldc, mt, nt, vec, kslices, slice_slabs);
+}
+
 int prefill_cus();
 
+// Which tile of the K-split kernel (four waves) an unsliced launch takes: 0 none, 1: 32 x 32
+// (two workgroups per CU), 2: 64 x 32, 3: 64 x 64 (one per CU). It pays while every tile has
+// a CU of its own, smallest tile first, and for up to 32 rows at any width, where the larger
+// kernels' tiles are mostly padding. Up to 64 rows, or K below 8192 (beyond, the other
+// kernels' slices over workgroups are the better split); a wave wants 3 slabs (K of 768; a
+// 64 x 64 tile 5): the pipelined kernel's ring nearly holds shorter rows (40 x 512 -> 256 5.1
+// / 5.1, 40 x 256 -> 512 4.7 / 4.3, 40 x 768 -> 1024 4.9 / 6.3).
+// Measured on MI355X (us, this kernel / the pipelined one): 37 x 1536 -> 2048 4.4 / 9.9,
+// 19 x 896 -> 1152 4.3 / 6.7, 24 x 1536 -> 17920 14.2 / 20.0, 256 x 1536 -> 2048 6.2 / 10.0,
+// 100 x 3584 -> 4608 15.9 / 19.3, 512 x 1536 -> 2048 9.2 / 10.4, 24 x 8960 -> 1536 13.6 /
+// 17.4 (sliced); not: 1344 x 2048 -> 2560 37.9 / 25.2, 256 x 3584 -> 4608 28.7 / 30.1.
+// SwiGLU: 24 x 1536 -> 8960 14.6 / 16.7, 16 x 3584 -> 18944 48.1 / 67.8, 60 x 896 -> 4864
+// 7.6 / 9.9; not: 60 x 1536 -> 8960 22.4 / 17.9.
+static bool offsets_fit(long M, long b_rows, long K) {   // 32-bit byte offsets into both operands
+    return M * K * 2 < 0x7fffffffL && b_rows * K * 2 < 0x7fffffffL;
+}
+static int ksplit_tile(int M, int N, int K, bool swiglu) {
+    const int cus = prefill_cus(), nk = K / kPBK;
+    if (K % kPBK != 0 || nk < 12 || !offsets_fit(M, swiglu ? 2L * N : N, K)) return 0;
+    if (M <= 32) return 1;
+    const long mt32 = (M + 31) / 32, mt64 = (M + 63) / 64, nt32 = ((long)N + 31) / 32, nt64 = ((long)N + 63) / 64;
+    if (swiglu) return M <= 64 && mt64 * nt32 <= cus ? 3 : 0;
+    if (M > 64 && nk >= 128) return 0;
+    if (mt32 * nt32 <= cus) return 1;
+    if (mt64 * nt32 <= cus) return 2;
+    return mt64 * nt64 <= cus && nk >= 20 ? 3 : 0;
+}
+
 // Split-K plan for a plain (non-SwiGLU) projection with K % 64 == 0 and K >= 4096 whose
-// 128 x 128 tiles leave the chip's workgroup slots empty; ksplit 0 = no split. Each slice
-// covers at least 16 slabs (1024 keys). Measured on MI355X (us):
+// tiles leave the chip's workgroup slots empty; ksplit 0 = no split over workgroups. Each
+// slice covers at least 16 slabs (1024 keys). Measured on MI355X (us):
+//  * up to 32 rows, and up to 64 with at most 64 MB of weights: the K-split kernel's 32 x 32
+//    (64 x 32) tiles, as many slices as leave the fewest slabs to the busiest CU, at two
+//    (one) workgroups per CU: 24 x 8960 -> 1536 17.4 -> 8.9, 19 x 4864 -> 896 17.6 -> 7.3,
+//    60 x 11008 -> 2048 22.3 -> 16.6, 24 x 18944 -> 3584 35.2 -> 31.2 (128 x 128 tiles
+//    before); 64 x 18944 -> 3584 stays (36.7 against 40.4);
+//  * more rows, half the CUs in 64 x 64 tiles at most and at most 64 MB of weights: the
+//    K-split kernel's 64 x 64 tiles, one workgroup per CU: 300 x 8960 -> 1536 24.0 -> 19.9,
+//    128 x 8960 -> 1536 20.1 -> 13.4, 300 x 4864 -> 896 20.7 -> 12.9; 128 x 18944 -> 3584
+//    stays (39.5 against 49.1);
+//  * K < 8192 and a 64 x 64 tile (or fewer rows: a 32 x 32 tile) for every CU: unsliced
+//    (ksplit_tile): 700 x 4864 -> 896 24.2 -> 18.6;
 //  * tiles for at most a third of the CUs: as many slices as fill every CU once (at most
 //    8), one workgroup per CU over a 4-deep ring: 512 x 8960 -> 1536 33.6 -> 28.3 (5
 //    slices, against 8 slices over 2-deep rings, two workgroups per CU), 512 x 11008 ->
@@ -755,7 +1027,8 @@ int prefill_cus();
 //    4-deep rings: 1024 x 8960 -> 1536 46.1 -> 50.9, 512 x 18944 -> 3584 101.2 -> 102.9).
 struct SplitK {
     int ksplit = 0, kt_per = 0;
-    bool deep = false;  // 4-deep ring, one workgroup per CU (else 2-deep, two per CU)
+    int tile = 0;       // tile of the K-split kernel (ksplit_tile), or 0: 128 x 128
+    bool deep = false;  // 128 x 128: 4-deep ring, one workgroup per CU (else 2-deep, two per CU)
 };
 static SplitK splitk_plan(int M, int N, int K) {
     SplitK p;
@@ -763,16 +1036,37 @@ static SplitK splitk_plan(int M, int N, int K) {
     const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
     const int nk = K / kPBK;
     if (tiles > 128 || nk < 64) return p;
-    const int fill = (int)std::min<long>({8L, prefill_cus() / tiles, (long)(nk / 16)});
-    int ks;
-    if (fill >= 3) {
-        ks = fill;
-        p.deep = true;
+    const int cus = prefill_cus();
+    const bool small_w = (long)N * K * 2 <= (64L << 20);
+    const long mt32 = (M + 31) / 32, mt64 = (M + 63) / 64, nt32 = (N + 31) / 32, nt64 = (N + 63) / 64;
+    const int most = std::min(8, nk / 16);
+    int ks = 0;
+    if (M <= 32 || (M <= 64 && small_w)) {
+        p.tile = M <= 32 ? 1 : 2;
+        const long t = M <= 32 ? mt32 * nt32 : mt64 * nt32, slots = (M <= 32 ? 2L : 1L) * cus;
+        ks = 1;
+        for (int n = 2; n <= most && t * n <= slots; ++n) {   // fewest (workgroups on a CU) / n
+            const long a = (t * n + cus - 1) / cus * ks, b = (t * ks + cus - 1) / cus * n;
+            if (a <= b) ks = n;
+        }
+    } else if (nk < 128 && mt32 * nt32 <= cus) {
+        return p;
+    } else if (2 * mt64 * nt64 <= cus && small_w) {
+        p.tile = 3;
+        ks = (int)std::min<long>(most, cus / (mt64 * nt64));
+    } else if (nk < 128 && mt64 * nt64 <= cus) {
+        return p;
     } else {
-        ks = (int)std::min<long>(8, (384 + tiles - 1) / tiles);
-        ks = std::min(ks, nk / 16);
+        const int fill = (int)std::min<long>(most, cus / tiles);
+        if (fill >= 3) {
+            ks = fill;
+            p.deep = true;
+        } else {
+            ks = (int)std::min<long>(8, (384 + tiles - 1) / tiles);
+            ks = std::min(ks, nk / 16);
+        }
     }
-    if (ks < 2) return p;
+    if (ks < 2 || (p.tile != 0 && !offsets_fit(M, N, K))) return SplitK{};
     p.kt_per = (nk + ks - 1) / ks;
     p.ksplit = (nk + p.kt_per - 1) / p.kt_per;
     return p;
@@ -788,7 +1082,13 @@ static void gemm_splitk_launch(int M, int N, int K, const bf16_t* A, const bf16_
                                bool f32out, float* part, const SplitK& p, hipStream_t stream) {
     const int mt = (M + 127) / 128, nt = (N + 127) / 128;
     const int grid = 8 * ((mt * nt * p.ksplit + 7) / 8);
-    if (p.deep)
+    if (p.tile == 1)
+        gemm_ksplit_launch<1, 1, 4, 2, GEPI_PARTIAL, 2>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
+    else if (p.tile == 2)
+        gemm_ksplit_launch<2, 1, 4, 2, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
+    else if (p.tile == 3)
+        gemm_ksplit_launch<2, 2, 4, 2, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
+    else if (p.deep)
         hipLaunchKernelGGL((gemm_pipe_kernel<128, 128, 4, GEPI_PARTIAL>), dim3(grid), dim3(kGemmThreads), 0, stream, A,
                            B, nullptr, part, M, N, K, N, mt, nt, p.ksplit, p.kt_per);
     else
@@ -817,7 +1117,24 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
     // does not (3 wide rounds, the last nearly empty, against 3.7 narrow ones).
     const int tile_knob = kernel_knob(EFM_KNOB_GEMM_TILE);
     const long b_rows = (EPI == GEPI_SWIGLU) ? 2L * N : (long)N;
-    const bool wide_ok = K % kPBK == 0 && (long)M * K * 2 < 0x7fffffffL && b_rows * K * 2 < 0x7fffffffL;
+    const bool wide_ok = K % kPBK == 0 && offsets_fit(M, b_rows, K);
+    if (tile_knob == 0) {
+        switch (ksplit_tile(M, N, K, EPI == GEPI_SWIGLU)) {
+            case 1:
+                gemm_ksplit_launch<1, 1, 4, 2, EPI, 2>(M, N, K, A, B, bias, C, ldc, stream);
+                return check_launch("gemm_bf16");
+            case 2:
+                if constexpr (EPI != GEPI_SWIGLU) {
+                    gemm_ksplit_launch<2, 1, 4, 2, EPI, 1>(M, N, K, A, B, bias, C, ldc, stream);
+                    return check_launch("gemm_bf16");
+                }
+                break;
+            case 3:
+                gemm_ksplit_launch<2, 2, 4, 2, EPI, 1>(M, N, K, A, B, bias, C, ldc, stream);
+                return check_launch("gemm_bf16");
+            default: break;
+        }
+    }
     if (wide_ok && tile_knob != 1) {
         const long r_wide = (tiles(256, 256) + 255) / 256, r_pipe = (tiles(128, 128) + 511) / 512;
         // 192 x 256 tiles (six MFMA tiles per wave instead of eight) take 0.9 of a 256 x

@@ -651,6 +651,67 @@ def test_linear_split_k_matches_unsplit_and_oracle(gpu, m, k, n, kind):
         assert_close_bf16(outs[0][rows], exp)
 
 
+@pytest.mark.parametrize("m,k,n,kind,split", [
+    # tile edges in rows and columns, waves with unequal slabs (K 832), ragged columns that
+    # take scalar stores, every epilogue, and the sliced forms of the three tiles
+    pytest.param(2, 768, 32, "bf16", False, id="one_tile"),
+    pytest.param(31, 832, 100, "bias", False, id="unequal_slabs"),
+    pytest.param(32, 1536, 1001, "f32", False, id="ragged_f32"),
+    pytest.param(33, 1536, 2048, "bias", False, id="second_row_block"),
+    pytest.param(64, 896, 1154, "f32", False, id="f32_64_rows"),
+    pytest.param(200, 2048, 2048, "bias", False, id="64x32_tiles"),
+    pytest.param(257, 2048, 1090, "f32", False, id="64x32_ragged"),
+    pytest.param(400, 1536, 2050, "bias", False, id="64x64_ragged"),
+    pytest.param(700, 4864, 896, "bf16", False, id="64x64_long_k"),
+    pytest.param(2, 896, 8, "swiglu", False, id="swiglu_one_tile"),
+    pytest.param(32, 1536, 8950, "swiglu", False, id="swiglu_ragged"),
+    pytest.param(60, 896, 4864, "swiglu", False, id="swiglu_64_rows"),
+    pytest.param(24, 8960, 1536, "bias", True, id="sliced_32x32"),
+    pytest.param(61, 11008, 2044, "f32", True, id="sliced_64x32"),
+    pytest.param(130, 8960, 1000, "bias", True, id="sliced_64x64"),
+])
+def test_gemm_k_split_over_waves(gpu, knob, m, k, n, kind, split):
+    """Launches that split K over the waves of a workgroup (and, with a workspace, over
+    workgroups): against float64 products of the same bf16 operands, every output written
+    and nothing past the last one, deterministic, and the pipelined kernel's result to the
+    rounding of the sums. Bounds: an fp32 sum of k products in any order is within k 2^-24 of
+    sum |x w|; a bf16 output adds half an ulp (2^-8 of its value), SwiGLU's two rounded
+    factors and its silu (slope at most 1.1) three more."""
+    torch.manual_seed(m + n)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=gpu)
+    w = (torch.randn((2 if kind == "swiglu" else 1) * n, k, device=gpu) * 0.02).to(torch.bfloat16)
+    b = (torch.randn(n, device=gpu) * 0.05).to(torch.bfloat16) if kind in ("bias", "f32") else None
+    dt, cd = (torch.float32, C.EFM_DTYPE_F32) if kind == "f32" else (torch.bfloat16, C.EFM_DTYPE_BF16)
+    need = C.load().efm_linear_workspace_bytes(m, k, n)
+    assert (need > 0) == split
+    ws = torch.full((max(need, 256),), 0x7f, dtype=torch.uint8, device=gpu)
+    outs = []
+    for path in (0, 0, 1):
+        knob(C.EFM_KNOB_GEMM_TILE, path)
+        y = torch.full((m * n + 8,), -7.0, dtype=dt, device=gpu)
+        if kind == "swiglu":
+            C.call("efm_fused_gate_up_swiglu", m, k, n, ptr(x), ptr(w), ptr(y), stream())
+        elif path == 0 and split:
+            C.call("efm_linear_ws", m, k, n, ptr(x), ptr(w), ptr(b), ptr(y), cd, ptr(ws), need, stream())
+        else:
+            C.call("efm_linear", m, k, n, ptr(x), ptr(w), ptr(b), ptr(y), cd, stream())
+        torch.cuda.synchronize()
+        assert (y[m * n:] == -7.0).all()
+        outs.append(y[:m * n].reshape(m, n))
+    assert torch.equal(outs[0], outs[1])
+    h = x.double() @ w.double().T
+    mag = x.double().abs() @ w.double().abs().T * (k * 2.0 ** -24)
+    if kind == "swiglu":
+        u, g = h[:, :n], h[:, n:]
+        ref = torch.nn.functional.silu(g) * u
+        err = 2.0 ** -8 * (2 * ref.abs() + 1.1 * (g * u).abs()) + 1.1 * (mag[:, n:] * u.abs() + mag[:, :n] * g.abs()) + 1e-6
+    else:
+        ref = h if b is None else h + b.double()
+        err = mag + (0 if kind == "f32" else 2.0 ** -8 * ref.abs()) + 1e-6
+    for y in outs[1:]:
+        assert ((y.double() - ref).abs() <= err).all()
+
+
 def test_gemm_long_k_tiles_agree_bit_exact(gpu):
     """K = 11008 (the VL-3B down projection) at three M: 100 rows run 64 x 64 tiles, 1344
     rows (176 tiles of 128 x 128, at most one per CU) 128 x 128 tiles over a 4-deep ring
