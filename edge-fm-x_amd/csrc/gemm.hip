@@ -1,12 +1,12 @@
 // Prefill projections on the gfx950 matrix cores: C[M, N] = A[M, K] . B[N, K]^T in
-// bf16 with fp32 accumulation (v_mfma_f32_32x32x16_bf16). A holds activations (one
-// row per token) and B the weights in their [out, in] layout, so both operands are
-// K-contiguous and feed the MFMA lanes with 16-byte loads.
+// bf16 with fp32 accumulation (v_mfma_f32_32x32x16_bf16, 16x16x32 in the tall kernel). A
+// holds activations (one row per token) and B the weights in their [out, in] layout, so both
+// operands are K-contiguous and feed the MFMA lanes with 16-byte loads.
 //
 //  * K % 64 == 0 (every Qwen2.5 projection), kernels fed by global_load_lds DMA into
 //    XOR-swizzled LDS rings, operand reads software-pipelined against the MFMAs and a
 //    grouped tile order per XCD:
-//      - the wide kernel: 256 x 256 tiles, one 8-wave workgroup per CU (large M);
+//      - the tall kernel: 256 x 256 or 192 x 256 tiles, one 4-wave workgroup per CU;
 //      - the pipelined kernel: 128 x 128 (128 x 64, 64 x 64) tiles, two 4-wave
 //        workgroups per CU (few tiles), plus its split-K form.
 //    A cost model (rounds of resident workgroups) picks between them.
@@ -213,10 +213,8 @@ __device__ __forceinline__ void tile_of(int t, int mt, int nt, int& tm, int& tn)
 // lanes at a time: the 16 rows an MFMA operand read touches at once must land in 16
 // distinct 16-byte bank groups. With 128-byte rows (8 chunks) two rows fill the 256-byte
 // bank period, so rows of equal parity need distinct chunks: (row / 2) % 8, with the
-// parity folded into bit 2 so that any 8 consecutive rows also differ. With 64-byte rows
-// (4 chunks) four rows fill the period: rows equal mod 4 need distinct chunks.
+// parity folded into bit 2 so that any 8 consecutive rows also differ.
 __device__ __forceinline__ int pipe_swz(int row) { return ((row >> 1) ^ ((row & 1) << 2)) & 7; }
-__device__ __forceinline__ int wide_swz(int row) { return ((row >> 1) ^ (row >> 2)) & 3; }
 
 constexpr int kPBK = 64;            // K per slab
 constexpr int kPRow = kPBK * 2;     // bytes per operand row in LDS
@@ -413,28 +411,6 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_pipe_kernel(const bf16_t* _
     }
 }
 
-// ---------------------------------------------------------------------------------
-// Wide-tile kernel: BM x BN workgroup tiles (256 x 256 in use), one workgroup per CU, its
-// WGM x WGN waves (2 x 4 in use: two per SIMD) each owning a (BM/WGM) x (BN/WGN) block of
-// 32 x 32 MFMA tiles. Relative to 128 x 128 tiles each MFMA needs half the bytes from L2
-// and, with 128 x 64 wave blocks, three quarters of the LDS reads; the second wave on
-// each SIMD issues MFMAs while the first waits on its memory instructions. (Measured on
-// the 7B gate/up shape: 4 waves with 128 x 128 blocks and 256 AGPR accumulators reach
-// 1.08 PF/s, the 2 x 4 layout 1.16 PF/s; the per-stage DMA is the largest cost beyond
-// the MFMAs themselves, about a quarter of the time, whether or not its loads hit L2.)
-//  * 32-key stages in an S-deep LDS ring filled by global_load_lds (16 bytes per lane,
-//    one 1 KB wave load covers 16 rows x 64 bytes). Lane i of a wave load lands at byte
-//    16 i of its 1 KB block, so the lane fetches the chunk that belongs there: row i / 4,
-//    logical chunk (i % 4) ^ wide_swz(row).
-//  * Per stage and wave: two 16-key steps. Step 0's MFMAs run with step 1's operand reads
-//    and the DMA of stage s + S - 1 interleaved, one memory instruction per MFMA; step 1's
-//    MFMAs run with the reads of stage s + 1's step 0, behind a bare barrier that follows
-//    this wave's own vmcnt wait for stage s + 1. That barrier also orders every wave's
-//    reads of stage s - 1 before its slot is refilled in the next stage.
-// ---------------------------------------------------------------------------------
-constexpr int kWBK = 32;            // keys per stage
-constexpr int kWRow = kWBK * 2;     // bytes per operand row per stage
-
 template <int OFF>
 __device__ __forceinline__ bf16x8_t ds_read16(uint32_t addr) {
     bf16x8_t d;
@@ -442,100 +418,63 @@ __device__ __forceinline__ bf16x8_t ds_read16(uint32_t addr) {
     return d;
 }
 
-// One key step's operand fragments: A rows at a + 2048 i, B rows at b + 2048 j.
-template <int TM, int TN>
-struct WideFrags {
-    bf16x8_t a[TM], b[TN];
-};
-
-template <int I, int TM, int TN>
-__device__ __forceinline__ void wide_read_one(WideFrags<TM, TN>& f, uint32_t a, uint32_t b) {
-    if constexpr (I < TM) f.a[I] = ds_read16<I * 32 * kWRow>(a);
-    else f.b[I - TM] = ds_read16<(I - TM) * 32 * kWRow>(b);
-}
-
-template <int TM, int TN, int... I>
-__device__ __forceinline__ void wide_read_all(WideFrags<TM, TN>& f, uint32_t a, uint32_t b,
-                                              std::integer_sequence<int, I...>) {
-    (wide_read_one<I>(f, a, b), ...);
-}
-
 template <int N>
 __device__ __forceinline__ void lgkm_wait() {
     asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// DMA of one stage's operand rows: per-lane byte offsets (row, swizzled chunk) of each
-// of the wave's loads from the operand base; the stage's base pointers and LDS slot are
-// uniform values computed once per stage. EXACT: both operands' 1 KB blocks divide evenly
-// over the waves, so load i of every wave reads A for i < LA and lands i * NW blocks past
-// the wave's first. Otherwise (192-row tiles: 12 A + 16 B blocks over 8 waves) each load
-// carries a wave-uniform operand choice and LDS offset.
-template <int LPW, int LA, int NW, bool EXACT>
-struct WideDma {
-    uint32_t voff[LPW];
-    uint32_t dst[EXACT ? 1 : LPW];
-    bool from_a[EXACT ? 1 : LPW];
-    __device__ __forceinline__ void issue(int i, const unsigned char* sa, const unsigned char* sb,
-                                          unsigned char* slot_wave) const {
-        const unsigned char* base;
-        unsigned char* d;
-        if constexpr (EXACT) {
-            base = i < LA ? sa : sb;
-            d = slot_wave + i * NW * 1024;
-        } else {
-            base = from_a[i] ? sa : sb;
-            d = slot_wave + dst[i];
-        }
-        __builtin_amdgcn_global_load_lds(static_cast<const void*>(base + voff[i]),
-                                         (__attribute__((address_space(3))) void*)d, 16, 0, 0);
-    }
+// ---------------------------------------------------------------------------------
+// Tall kernel (launches that fill the chip): 256 x 256 (192 x 256) tiles, one workgroup per
+// CU, four waves, one per SIMD, each owning a 128 x 128 (96 x 128) block of 16 x 16 MFMA
+// tiles in 256 (192) accumulator registers.
+//  * What bounds it is the card's power: on zero operands the same launches run at 1.6-1.7
+//    PF/s, on N(0, 1) ones at 1.3-1.4, and removing the DMA or the operand reads changes the
+//    rate through what they consume. So the layout moves as little as it can: a 128 x 128
+//    block reads two thirds of the LDS bytes per MFMA of a 128 x 64 one, rows of 64 keys
+//    are whole 128-byte lines, buffer loads carry 32-bit offsets, and the 16 x 16 x 32 MFMA
+//    sustains 1.97 PF/s on random operands where the 32 x 32 x 16 one sustains 1.65 (2 waves
+//    a SIMD; the two give the same bits).
+//  * 64-key operand slabs (32 KB) in a ring of five slots, A and B in turn. Step 0 of slab s
+//    runs with its second half's operand reads and the loads of A(s + 2); then one barrier
+//    (slab s is in registers everywhere, slab s + 1 has landed), and step 1 runs with the
+//    first reads of slab s + 1 and the loads of B(s + 2) into the slot that A(s) has left.
+//  * The weight rows are the MFMA's first operand: a lane ends with four consecutive columns
+//    of one row. SwiGLU interleaves 16-row blocks of up and gate weights.
+//  Measured against the 8-wave 32 x 32 x 16 kernel over 32-key stages that it replaces (us):
+//  4096 x 3584 -> 2 x 18944 SwiGLU 1103 -> 855 (1.30 PF/s), 4096 x 18944 -> 3584 515 -> 436,
+//  4096 x 3584 -> 4608 156 -> 129, 512 x 1536 -> 2 x 8960 38.8 -> 33.6.
+// ---------------------------------------------------------------------------------
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void tall_load(const unsigned char* src, uint32_t off, unsigned char* dst) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(src), (short)0, 0x7fffffff, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, (int)off, 0, 0, 0);
+}
+
+template <int TM, int TN>
+struct TallFrags {
+    bf16x8_t a[TM], b[TN];
 };
 
-// MFMA I of a key step (tile I / TN, I % TN) on f, then (READS) operand read I of the next
-// step into g and (DMA) this wave's load I of the stage at sa / sb into slot_wave. Each
-// group is a scheduling barrier: the memory instructions go out one per MFMA, early in
-// the step (measured: issuing the loads evenly over the step is slower).
-template <int I, int TM, int TN, int LPW, bool READS, bool DMA, class Dma>
-__device__ __forceinline__ void wide_slot(f32x16_t (&acc)[TM][TN], const WideFrags<TM, TN>& f,
-                                          WideFrags<TM, TN>& g, uint32_t ga, uint32_t gb, const Dma& dma,
-                                          const unsigned char* sa, const unsigned char* sb,
-                                          unsigned char* slot_wave) {
-    constexpr int i = I / TN, j = I % TN;
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
-    if constexpr (READS && I < TM + TN) wide_read_one<I>(g, ga, gb);
-    if constexpr (DMA && I < LPW) dma.issue(I, sa, sb, slot_wave);
-    __builtin_amdgcn_sched_barrier(0);
+// Keeps the accumulators in their AGPRs at this point: otherwise the compiler may move them
+// about inside the loop.
+template <int TM, int TN>
+__device__ __forceinline__ void pin_acc(f32x4_t (&acc)[TM][TN]) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
-template <int TM, int TN, int LPW, bool READS, bool DMA, class Dma, int... I>
-__device__ __forceinline__ void wide_mma_step(f32x16_t (&acc)[TM][TN], const WideFrags<TM, TN>& f,
-                                              WideFrags<TM, TN>& g, uint32_t ga, uint32_t gb, const Dma& dma,
-                                              const unsigned char* sa, const unsigned char* sb,
-                                              unsigned char* slot_wave, std::integer_sequence<int, I...>) {
-    (wide_slot<I, TM, TN, LPW, READS, DMA>(acc, f, g, ga, gb, dma, sa, sb, slot_wave), ...);
-}
-
-template <int BM, int BN, int WGM, int WGN, int S, int EPI>
-__global__ __launch_bounds__(WGM * WGN * kWave, 1) void gemm_wide_kernel(const bf16_t* __restrict__ A,
-                                                                    const bf16_t* __restrict__ B,
-                                                                    const bf16_t* __restrict__ bias,
-                                                                    void* __restrict__ Cout, int M, int N, int K,
-                                                                    int ldc, int mt, int nt) {
-    constexpr int NW = WGM * WGN;                // waves: a WGM x WGN grid over the tile
-    constexpr int WM = BM / WGM, WN = BN / WGN;
-    constexpr int TM = WM / 32, TN = WN / 32;
-    constexpr int STAGE = (BM + BN) * kWRow;
-    constexpr int QA = BM / 16, QB = BN / 16;   // 1 KB wave loads per operand per stage
-    constexpr int Q = QA + QB;
-    constexpr bool kExact = QA % NW == 0 && QB % NW == 0;
-    constexpr int LA = QA / NW, LPW = (Q + NW - 1) / NW;
-    constexpr int NR = TM + TN;                 // operand reads per key step
-    static_assert(QA >= NW && S >= 2 && (S - 2) * LPW <= 63, "bad wide GEMM shape");
-    static_assert(LPW <= TM * TN && NR <= TM * TN && NR <= 15, "interleave slots");
-    static_assert(EPI != GEPI_SWIGLU || TN % 2 == 0, "SwiGLU needs paired N tiles");
-    static_assert(EPI != GEPI_PARTIAL, "no split-K in the wide kernel");
-    __shared__ __align__(1024) unsigned char smem[S * STAGE];
+template <int TM, int EPI>
+__global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+                                                           const bf16_t* __restrict__ bias, void* __restrict__ Cout,
+                                                           int M, int N, int K, int ldc, int mt, int nt, int vec) {
+    constexpr int TN = 8, BM = 32 * TM, BN = 256;   // a wave: TM x TN tiles of 16 x 16
+    constexpr int SLOT = 256 * kPRow;               // one operand slab (64 keys), 32 KB
+    constexpr int LA = BM / 32, LB = BN / 32;       // 1 KB wave loads per operand slab and wave
+    __shared__ __align__(1024) unsigned char smem[5 * SLOT];
 
     const int T = mt * nt;
     const int per = (T + 7) / 8;
@@ -545,153 +484,194 @@ __global__ __launch_bounds__(WGM * WGN * kWave, 1) void gemm_wide_kernel(const b
     tile_of(t, mt, nt, tm, tn);
     const int m0 = tm * BM;
     const int n0 = (EPI == GEPI_SWIGLU) ? tn * (BN / 2) : tn * BN;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int wm = wave >> 1, wn = wave & 1;
 
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int lane = threadIdx.x % kWave;
-    const int wm = wave / WGN, wn = wave % WGN;
-
-    auto b_row = [&](int r) -> int {
-        if (EPI == GEPI_SWIGLU) {
-            const int blk = r / 32;
-            const int col = n0 + (blk / 2) * 32 + (r % 32);
-            return (col < N) ? ((blk % 2 == 0) ? col : N + col) : -1;
-        }
-        const int n = n0 + r;
-        return (n < N) ? n : -1;
-    };
-
-    // DMA sources (the host keeps both operands under 2 GB: 32-bit byte offsets)
-    WideDma<LPW, LA, NW, kExact> dma;
-    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A);
-    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B);
-    auto issue_stage = [&](int stage) {
-        const unsigned char* sa = pa + stage * kWRow;
-        const unsigned char* sb = pb + stage * kWRow;
-        unsigned char* sw = smem + (stage % S) * STAGE + wave * 1024;
-#pragma unroll
-        for (int i = 0; i < LPW; ++i) dma.issue(i, sa, sb, sw);
-    };
+    uint32_t va[LA], vb[LB];
     {
-        const int rr = lane >> 2, cs = lane & 3;
+        const int rr = lane >> 3, cs = lane & 7;
 #pragma unroll
-        for (int i = 0; i < LPW; ++i) {
-            // Block q of the stage; past the last block (Q % NW != 0), a repeat of the
-            // wave's first load (same source, same LDS bytes), so that every wave issues
-            // LPW loads per stage and the vmcnt waits below count alike in all waves.
-            int q = wave + NW * i;
-            if (q >= Q) q = wave;
-            if constexpr (!kExact) {
-                dma.from_a[i] = q < QA;
-                dma.dst[i] = (uint32_t)((q - wave) * 1024);
-            }
-            if (q < QA) {
-                const int row = q * 16 + rr;
-                const int grow = min(m0 + row, M - 1);
-                dma.voff[i] = (uint32_t)((grow * K + ((cs ^ wide_swz(row)) << 3)) * 2);
+        for (int i = 0; i < LA; ++i) {
+            const int r = (i * 4 + wave) * 8 + rr;
+            va[i] = (uint32_t)((min(m0 + r, M - 1) * K + ((cs ^ pipe_swz(r)) << 3)) * 2);
+        }
+#pragma unroll
+        for (int i = 0; i < LB; ++i) {
+            const int r = (i * 4 + wave) * 8 + rr;
+            int row;
+            if (EPI == GEPI_SWIGLU) {   // 16-row blocks of up (even) and gate (odd) weights
+                const int blk = r / 16;
+                row = min(n0 + (blk / 2) * 16 + r % 16, N - 1) + (blk % 2) * N;
             } else {
-                const int row = (q - QA) * 16 + rr;
-                int br = b_row(row);
-                if (br < 0) br = 0;
-                dma.voff[i] = (uint32_t)((br * K + ((cs ^ wide_swz(row)) << 3)) * 2);
+                row = min(n0 + r, N - 1);
             }
+            vb[i] = (uint32_t)((row * K + ((cs ^ pipe_swz(r)) << 3)) * 2);
         }
     }
+    const int nk = K / kPBK;
+    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A);
+    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B);
+    // operand slab q: A of slab q / 2 (even) or B (odd), in slot q % 5; slabs past the end
+    // repeat the last one (never read, so that every step issues the same loads)
+    auto slot = [&](int q) { return smem + (q % 5) * SLOT + wave * 1024; };
+    auto src_a = [&](int s) { return pa + min(s, nk - 1) * kPRow; };
+    auto src_b = [&](int s) { return pb + min(s, nk - 1) * kPRow; };
 
-    // Operand read addresses: row (lane % 32) of each 32-row tile, chunk ks * 2 + lane / 32
-    // under the stage's swizzle.
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)smem);
-    const int r32 = lane & 31, sw = wide_swz(r32);
-    const uint32_t x0 = (uint32_t)(((lane >> 5) ^ sw) << 4), x1 = (uint32_t)(((2 + (lane >> 5)) ^ sw) << 4);
-    const uint32_t rowA = (uint32_t)((wm * WM + r32) * kWRow), rowB = (uint32_t)(BM * kWRow + (wn * WN + r32) * kWRow);
-
-    f32x16_t acc[TM][TN];
+    const int r16 = lane & 15;
+    uint32_t ra[2], rb[2];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-    WideFrags<TM, TN> f0, f1;
-    auto tie = [&](WideFrags<TM, TN>& f) {
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t c = (uint32_t)(((h * 4 + (lane >> 4)) ^ pipe_swz(r16)) << 4);
+        ra[h] = lds0 + (uint32_t)((wm * (BM / 2) + r16) * kPRow) + c;
+        rb[h] = lds0 + (uint32_t)((wn * (BN / 2) + r16) * kPRow) + c;
+    }
+    typedef TallFrags<TM, TN> Frags;
+    auto tie = [&](Frags& f) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(f.a[i]));
 #pragma unroll
         for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(f.b[j]));
     };
+    auto read_one = [&](auto ic, Frags& f, uint32_t a, uint32_t b) {
+        constexpr int I = decltype(ic)::value;
+        if constexpr (I < TN) f.b[I] = ds_read16<I * 16 * kPRow>(b);
+        else if constexpr (I < TN + TM) f.a[I - TN] = ds_read16<(I - TN) * 16 * kPRow>(a);
+    };
 
-    const int nk = K / kWBK;
-    const int pre = min(S - 1, nk);
-    for (int p = 0; p < pre; ++p) issue_stage(p);
-    vm_wait_slabs<LPW>(min(S - 2, nk - 1));
+    f32x4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
+    pin_acc(acc);
+
+#pragma unroll
+    for (int i = 0; i < LA; ++i) tall_load(src_a(0), va[i], slot(0) + i * 4096);
+#pragma unroll
+    for (int i = 0; i < LB; ++i) tall_load(src_b(0), vb[i], slot(1) + i * 4096);
+#pragma unroll
+    for (int i = 0; i < LA; ++i) tall_load(src_a(1), va[i], slot(2) + i * 4096);
+#pragma unroll
+    for (int i = 0; i < LB; ++i) tall_load(src_b(1), vb[i], slot(3) + i * 4096);
+    vm_wait<LA + LB>();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    wide_read_all(f0, lds0 + rowA + x0, lds0 + rowB + x0, std::make_integer_sequence<int, NR>{});
+    Frags f0, f1;
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (read_one(std::integral_constant<int, I>{}, f0, ra[0], rb[0] + SLOT), ...);
+    }(std::make_integer_sequence<int, TM + TN>{});
 
-    // Stage s: key step 0 on f0 with step 1's reads and, while stages remain, this wave's
-    // loads of stage s + S - 1 (into the slot of stage s - 1, which every wave finished
-    // reading before the previous barrier); then key step 1 on f1 with the reads of stage
-    // s + 1, behind this wave's vmcnt wait for stage s + 1 and the barrier.
-    auto run_stage = [&](int s, auto dma_on, auto next_on) {
-        constexpr bool kDma = decltype(dma_on)::value, kNext = decltype(next_on)::value;
-        const uint32_t cur = lds0 + (uint32_t)((s % S) * STAGE);
-        const int ds = s + S - 1;
+    // one 32-key step: MFMA I, then behind every second one of the first 2 (TM + TN) an
+    // operand read of the next step, and behind the odd ones the step's DMA loads
+    auto mma_step = [&](Frags& f, Frags& g, uint32_t na, uint32_t nb, auto&& dma) {
+        [&]<int... I>(std::integer_sequence<int, I...>) {
+            ((acc[I / TN][I % TN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.b[I % TN], f.a[I / TN], acc[I / TN][I % TN],
+                                                                            0, 0, 0),
+              read_one(std::integral_constant<int, (I % 2 == 0 ? I / 2 : 99)>{}, g, na, nb),
+              dma(std::integral_constant<int, I>{}), __builtin_amdgcn_sched_barrier(0)),
+             ...);
+        }(std::make_integer_sequence<int, TM * TN>{});
+    };
+    for (int s = 0; s < nk; ++s) {
+        const uint32_t sa = (uint32_t)(((2 * s) % 5) * SLOT), sb = (uint32_t)(((2 * s + 1) % 5) * SLOT);
+        const uint32_t xa = (uint32_t)(((2 * s + 2) % 5) * SLOT), xb = (uint32_t)(((2 * s + 3) % 5) * SLOT);
+        const unsigned char* ga = src_a(s + 2);
+        unsigned char* da = slot(2 * s + 4);
         lgkm_wait<0>();
         tie(f0);
-        wide_mma_step<TM, TN, LPW, true, kDma>(acc, f0, f1, cur + rowA + x1, cur + rowB + x1, dma, pa + ds * kWRow,
-                                               pb + ds * kWRow, smem + (ds % S) * STAGE + wave * 1024,
-                                               std::make_integer_sequence<int, TM * TN>{});
+        mma_step(f0, f1, ra[1] + sa, rb[1] + sb, [&](auto ic) {
+            constexpr int I = decltype(ic)::value;
+            if constexpr (I % 4 == 3 && I / 4 < LA) tall_load(ga, va[I / 4], da + (I / 4) * 4096);
+        });
+        // slab s is in registers, slab s + 1 has landed for every wave
+        const unsigned char* gb = src_b(s + 2);
+        unsigned char* db = slot(2 * s + 5);
         lgkm_wait<0>();
         tie(f1);
-        if constexpr (kNext) {
-            if constexpr (kDma) vm_wait<(S - 2) * LPW>();
-            else vm_wait_slabs<LPW>(min(S - 2, nk - 2 - s));
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        }
-        const uint32_t nxt = lds0 + (uint32_t)(((s + 1) % S) * STAGE);
-        wide_mma_step<TM, TN, LPW, kNext, false>(acc, f1, f0, nxt + rowA + x0, nxt + rowB + x0, dma, pa, pb, smem,
-                                                 std::make_integer_sequence<int, TM * TN>{});
-    };
-    int s = 0;
-    for (; s < nk - (S - 1); ++s) run_stage(s, std::true_type{}, std::true_type{});
-    for (; s < nk - 1; ++s) run_stage(s, std::false_type{}, std::true_type{});
-    run_stage(nk - 1, std::false_type{}, std::false_type{});
+        vm_wait<LA>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        mma_step(f1, f0, ra[0] + xa, rb[0] + xb, [&](auto ic) {
+            constexpr int I = decltype(ic)::value;
+            if constexpr (I % 4 == 3 && I / 4 < LB) tall_load(gb, vb[I / 4], db + (I / 4) * 4096);
+        });
+        pin_acc(acc);
+    }
+    lgkm_wait<0>();
+    tie(f0);
+    vm_wait<0>();
+    __syncthreads();   // every wave is done with the operand slots
 
-    // Epilogue. Accumulator element e of tile (i, j): row = (e/4)*8 + (lane/32)*4 + e%4,
-    // column = lane % 32 within the 32 x 32 tile.
+    // Epilogue, half of the wave's row blocks at a time: the partial tile goes through the
+    // wave's own 32 KB slot as fp32 (element e of tile (i, j): row 16 i + lane % 16, column
+    // 16 j + (lane / 16) * 4 + e; float4 chunk c of row r at c ^ (r % 16): distinct bank
+    // groups), so that the stores are whole row segments, 16 lanes to a row.
+    constexpr int H = TM / 2;
+    float4* const part = reinterpret_cast<float4*>(smem + wave * SLOT);
+    const int seg = lane & 15;
+    const int col = n0 + wn * (EPI == GEPI_SWIGLU ? 64 : 128) + seg * (EPI == GEPI_SWIGLU ? 4 : 8);
+    float bv[8];
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int e = 0; e < 8; ++e)
+        bv[e] = (EPI != GEPI_SWIGLU && bias != nullptr && col + e < N) ? bf16_to_f32(bias[col + e]) : 0.f;
+    auto half = [&](auto hc) {
+        constexpr int i0 = decltype(hc)::value * H;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int row = m0 + wm * WM + i * 32 + (e / 4) * 8 + (lane / 32) * 4 + (e % 4);
+        for (int i = 0; i < H; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const f32x4_t x = acc[i0 + i][j];
+                part[(i * 16 + r16) * 32 + ((j * 4 + (lane >> 4)) ^ r16)] = make_float4(x[0], x[1], x[2], x[3]);
+            }
+#pragma unroll 4
+        for (int q = 0; q < H * 4; ++q) {
+            const int r = q * 4 + (lane >> 4);
+            const int row = m0 + wm * (BM / 2) + i0 * 16 + r, sw = r & 15;
+            constexpr int NV = EPI == GEPI_SWIGLU ? 4 : 8;
+            const int c0 = EPI == GEPI_SWIGLU ? (seg >> 2) * 8 + (seg & 3) : seg * 2;
+            const float4 x = part[r * 32 + (c0 ^ sw)], y = part[r * 32 + ((c0 + (EPI == GEPI_SWIGLU ? 4 : 1)) ^ sw)];
+            float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int e = 0; e < NV; ++e) {
+                if constexpr (EPI == GEPI_SWIGLU) v[e] = silu_f32(round_bf16(v[4 + e])) * round_bf16(v[e]);
+                else if (bias != nullptr) v[e] += bv[e];
+            }
             if (row >= M) continue;
-            if (EPI == GEPI_SWIGLU) {
-#pragma unroll
-                for (int j = 0; j < TN; j += 2) {
-                    const int col = n0 + ((wn * WN + j * 32) / 64) * 32 + (lane % 32);
+            const size_t at = (size_t)row * ldc + col;
+            if constexpr (EPI == GEPI_F32) {
+                float* o = reinterpret_cast<float*>(Cout) + at;
+                if (vec) {
                     if (col < N) {
-                        const float u = round_bf16(acc[i][j][e]);
-                        const float g = round_bf16(acc[i][j + 1][e]);
-                        const float o = silu_f32(g) * u;
-                        reinterpret_cast<bf16_t*>(Cout)[(size_t)row * ldc + col] = (bf16_t)f32_to_bf16(o);
+                        *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+                        *reinterpret_cast<float4*>(o + 4) = make_float4(v[4], v[5], v[6], v[7]);
                     }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < NV; ++e)
+                        if (col + e < N) o[e] = v[e];
                 }
             } else {
+                bf16_t* o = reinterpret_cast<bf16_t*>(Cout) + at;
+                if (vec) {
+                    if (col < N) {
+                        if constexpr (NV == 8) *reinterpret_cast<uint4*>(o) = pack8(v);
+                        else *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                    }
+                } else {
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = n0 + wn * WN + j * 32 + (lane % 32);
-                    if (col >= N) continue;
-                    float v = acc[i][j][e];
-                    if (bias != nullptr) v += bf16_to_f32(bias[col]);
-                    if (EPI == GEPI_F32) reinterpret_cast<float*>(Cout)[(size_t)row * ldc + col] = v;
-                    else reinterpret_cast<bf16_t*>(Cout)[(size_t)row * ldc + col] = (bf16_t)f32_to_bf16(v);
+                    for (int e = 0; e < NV; ++e)
+                        if (col + e < N) o[e] = (bf16_t)f32_to_bf16(v[e]);
                 }
             }
         }
-    }
+    };
+    half(std::integral_constant<int, 0>{});
+    half(std::integral_constant<int, 1>{});
 }
 
 // ---------------------------------------------------------------------------------
@@ -954,14 +934,15 @@ static void gemm_pipe_launch(int M, int N, int K, const bf16_t* A, const bf16_t*
                        M, N, K, ldc, mt, nt, 1, K / kPBK);
 }
 
-template <int BM, int BN, int WGM, int WGN, int S, int EPI>
-static void gemm_wide_launch(int M, int N, int K, const bf16_t* A, const bf16_t* B, const bf16_t* bias, void* C,
-                             int ldc, hipStream_t stream) {
-    const int ocols = (EPI == GEPI_SWIGLU) ? BN / 2 : BN;
-    const int mt = (M + BM - 1) / BM, nt = (N + ocols - 1) / ocols;
+template <int TM, int EPI>
+static void gemm_tall_launch(int M, int N, int K, const bf16_t* A, const bf16_t* B, const bf16_t* bias, void* C, int ldc,
+                             hipStream_t stream) {
+    const int ocols = (EPI == GEPI_SWIGLU) ? 128 : 256;
+    const int mt = (M + 32 * TM - 1) / (32 * TM), nt = (N + ocols - 1) / ocols;
     const int grid = 8 * ((mt * nt + 7) / 8);
-    hipLaunchKernelGGL((gemm_wide_kernel<BM, BN, WGM, WGN, S, EPI>), dim3(grid), dim3(WGM * WGN * kWave), 0, stream, A,
-                       B, bias, C, M, N, K, ldc, mt, nt);
+    const int vec = N % 8 == 0 && ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
+    hipLaunchKernelGGL((gemm_tall_kernel<TM, EPI>), dim3(grid), dim3(256), 0, stream, A, B, bias, C, M, N, K, ldc, mt, nt,
+                       vec);
 }
 
 template <int TM, int TN, int KW, int S, int EPI, int WPE>
@@ -1109,12 +1090,6 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
         return (long)((M + bm - 1) / bm) * ((N + ocols - 1) / ocols);
     };
     const dim3 block(kGemmThreads);
-    // 256 x 256 tiles (one 8-wave workgroup per CU, 32-bit operand offsets) against the
-    // 128 x 128 kernel (two workgroups per CU): rounds of resident workgroups times the
-    // work of one round, each at its measured rate on MI355X (about 1.15 and 0.95 PF/s on
-    // the 7B prefill projections), so the wide tile wins once it wastes no more than a
-    // partial round: 512 x 1536 -> 2 x 8960 (SwiGLU) runs wide, 1344 x 2048 -> 2 x 11008
-    // does not (3 wide rounds, the last nearly empty, against 3.7 narrow ones).
     const int tile_knob = kernel_knob(EFM_KNOB_GEMM_TILE);
     const long b_rows = (EPI == GEPI_SWIGLU) ? 2L * N : (long)N;
     const bool wide_ok = K % kPBK == 0 && offsets_fit(M, b_rows, K);
@@ -1136,18 +1111,25 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
         }
     }
     if (wide_ok && tile_knob != 1) {
-        const long r_wide = (tiles(256, 256) + 255) / 256, r_pipe = (tiles(128, 128) + 511) / 512;
-        // 192 x 256 tiles (six MFMA tiles per wave instead of eight) take 0.9 of a 256 x
-        // 256 round (measured, SwiGLU: 512 x 1536 -> 2 x 8960 48.3 -> 43.3 us in one round
-        // of 210 tiles against 140; 512 x 3584 -> 2 x 18944 198.2 -> 177.3 in two rounds,
-        // against 196.5 for the 128 x 128 kernel); the fewest weighted rounds wins.
-        const long r_192 = (tiles(192, 256) + 255) / 256;
-        if (tile_knob == 3 || (tile_knob == 0 && 171 * r_192 < std::min(190 * r_wide, 115 * r_pipe))) {
-            gemm_wide_launch<192, 256, 2, 4, 4, EPI>(M, N, K, A, B, bias, C, ldc, stream);
+        // Rounds of resident workgroups times the cost of one round: 100 for 192 x 256 tiles
+        // (one per CU), 127 for 256 x 256, 106 for 512 tiles of 128 x 128 (two per CU; 96
+        // below K 1536, where the larger tiles' first loads and epilogue weigh more), 75 for
+        // a last round of one per CU. Measured on MI355X (us, 192 / 256 / 128 x 128): 4096 x
+        // 3584 -> 4608 129 / 162 / 161, 4096 x 3584 -> 3584 123 / 91 / 125, 4096 x 3584 -> 2 x
+        // 18944 909 / 855 / 1286, 1344 x 2048 -> 2 x 11008 122 / 146 / 147, 4096 x 1536 -> 2048
+        // 32.7 / 42.8 / 33.9, 1344 x 2048 -> 2560 35.3 / 48.0 / 25.2, 700 x 896 -> 2 x 4864 21.6
+        // / 26.2 / 20.4. The choice is the fastest or within 3 % of it at all 27 shapes swept
+        // (1.5B, 3B, 7B and 0.5B projections at 300 to 16384 rows).
+        const long cus = 256, t128 = tiles(128, 128);
+        const long two = K < 1536 ? 96 : 106, rem = t128 % (2 * cus);
+        const long c128 = t128 / (2 * cus) * two + (rem == 0 ? 0 : rem <= cus ? 75 : two);
+        const long c192 = (tiles(192, 256) + cus - 1) / cus * 100, c256 = (tiles(256, 256) + cus - 1) / cus * 127;
+        if (tile_knob == 3 || (tile_knob == 0 && c192 < std::min(c256, c128))) {
+            gemm_tall_launch<6, EPI>(M, N, K, A, B, bias, C, ldc, stream);
             return check_launch("gemm_bf16");
         }
-        if (tile_knob == 2 || 190 * r_wide < 115 * r_pipe) {
-            gemm_wide_launch<256, 256, 2, 4, 4, EPI>(M, N, K, A, B, bias, C, ldc, stream);
+        if (tile_knob == 2 || c256 < c128) {
+            gemm_tall_launch<8, EPI>(M, N, K, A, B, bias, C, ldc, stream);
             return check_launch("gemm_bf16");
         }
     }

@@ -608,6 +608,37 @@ def test_gemm_wide_kernel_matches_narrow_bit_exact(gpu, knob, m, k, n, kind):
 
 
 @pytest.mark.parametrize("m,k,n,kind", [
+    pytest.param(2, 64, 8, "bf16", id="one_slab_two_rows"),
+    pytest.param(193, 128, 257, "f32", id="two_slabs_odd_columns"),
+    pytest.param(192, 192, 264, "bias", id="three_slabs"),
+    pytest.param(257, 320, 132, "swiglu", id="swiglu_second_tile"),
+    pytest.param(255, 384, 1003, "bias", id="odd_columns_bias"),
+    pytest.param(385, 448, 129, "swiglu", id="swiglu_odd_columns"),
+])
+def test_gemm_tall_kernel_edges(gpu, knob, m, k, n, kind):
+    """The one-workgroup-per-CU kernel (256- and 192-row tiles, knobs 2 and 3) at its tile
+    edges and its shortest rings: bit for bit the 128 x 128 family's outputs (knob 1; all sum
+    keys 16 at a time in increasing order), every output written and nothing past the last."""
+    torch.manual_seed(m + n)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=gpu)
+    w = (torch.randn((2 if kind == "swiglu" else 1) * n, k, device=gpu) * 0.05).to(torch.bfloat16)
+    b = (torch.randn(n, device=gpu) * 0.05).to(torch.bfloat16) if kind in ("bias", "f32") else None
+    dt, cd = (torch.float32, C.EFM_DTYPE_F32) if kind == "f32" else (torch.bfloat16, C.EFM_DTYPE_BF16)
+    outs = []
+    for path in (1, 2, 3):
+        knob(C.EFM_KNOB_GEMM_TILE, path)
+        y = torch.full((m * n + 8,), -7.0, dtype=dt, device=gpu)
+        if kind == "swiglu":
+            C.call("efm_fused_gate_up_swiglu", m, k, n, ptr(x), ptr(w), ptr(y), stream())
+        else:
+            C.call("efm_linear", m, k, n, ptr(x), ptr(w), ptr(b), ptr(y), cd, stream())
+        torch.cuda.synchronize()
+        assert (y[-8:] == -7.0).all()
+        outs.append(y[:-8])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("m,k,n,kind", [
     pytest.param(512, 8960, 1536, "bf16", id="c2_down"),
     pytest.param(300, 18944, 3584, "bf16", id="7b_down"),
     pytest.param(300, 4096, 1000, "bias", id="ragged_bias"),
