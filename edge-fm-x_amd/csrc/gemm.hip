@@ -1,17 +1,16 @@
 // Prefill projections on the gfx950 matrix cores: C[M, N] = A[M, K] . B[N, K]^T in
-// bf16 with fp32 accumulation (v_mfma_f32_32x32x16_bf16, 16x16x32 in the tall kernel). A
+// bf16 with fp32 accumulation (v_mfma_f32_16x16x32_bf16 in the slab kernel, 32x32x16). A
 // holds activations (one row per token) and B the weights in their [out, in] layout, so both
 // operands are K-contiguous and feed the MFMA lanes with 16-byte loads.
 //
 //  * K % 64 == 0 (every Qwen2.5 projection), kernels fed by global_load_lds DMA into
 //    XOR-swizzled LDS rings, operand reads software-pipelined against the MFMAs and a
 //    grouped tile order per XCD:
-//      - the tall kernel: 256 x 256 or 192 x 256 tiles, one 4-wave workgroup per CU;
-//      - the pipelined kernel: 128 x 128 (128 x 64, 64 x 64) tiles, two 4-wave
-//        workgroups per CU (few tiles), plus its split-K form.
-//    A cost model (rounds of resident workgroups) picks between them.
-//  * The same K, few rows or few tiles: the K-split kernel, whose four waves take a quarter
-//    of K each over 32 x 32 to 64 x 64 tiles.
+//      - the slab kernel (gemm_tall_kernel): 256 x 256 to 64 x 64 tiles on four waves, one
+//        or two workgroups per CU, plus its split-K form; a cost model (rounds of resident
+//        workgroups) picks the tile;
+//      - few rows, or few tiles and long K: the K-split kernel, whose four waves take a
+//        quarter of K each over 32 x 32 to 64 x 64 tiles.
 //  * Other K: a register-staged kernel with a padded LDS row pitch (40 bf16).
 //  * Epilogues: bf16 (+bias, the cuBLASLt BIAS epilogue), fp32, and SwiGLU, where the
 //    B tile interleaves 32-row blocks of up and gate weights so that each lane holds u
@@ -22,9 +21,9 @@
 #include "common.hpp"
 
 #include <algorithm>
+#include <iterator>
 #include <type_traits>
 #include <utility>
-#include <cstdlib>
 
 namespace efm {
 
@@ -182,18 +181,6 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_bf16_kernel(const bf16_t* _
     }
 }
 
-// ---------------------------------------------------------------------------------
-// Pipelined variant for K % 64 == 0: K slabs of 64 stream global -> LDS with
-// global_load_lds (no staging registers) into an S-deep ring, so S - 1 slabs are in
-// flight while the matrix cores work on one. Each wave's 1 KB DMA load covers 8 rows x 128
-// bytes; lane l fetches chunk (l % 8) ^ pipe_swz(row) of its row, so the ring holds an
-// XOR-swizzled layout and the 32-row MFMA operand reads spread over the LDS banks. The
-// operand reads are issued as ds_read_b128 with explicit waits: each wave waits for its
-// own DMA loads of the slab (vmcnt, counted exactly: every wave issues LPW loads per slab)
-// and a workgroup barrier makes all waves' loads visible. Tiles are assigned XCD by XCD
-// (dispatch is round-robin over the 8 XCDs), so workgroups that share weight columns
-// share an L2.
-// ---------------------------------------------------------------------------------
 // Tile order within one XCD's contiguous range of tile indices: groups of kGroupM row
 // tiles are walked column by column, so the workgroups resident on an XCD at one time
 // cover a kGroupM x (resident / kGroupM) block of output tiles and share its A and B
@@ -240,177 +227,6 @@ __device__ __forceinline__ void vm_wait_slabs(int slabs) {
     }
 }
 
-template <int BM, int BN, int S, int EPI>
-__global__ __launch_bounds__(kGemmThreads) void gemm_pipe_kernel(const bf16_t* __restrict__ A,
-                                                                 const bf16_t* __restrict__ B,
-                                                                 const bf16_t* __restrict__ bias,
-                                                                 void* __restrict__ Cout, int M, int N, int K, int ldc,
-                                                                 int mt, int nt, int ksplit, int kt_per) {
-    constexpr int WM = BM / 2, WN = BN / 2;
-    constexpr int TM = WM / 32, TN = WN / 32;
-    constexpr int STAGE = (BM + BN) * kPRow;
-    constexpr int QA = BM / 8, QB = BN / 8;  // 1 KB wave loads per operand per slab
-    constexpr int LPW = (QA + QB) / 4;       // wave loads per wave per slab
-    static_assert((QA + QB) % 4 == 0 && S >= 2 && S <= 8 && (S - 2) * LPW <= 63, "bad pipeline shape");
-    static_assert(EPI != GEPI_SWIGLU || TN % 2 == 0, "SwiGLU needs paired N tiles");
-    __shared__ __align__(1024) unsigned char smem[S * STAGE];
-
-    // split-K (GEPI_PARTIAL): work unit t covers K slice t / (mt * nt), slabs
-    // [slice * kt_per, (slice + 1) * kt_per), and writes fp32 partial sums
-    const int T = mt * nt * ksplit;
-    const int per = (T + 7) / 8;
-    const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-    if (t >= T) return;
-    const int slice = t / (mt * nt);
-    int tm, tn;
-    tile_of(t % (mt * nt), mt, nt, tm, tn);
-    const int kt0 = slice * kt_per;
-    const int m0 = tm * BM;
-    const int n0 = (EPI == GEPI_SWIGLU) ? tn * (BN / 2) : tn * BN;
-
-    const int tid = threadIdx.x;
-    const int wave = tid / kWave, lane = tid % kWave;
-    const int wm = wave / 2, wn = wave % 2;
-    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)smem);
-
-    auto b_row = [&](int r) -> int {
-        if (EPI == GEPI_SWIGLU) {
-            const int blk = r / 32;
-            const int col = n0 + (blk / 2) * 32 + (r % 32);
-            return (col < N) ? ((blk % 2 == 0) ? col : N + col) : -1;
-        }
-        const int n = n0 + r;
-        return (n < N) ? n : -1;
-    };
-
-    auto issue = [&](int kk, int slot) {
-        const int k0 = (kt0 + kk) * kPBK;
-        const int rr = lane >> 3, cs = lane & 7;
-#pragma unroll
-        for (int i = 0; i < LPW; ++i) {
-            const int q = wave + i * 4;
-            const bf16_t* src;
-            if (q < QA) {
-                const int row = min(m0 + q * 8 + rr, M - 1);
-                src = A + (size_t)row * K + k0 + ((cs ^ pipe_swz(q * 8 + rr)) << 3);
-            } else {
-                int br = b_row((q - QA) * 8 + rr);
-                if (br < 0) br = 0;
-                src = B + (size_t)br * K + k0 + ((cs ^ pipe_swz(q * 8 + rr)) << 3);
-            }
-            __builtin_amdgcn_global_load_lds(
-                static_cast<const void*>(src),
-                (__attribute__((address_space(3))) void*)(smem + slot * STAGE + q * 1024), 16, 0, 0);
-        }
-    };
-
-    f32x16_t acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-    // Operand reads of one 16-key step: TM A fragments and TN B fragments (ds_read_b128).
-    auto read_step = [&](uint32_t base, int ks, bf16x8_t (&af)[TM], bf16x8_t (&bfr)[TN]) {
-        const int c = ks * 2 + (lane >> 5);
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int r = wm * WM + i * 32 + (lane & 31);
-            const uint32_t addr = base + (uint32_t)(r * kPRow + ((c ^ pipe_swz(r)) << 4));
-            asm volatile("ds_read_b128 %0, %1" : "=v"(af[i]) : "v"(addr) : "memory");
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int r = wn * WN + j * 32 + (lane & 31);
-            const uint32_t addr = base + (uint32_t)(BM * kPRow + r * kPRow + ((c ^ pipe_swz(r)) << 4));
-            asm volatile("ds_read_b128 %0, %1" : "=v"(bfr[j]) : "v"(addr) : "memory");
-        }
-    };
-    // Software pipeline over the slab's four 16-key steps: the reads of step ks + 2 are
-    // issued behind the MFMAs of step ks, so LDS latency hides behind matrix work within
-    // the wave. The fragments come from inline-asm reads the compiler cannot track: each
-    // step waits for its own reads (lgkmcnt = the reads issued after them), then passes
-    // its fragments through an asm "write" so that no MFMA is scheduled above the wait.
-    auto compute = [&](int slot) {
-        const uint32_t base = lds0 + (uint32_t)(slot * STAGE);
-        constexpr int KSN = kPBK / 16;
-        constexpr int RPS = TM + TN;   // reads per step
-        static_assert(RPS <= 15, "lgkmcnt holds at most 15 outstanding reads");
-        bf16x8_t af[KSN][TM], bfr[KSN][TN];
-        read_step(base, 0, af[0], bfr[0]);
-        read_step(base, 1, af[1], bfr[1]);
-#pragma unroll
-        for (int ks = 0; ks < KSN; ++ks) {
-            if (ks + 1 < KSN) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(RPS) : "memory");
-            else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(af[ks][i]));
-#pragma unroll
-            for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(bfr[ks][j]));
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks][i], bfr[ks][j], acc[i][j], 0, 0, 0);
-            if (ks + 2 < KSN) read_step(base, ks + 2, af[ks + 2], bfr[ks + 2]);
-        }
-    };
-
-    const int nk = min(K / kPBK, kt0 + kt_per) - kt0;
-    const int pre = min(S - 1, nk);
-    for (int p = 0; p < pre; ++p) issue(p, p);
-    for (int kt = 0; kt < nk; ++kt) {
-        // Own DMA loads of slab kt have landed in LDS; the bare barrier (no fence, which
-        // would drain every slab in flight) then orders them before all waves' reads, and
-        // all waves' reads of slot (kt - 1) % S before it is refilled below.
-        vm_wait_slabs<LPW>(min(S - 2, nk - 1 - kt));
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (kt + S - 1 < nk) issue(kt + S - 1, (kt + S - 1) % S);
-        compute(kt % S);
-    }
-
-    // Epilogue. Accumulator element e of tile (i, j): row = (e/4)*8 + (lane/32)*4 + e%4,
-    // column = lane % 32 within the 32 x 32 tile.
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int row = m0 + wm * WM + i * 32 + (e / 4) * 8 + (lane / 32) * 4 + (e % 4);
-            if (row >= M) continue;
-            if (EPI == GEPI_SWIGLU) {
-#pragma unroll
-                for (int j = 0; j < TN; j += 2) {
-                    const int col = n0 + ((wn * WN + j * 32) / 64) * 32 + (lane % 32);
-                    if (col < N) {
-                        const float u = round_bf16(acc[i][j][e]);
-                        const float g = round_bf16(acc[i][j + 1][e]);
-                        const float o = silu_f32(g) * u;
-                        reinterpret_cast<bf16_t*>(Cout)[(size_t)row * ldc + col] = (bf16_t)f32_to_bf16(o);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = n0 + wn * WN + j * 32 + (lane % 32);
-                    if (col >= N) continue;
-                    float v = acc[i][j][e];
-                    if (EPI == GEPI_PARTIAL) {
-                        reinterpret_cast<float*>(Cout)[((size_t)slice * M + row) * N + col] = v;
-                        continue;
-                    }
-                    if (bias != nullptr) v += bf16_to_f32(bias[col]);
-                    if (EPI == GEPI_F32) reinterpret_cast<float*>(Cout)[(size_t)row * ldc + col] = v;
-                    else reinterpret_cast<bf16_t*>(Cout)[(size_t)row * ldc + col] = (bf16_t)f32_to_bf16(v);
-                }
-            }
-        }
-    }
-}
-
 template <int OFF>
 __device__ __forceinline__ bf16x8_t ds_read16(uint32_t addr) {
     bf16x8_t d;
@@ -424,25 +240,30 @@ __device__ __forceinline__ void lgkm_wait() {
 }
 
 // ---------------------------------------------------------------------------------
-// Tall kernel (launches that fill the chip): 256 x 256 (192 x 256) tiles, one workgroup per
-// CU, four waves, one per SIMD, each owning a 128 x 128 (96 x 128) block of 16 x 16 MFMA
-// tiles in 256 (192) accumulator registers.
-//  * What bounds it is the card's power: on zero operands the same launches run at 1.6-1.7
+// Slab kernel: a 32 TM x 32 TN tile on four waves, each owning a 16 TM x 16 TN block of 16 x
+// 16 MFMA tiles (256 x 256: 128 x 128 blocks, 256 accumulator registers, one wave per SIMD),
+// over 64-key slabs that buffer loads bring into LDS: a wave's 1 KB load is 8 rows x 128
+// bytes, and lane l fetches chunk (l % 8) ^ pipe_swz(row), so that the operand reads (16 rows
+// of one chunk) spread over the banks.
+//  * What bounds the large tiles is the card's power: on zero operands the same launches run at 1.6-1.7
 //    PF/s, on N(0, 1) ones at 1.3-1.4, and removing the DMA or the operand reads changes the
 //    rate through what they consume. So the layout moves as little as it can: a 128 x 128
 //    block reads two thirds of the LDS bytes per MFMA of a 128 x 64 one, rows of 64 keys
 //    are whole 128-byte lines, buffer loads carry 32-bit offsets, and the 16 x 16 x 32 MFMA
 //    sustains 1.97 PF/s on random operands where the 32 x 32 x 16 one sustains 1.65 (2 waves
 //    a SIMD; the two give the same bits).
-//  * 64-key operand slabs (32 KB) in a ring of five slots, A and B in turn. Step 0 of slab s
-//    runs with its second half's operand reads and the loads of A(s + 2); then one barrier
-//    (slab s is in registers everywhere, slab s + 1 has landed), and step 1 runs with the
-//    first reads of slab s + 1 and the loads of B(s + 2) into the slot that A(s) has left.
+//  * 64-key operand slabs in a ring of D + 1 slabs of A and one of D slabs of B. Step 0 of
+//    slab s runs with its second half's operand reads and the loads of A(s + D); then one
+//    barrier (slab s is in registers everywhere, slab s + 1 has landed), and step 1 runs with
+//    the first reads of slab s + 1 and the loads of B(s + D) into the slab that B(s) has left.
 //  * The weight rows are the MFMA's first operand: a lane ends with four consecutive columns
 //    of one row. SwiGLU interleaves 16-row blocks of up and gate weights.
-//  Measured against the 8-wave 32 x 32 x 16 kernel over 32-key stages that it replaces (us):
-//  4096 x 3584 -> 2 x 18944 SwiGLU 1103 -> 855 (1.30 PF/s), 4096 x 18944 -> 3584 515 -> 436,
-//  4096 x 3584 -> 4608 156 -> 129, 512 x 1536 -> 2 x 8960 38.8 -> 33.6.
+//  * Small tiles are bound by the latency of their slabs: D of 3 or 4 where LDS allows.
+//  Measured (us, before: an 8-wave kernel over 32-key stages for the large tiles, a shared
+//  ring with a barrier before every slab's reads for the small ones): 4096 x 3584 -> 2 x 18944
+//  SwiGLU 1103 -> 850 (1.31 PF/s), 4096 x 18944 -> 3584 515 -> 405, 4096 x 3584 -> 4608 156 ->
+//  120, 1344 x 11008 -> 2048 107 -> 89, 1000 x 3584 -> 4608 66 -> 35, 1344 x 2048 -> 2560 25.7
+//  -> 19.0, 512 x 1536 -> 2048 10.0 -> 8.0, 700 x 896 -> 1152 7.3 -> 5.8.
 // ---------------------------------------------------------------------------------
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -467,21 +288,32 @@ __device__ __forceinline__ void pin_acc(f32x4_t (&acc)[TM][TN]) {
         for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
-template <int TM, int EPI>
-__global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-                                                           const bf16_t* __restrict__ bias, void* __restrict__ Cout,
-                                                           int M, int N, int K, int ldc, int mt, int nt, int vec) {
-    constexpr int TN = 8, BM = 32 * TM, BN = 256;   // a wave: TM x TN tiles of 16 x 16
-    constexpr int SLOT = 256 * kPRow;               // one operand slab (64 keys), 32 KB
-    constexpr int LA = BM / 32, LB = BN / 32;       // 1 KB wave loads per operand slab and wave
-    __shared__ __align__(1024) unsigned char smem[5 * SLOT];
+// LDS of the slab kernel: D + 1 slabs of A and D of B.
+constexpr int tall_lds(int tm, int tn, int d) { return 32 * kPRow * ((d + 1) * tm + d * tn); }
 
-    const int T = mt * nt;
+template <int TM, int TN, int D, int EPI>
+__global__ __launch_bounds__(256, tall_lds(TM, TN, D) <= 80 * 1024 ? 2 : 1) void gemm_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+                                                           const bf16_t* __restrict__ bias, void* __restrict__ Cout,
+                                                           int M, int N, int K, int ldc, int mt, int nt, int vec,
+                                                           int kslices, int slice_slabs) {
+    constexpr int BM = 32 * TM, BN = 32 * TN;       // a wave: TM x TN tiles of 16 x 16
+    constexpr int ASZ = BM * kPRow, BSZ = BN * kPRow;   // an operand slab (64 keys)
+    constexpr int B0 = (D + 1) * ASZ;                   // the B ring, behind D + 1 slabs of A
+    constexpr int LA = BM / 32, LB = BN / 32;       // 1 KB wave loads per operand slab and wave
+    constexpr int NM = TM * TN, NR = TM + TN, NL = LA > LB ? LA : LB;   // MFMAs, reads, loads of a step
+    constexpr int RS = NM >= 2 * NR ? 2 : 1;        // MFMAs per operand read
+    constexpr int DS = NM / NL;                     // and per DMA load
+    static_assert(NM >= NR && DS >= 2, "a step's memory instructions go out behind its MFMAs");
+    __shared__ __align__(1024) unsigned char smem[B0 + D * BSZ];
+
+    // GEPI_PARTIAL: work unit t covers slice t / (mt * nt) of the slabs
+    const int T = mt * nt * kslices;
     const int per = (T + 7) / 8;
     const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
     if (t >= T) return;
+    const int slice = t / (mt * nt);
     int tm, tn;
-    tile_of(t, mt, nt, tm, tn);
+    tile_of(t % (mt * nt), mt, nt, tm, tn);
     const int m0 = tm * BM;
     const int n0 = (EPI == GEPI_SWIGLU) ? tn * (BN / 2) : tn * BN;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
@@ -508,12 +340,12 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restr
             vb[i] = (uint32_t)((row * K + ((cs ^ pipe_swz(r)) << 3)) * 2);
         }
     }
-    const int nk = K / kPBK;
-    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A);
-    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B);
-    // operand slab q: A of slab q / 2 (even) or B (odd), in slot q % 5; slabs past the end
-    // repeat the last one (never read, so that every step issues the same loads)
-    auto slot = [&](int q) { return smem + (q % 5) * SLOT + wave * 1024; };
+    const int s0 = slice * slice_slabs, nk = min(K / kPBK - s0, slice_slabs);
+    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A) + (size_t)s0 * kPRow;
+    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B) + (size_t)s0 * kPRow;
+    // slabs past the end repeat the last one (never read, so that every step issues the same
+    // loads)
+    unsigned char* const base = smem + wave * 1024;
     auto src_a = [&](int s) { return pa + min(s, nk - 1) * kPRow; };
     auto src_b = [&](int s) { return pb + min(s, nk - 1) * kPRow; };
 
@@ -549,58 +381,60 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restr
     pin_acc(acc);
 
 #pragma unroll
-    for (int i = 0; i < LA; ++i) tall_load(src_a(0), va[i], slot(0) + i * 4096);
+    for (int d = 0; d < D; ++d) {
 #pragma unroll
-    for (int i = 0; i < LB; ++i) tall_load(src_b(0), vb[i], slot(1) + i * 4096);
+        for (int i = 0; i < LA; ++i) tall_load(src_a(d), va[i], base + d * ASZ + i * 4096);
 #pragma unroll
-    for (int i = 0; i < LA; ++i) tall_load(src_a(1), va[i], slot(2) + i * 4096);
-#pragma unroll
-    for (int i = 0; i < LB; ++i) tall_load(src_b(1), vb[i], slot(3) + i * 4096);
-    vm_wait<LA + LB>();
+        for (int i = 0; i < LB; ++i) tall_load(src_b(d), vb[i], base + B0 + d * BSZ + i * 4096);
+    }
+    vm_wait<vm_count((D - 1) * (LA + LB))>();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     Frags f0, f1;
     [&]<int... I>(std::integer_sequence<int, I...>) {
-        (read_one(std::integral_constant<int, I>{}, f0, ra[0], rb[0] + SLOT), ...);
+        (read_one(std::integral_constant<int, I>{}, f0, ra[0], rb[0] + B0), ...);
     }(std::make_integer_sequence<int, TM + TN>{});
 
-    // one 32-key step: MFMA I, then behind every second one of the first 2 (TM + TN) an
-    // operand read of the next step, and behind the odd ones the step's DMA loads
+    // one 32-key step: MFMA I, then an operand read of the next step behind every RS-th and a
+    // DMA load behind every DS-th one
     auto mma_step = [&](Frags& f, Frags& g, uint32_t na, uint32_t nb, auto&& dma) {
         [&]<int... I>(std::integer_sequence<int, I...>) {
             ((acc[I / TN][I % TN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.b[I % TN], f.a[I / TN], acc[I / TN][I % TN],
                                                                             0, 0, 0),
-              read_one(std::integral_constant<int, (I % 2 == 0 ? I / 2 : 99)>{}, g, na, nb),
+              read_one(std::integral_constant<int, (I % RS == 0 ? I / RS : 99)>{}, g, na, nb),
               dma(std::integral_constant<int, I>{}), __builtin_amdgcn_sched_barrier(0)),
              ...);
         }(std::make_integer_sequence<int, TM * TN>{});
     };
+    uint32_t sa = 0, sb = B0;   // offsets of A(s) and B(s); A(s + D) goes one slab behind A(s)
     for (int s = 0; s < nk; ++s) {
-        const uint32_t sa = (uint32_t)(((2 * s) % 5) * SLOT), sb = (uint32_t)(((2 * s + 1) % 5) * SLOT);
-        const uint32_t xa = (uint32_t)(((2 * s + 2) % 5) * SLOT), xb = (uint32_t)(((2 * s + 3) % 5) * SLOT);
-        const unsigned char* ga = src_a(s + 2);
-        unsigned char* da = slot(2 * s + 4);
+        const uint32_t xa = sa == (uint32_t)(D * ASZ) ? 0u : sa + ASZ;
+        const uint32_t xb = sb == (uint32_t)(B0 + (D - 1) * BSZ) ? (uint32_t)B0 : sb + BSZ;
+        const unsigned char* ga = src_a(s + D);
+        unsigned char* da = base + (sa == 0 ? (uint32_t)(D * ASZ) : sa - ASZ);
         lgkm_wait<0>();
         tie(f0);
         mma_step(f0, f1, ra[1] + sa, rb[1] + sb, [&](auto ic) {
             constexpr int I = decltype(ic)::value;
-            if constexpr (I % 4 == 3 && I / 4 < LA) tall_load(ga, va[I / 4], da + (I / 4) * 4096);
+            if constexpr (I % DS == DS - 1 && I / DS < LA) tall_load(ga, va[I / DS], da + (I / DS) * 4096);
         });
         // slab s is in registers, slab s + 1 has landed for every wave
-        const unsigned char* gb = src_b(s + 2);
-        unsigned char* db = slot(2 * s + 5);
+        const unsigned char* gb = src_b(s + D);
+        unsigned char* db = base + sb;
         lgkm_wait<0>();
         tie(f1);
-        vm_wait<LA>();
+        vm_wait<vm_count((D - 1) * LA + (D - 2) * LB)>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         mma_step(f1, f0, ra[0] + xa, rb[0] + xb, [&](auto ic) {
             constexpr int I = decltype(ic)::value;
-            if constexpr (I % 4 == 3 && I / 4 < LB) tall_load(gb, vb[I / 4], db + (I / 4) * 4096);
+            if constexpr (I % DS == DS - 1 && I / DS < LB) tall_load(gb, vb[I / DS], db + (I / DS) * 4096);
         });
         pin_acc(acc);
+        sa = xa;
+        sb = xb;
     }
     lgkm_wait<0>();
     tie(f0);
@@ -608,13 +442,15 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restr
     __syncthreads();   // every wave is done with the operand slots
 
     // Epilogue, half of the wave's row blocks at a time: the partial tile goes through the
-    // wave's own 32 KB slot as fp32 (element e of tile (i, j): row 16 i + lane % 16, column
-    // 16 j + (lane / 16) * 4 + e; float4 chunk c of row r at c ^ (r % 16): distinct bank
-    // groups), so that the stores are whole row segments, 16 lanes to a row.
-    constexpr int H = TM / 2;
+    // wave's own quarter of the ring as fp32 (element e of tile (i, j): row 16 i + lane % 16, column 16 j +
+    // (lane / 16) * 4 + e; float4 chunk c of row r at c ^ (r % 16), over fewer chunks modulo
+    // theirs), so that the stores are whole row segments, LPR lanes to a row.
+    constexpr int SLOT = (B0 + D * BSZ) / 4 / 1024 * 1024;
+    constexpr int H = TM / 2, CPR = TN * 4, LPR = TN * 2, RPP = kWave / LPR;
+    static_assert(H * 16 * CPR * 16 <= SLOT, "half a wave's tile fits a slot");
     float4* const part = reinterpret_cast<float4*>(smem + wave * SLOT);
-    const int seg = lane & 15;
-    const int col = n0 + wn * (EPI == GEPI_SWIGLU ? 64 : 128) + seg * (EPI == GEPI_SWIGLU ? 4 : 8);
+    const int seg = lane % LPR;
+    const int col = n0 + wn * (EPI == GEPI_SWIGLU ? BN / 4 : BN / 2) + seg * (EPI == GEPI_SWIGLU ? 4 : 8);
     float bv[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e)
@@ -626,15 +462,15 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restr
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const f32x4_t x = acc[i0 + i][j];
-                part[(i * 16 + r16) * 32 + ((j * 4 + (lane >> 4)) ^ r16)] = make_float4(x[0], x[1], x[2], x[3]);
+                part[(i * 16 + r16) * CPR + ((j * 4 + (lane >> 4)) ^ (r16 % CPR))] = make_float4(x[0], x[1], x[2], x[3]);
             }
 #pragma unroll 4
-        for (int q = 0; q < H * 4; ++q) {
-            const int r = q * 4 + (lane >> 4);
-            const int row = m0 + wm * (BM / 2) + i0 * 16 + r, sw = r & 15;
+        for (int q = 0; q < H * 16 / RPP; ++q) {
+            const int r = q * RPP + lane / LPR;
+            const int row = m0 + wm * (BM / 2) + i0 * 16 + r, sw = (r & 15) % CPR;
             constexpr int NV = EPI == GEPI_SWIGLU ? 4 : 8;
             const int c0 = EPI == GEPI_SWIGLU ? (seg >> 2) * 8 + (seg & 3) : seg * 2;
-            const float4 x = part[r * 32 + (c0 ^ sw)], y = part[r * 32 + ((c0 + (EPI == GEPI_SWIGLU ? 4 : 1)) ^ sw)];
+            const float4 x = part[r * CPR + (c0 ^ sw)], y = part[r * CPR + ((c0 + (EPI == GEPI_SWIGLU ? 4 : 1)) ^ sw)];
             float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
 #pragma unroll
             for (int e = 0; e < NV; ++e) {
@@ -642,8 +478,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restr
                 else if (bias != nullptr) v[e] += bv[e];
             }
             if (row >= M) continue;
-            const size_t at = (size_t)row * ldc + col;
-            if constexpr (EPI == GEPI_F32) {
+            const size_t at = (size_t)(EPI == GEPI_PARTIAL ? (size_t)slice * M + row : (size_t)row) * ldc + col;
+            if constexpr (EPI == GEPI_F32 || EPI == GEPI_PARTIAL) {
                 float* o = reinterpret_cast<float*>(Cout) + at;
                 if (vec) {
                     if (col < N) {
@@ -676,11 +512,10 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(const bf16_t* __restr
 
 // ---------------------------------------------------------------------------------
 // K split over the waves of a workgroup: for launches whose tiles are too few to keep the
-// CUs busy by themselves. The pipelined kernel's four waves share every slab, so one wave
-// runs a single 32 x 32 MFMA tile (64 x 64 workgroup tiles) between two barriers: 512 x
-// 1536 -> 2048 takes 24 slabs at 0.5 us. Here each of KW waves owns a contiguous range of
-// the slabs and the whole 32 TM x 32 TN tile, with an S-deep LDS ring of its own: no
-// barrier until the partial tiles are summed through LDS, in wave order.
+// CUs busy by themselves. The slab kernel's four waves share every slab and meet at a barrier
+// for each. Here each of KW waves owns a contiguous range of the slabs and the whole 32 TM x
+// 32 TN tile, with an S-deep LDS ring of its own: no barrier until the partial tiles are
+// summed through LDS, in wave order.
 //  * A slab's operand reads are all issued one slab ahead of their MFMAs (two register
 //    sets); its LDS slot is refilled as soon as they have landed.
 //  * The weight rows are the MFMA's first operand, so a lane ends with four consecutive
@@ -924,25 +759,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     }
 }
 
-template <int BM, int BN, int S, int EPI>
-static void gemm_pipe_launch(int M, int N, int K, const bf16_t* A, const bf16_t* B, const bf16_t* bias, void* C,
-                             int ldc, hipStream_t stream) {
-    const int ocols = (EPI == GEPI_SWIGLU) ? BN / 2 : BN;
-    const int mt = (M + BM - 1) / BM, nt = (N + ocols - 1) / ocols;
-    const int grid = 8 * ((mt * nt + 7) / 8);
-    hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, S, EPI>), dim3(grid), dim3(kGemmThreads), 0, stream, A, B, bias, C,
-                       M, N, K, ldc, mt, nt, 1, K / kPBK);
-}
-
-template <int TM, int EPI>
+template <int TM, int TN, int D, int EPI>
 static void gemm_tall_launch(int M, int N, int K, const bf16_t* A, const bf16_t* B, const bf16_t* bias, void* C, int ldc,
-                             hipStream_t stream) {
-    const int ocols = (EPI == GEPI_SWIGLU) ? 128 : 256;
+                             hipStream_t stream, int kslices = 1, int slice_slabs = 1 << 30) {
+    const int ocols = (EPI == GEPI_SWIGLU) ? 16 * TN : 32 * TN;
     const int mt = (M + 32 * TM - 1) / (32 * TM), nt = (N + ocols - 1) / ocols;
-    const int grid = 8 * ((mt * nt + 7) / 8);
+    const int grid = 8 * ((mt * nt * kslices + 7) / 8);
     const int vec = N % 8 == 0 && ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
-    hipLaunchKernelGGL((gemm_tall_kernel<TM, EPI>), dim3(grid), dim3(256), 0, stream, A, B, bias, C, M, N, K, ldc, mt, nt,
-                       vec);
+    hipLaunchKernelGGL((gemm_tall_kernel<TM, TN, D, EPI>), dim3(grid), dim3(256), 0, stream, A, B, bias, C, M, N, K, ldc, mt, nt,
+                       vec, kslices, slice_slabs);
 }
 
 template <int TM, int TN, int KW, int S, int EPI, int WPE>
@@ -960,17 +785,16 @@ int prefill_cus();
 
 // Which tile of the K-split kernel (four waves) an unsliced launch takes: 0 none, 1: 32 x 32
 // (two workgroups per CU), 2: 64 x 32, 3: 64 x 64 (one per CU). It pays while every tile has
-// a CU of its own, smallest tile first, and for up to 32 rows at any width, where the larger
-// kernels' tiles are mostly padding. Up to 64 rows, or K below 8192 (beyond, the other
-// kernels' slices over workgroups are the better split); a wave wants 3 slabs (K of 768; a
-// 64 x 64 tile 5): the pipelined kernel's ring nearly holds shorter rows (40 x 512 -> 256 5.1
-// / 5.1, 40 x 256 -> 512 4.7 / 4.3, 40 x 768 -> 1024 4.9 / 6.3).
-// Measured on MI355X (us, this kernel / the pipelined one): 37 x 1536 -> 2048 4.4 / 9.9,
-// 19 x 896 -> 1152 4.3 / 6.7, 24 x 1536 -> 17920 14.2 / 20.0, 256 x 1536 -> 2048 6.2 / 10.0,
-// 100 x 3584 -> 4608 15.9 / 19.3, 512 x 1536 -> 2048 9.2 / 10.4, 24 x 8960 -> 1536 13.6 /
-// 17.4 (sliced); not: 1344 x 2048 -> 2560 37.9 / 25.2, 256 x 3584 -> 4608 28.7 / 30.1.
-// SwiGLU: 24 x 1536 -> 8960 14.6 / 16.7, 16 x 3584 -> 18944 48.1 / 67.8, 60 x 896 -> 4864
-// 7.6 / 9.9; not: 60 x 1536 -> 8960 22.4 / 17.9.
+// a CU of its own, smallest tile first, and for up to 32 rows at any width, where the slab
+// kernel's tiles are mostly padding. Up to 64 rows, or K below 8192 (beyond, slices over
+// workgroups are the better split); a wave wants 3 slabs (K of 768: 40 x 512 -> 256 5.1 us
+// against 5.1, 40 x 256 -> 512 4.7 / 4.3, 40 x 768 -> 1024 4.9 / 6.3), of a 64 x 64 tile 12.
+// Measured on MI355X (us, this kernel / the slab kernel's best tile): 200 x 3584 -> 3584 14.2
+// / 17.5, 100 x 3584 -> 4608 17.2 / 20, 256 x 1536 -> 2048 6.2 / 7.9; not: 512 x 1536 -> 2048
+// 9.8 / 8.0, 256 x 2048 -> 2560 10.2 / 8.7. Against the kernels before either: 37 x 1536 ->
+// 2048 4.4 / 9.9, 19 x 896 -> 1152 4.3 / 6.7, 24 x 1536 -> 17920 14.2 / 20.0, 24 x 8960 -> 1536
+// 13.6 / 17.4 (sliced). SwiGLU only up to 32 rows: 24 x 1536 -> 8960 14.6 / 16.7, 16 x 3584 ->
+// 18944 48.1 / 67.8; 60 x 896 -> 4864 7.6 / 5.8.
 static bool offsets_fit(long M, long b_rows, long K) {   // 32-bit byte offsets into both operands
     return M * K * 2 < 0x7fffffffL && b_rows * K * 2 < 0x7fffffffL;
 }
@@ -979,11 +803,11 @@ static int ksplit_tile(int M, int N, int K, bool swiglu) {
     if (K % kPBK != 0 || nk < 12 || !offsets_fit(M, swiglu ? 2L * N : N, K)) return 0;
     if (M <= 32) return 1;
     const long mt32 = (M + 31) / 32, mt64 = (M + 63) / 64, nt32 = ((long)N + 31) / 32, nt64 = ((long)N + 63) / 64;
-    if (swiglu) return M <= 64 && mt64 * nt32 <= cus ? 3 : 0;
+    if (swiglu) return 0;
     if (M > 64 && nk >= 128) return 0;
     if (mt32 * nt32 <= cus) return 1;
     if (mt64 * nt32 <= cus) return 2;
-    return mt64 * nt64 <= cus && nk >= 20 ? 3 : 0;
+    return mt64 * nt64 <= cus && nk >= 48 ? 3 : 0;
 }
 
 // Split-K plan for a plain (non-SwiGLU) projection with K % 64 == 0 and K >= 4096 whose
@@ -1000,16 +824,13 @@ static int ksplit_tile(int M, int N, int K, bool swiglu) {
 //    stays (39.5 against 49.1);
 //  * K < 8192 and a 64 x 64 tile (or fewer rows: a 32 x 32 tile) for every CU: unsliced
 //    (ksplit_tile): 700 x 4864 -> 896 24.2 -> 18.6;
-//  * tiles for at most a third of the CUs: as many slices as fill every CU once (at most
-//    8), one workgroup per CU over a 4-deep ring: 512 x 8960 -> 1536 33.6 -> 28.3 (5
-//    slices, against 8 slices over 2-deep rings, two workgroups per CU), 512 x 11008 ->
-//    2048 47.7 -> 39.1 (4 against 6), 768 x 8960 -> 1536 40.9 -> 39.7 (3 against 6);
-//  * up to 128 tiles: about 384 workgroups over 2-deep rings, two per CU (two slices over
-//    4-deep rings: 1024 x 8960 -> 1536 46.1 -> 50.9, 512 x 18944 -> 3584 101.2 -> 102.9).
+//  * else 128 x 128 tiles of the slab kernel, slices chosen the same way over two workgroups
+//    per CU (D 4 rings where one per CU is enough): 512 x 8960 -> 1536 29.0 -> 26.3 (5
+//    slices), 300 x 18944 -> 3584 71.6 -> 57.5 (6), 1024 x 8960 -> 1536 45.6 -> 41.0 (5),
+//    128 x 18944 -> 3584 35.1 -> 32.7 (8).
 struct SplitK {
     int ksplit = 0, kt_per = 0;
-    int tile = 0;       // tile of the K-split kernel (ksplit_tile), or 0: 128 x 128
-    bool deep = false;  // 128 x 128: 4-deep ring, one workgroup per CU (else 2-deep, two per CU)
+    int tile = 0;   // tile of the K-split kernel (ksplit_tile), or 0: 128 x 128 of the slab kernel
 };
 static SplitK splitk_plan(int M, int N, int K) {
     SplitK p;
@@ -1021,15 +842,18 @@ static SplitK splitk_plan(int M, int N, int K) {
     const bool small_w = (long)N * K * 2 <= (64L << 20);
     const long mt32 = (M + 31) / 32, mt64 = (M + 63) / 64, nt32 = (N + 31) / 32, nt64 = (N + 63) / 64;
     const int most = std::min(8, nk / 16);
+    // slices that leave the fewest slabs to the busiest CU, over at most `slots` workgroups
+    auto fill_slices = [&](long t, long slots) {
+        int ks = 1;
+        for (int n = 2; n <= most && t * n <= slots; ++n)
+            if ((t * n + cus - 1) / cus * ks <= (t * ks + cus - 1) / cus * n) ks = n;
+        return ks;
+    };
     int ks = 0;
     if (M <= 32 || (M <= 64 && small_w)) {
         p.tile = M <= 32 ? 1 : 2;
         const long t = M <= 32 ? mt32 * nt32 : mt64 * nt32, slots = (M <= 32 ? 2L : 1L) * cus;
-        ks = 1;
-        for (int n = 2; n <= most && t * n <= slots; ++n) {   // fewest (workgroups on a CU) / n
-            const long a = (t * n + cus - 1) / cus * ks, b = (t * ks + cus - 1) / cus * n;
-            if (a <= b) ks = n;
-        }
+        ks = fill_slices(t, slots);
     } else if (nk < 128 && mt32 * nt32 <= cus) {
         return p;
     } else if (2 * mt64 * nt64 <= cus && small_w) {
@@ -1038,14 +862,7 @@ static SplitK splitk_plan(int M, int N, int K) {
     } else if (nk < 128 && mt64 * nt64 <= cus) {
         return p;
     } else {
-        const int fill = (int)std::min<long>(most, cus / tiles);
-        if (fill >= 3) {
-            ks = fill;
-            p.deep = true;
-        } else {
-            ks = (int)std::min<long>(8, (384 + tiles - 1) / tiles);
-            ks = std::min(ks, nk / 16);
-        }
+        ks = fill_slices(tiles, 2L * cus);
     }
     if (ks < 2 || (p.tile != 0 && !offsets_fit(M, N, K))) return SplitK{};
     p.kt_per = (nk + ks - 1) / ks;
@@ -1062,23 +879,54 @@ static size_t splitk_bytes(int M, int N, int K) {
 static void gemm_splitk_launch(int M, int N, int K, const bf16_t* A, const bf16_t* B, const bf16_t* bias, void* C,
                                bool f32out, float* part, const SplitK& p, hipStream_t stream) {
     const int mt = (M + 127) / 128, nt = (N + 127) / 128;
-    const int grid = 8 * ((mt * nt * p.ksplit + 7) / 8);
     if (p.tile == 1)
         gemm_ksplit_launch<1, 1, 4, 2, GEPI_PARTIAL, 2>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     else if (p.tile == 2)
         gemm_ksplit_launch<2, 1, 4, 2, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     else if (p.tile == 3)
         gemm_ksplit_launch<2, 2, 4, 2, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
-    else if (p.deep)
-        hipLaunchKernelGGL((gemm_pipe_kernel<128, 128, 4, GEPI_PARTIAL>), dim3(grid), dim3(kGemmThreads), 0, stream, A,
-                           B, nullptr, part, M, N, K, N, mt, nt, p.ksplit, p.kt_per);
+    else if (mt * nt * p.ksplit <= prefill_cus())
+        gemm_tall_launch<4, 4, 4, GEPI_PARTIAL>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     else
-        hipLaunchKernelGGL((gemm_pipe_kernel<128, 128, 2, GEPI_PARTIAL>), dim3(grid), dim3(kGemmThreads), 0, stream, A,
-                           B, nullptr, part, M, N, K, N, mt, nt, p.ksplit, p.kt_per);
+        gemm_tall_launch<4, 4, 2, GEPI_PARTIAL>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     const size_t quads = (size_t)M * N / 4;
     const dim3 rgrid((unsigned)((quads + 255) / 256));
     if (f32out) hipLaunchKernelGGL((gemm_splitk_reduce_kernel<true>), rgrid, dim3(256), 0, stream, part, p.ksplit, M, N, bias, C);
     else hipLaunchKernelGGL((gemm_splitk_reduce_kernel<false>), rgrid, dim3(256), 0, stream, part, p.ksplit, M, N, bias, C);
+}
+
+// Tiles of the slab kernel and what a launch of them takes, fitted to sweeps on MI355X over
+// weights that rotate through the memory-side cache (us). A launch is rounds of 256 x occ
+// resident workgroups. A round of c tiles per CU takes s us a 64-key slab: s0 at one tile on
+// few CUs rising to s1 at one on each (the same work draws more power, and the clock drops),
+// and from s1b just above one per CU to s2 at occ per CU; plus o us before the first and
+// after the last slab, which a next round hides where two workgroups share a CU. The deep
+// rings (D 3 and 4) carry launches of at most a tile per CU over the latency of the
+// memory-side cache (300 x 3584 -> 4608: 128 x 64 tiles 36.9 us over 2 slabs, 20.1 over 4);
+// where two workgroups share the LDS, the second one does.
+struct TallTile {
+    int tm, tn, occ;
+    double o, s0, s1, s1b, s2;
+};
+constexpr TallTile kTallTiles[] = {
+    {8, 8, 1, 8.0, 1.05, 1.42, 0, 0},         // 256 x 256, D 2
+    {6, 8, 1, 7.4, 0.72, 1.06, 0, 0},         // 192 x 256, D 2
+    {6, 4, 1, 4.7, 0.47, 0.56, 0, 0},         // 192 x 128, D 3
+    {4, 4, 1, 4.2, 0.36, 0.46, 0, 0},         // 128 x 128, D 4
+    {4, 4, 2, 4.5, 0.47, 0.50, 0.68, 0.92},   // 128 x 128, D 2
+    {4, 2, 1, 3.6, 0.235, 0.28, 0, 0},        // 128 x 64, D 4
+    {4, 2, 2, 3.6, 0.38, 0.38, 0.45, 0.57},   // 128 x 64, D 2
+    {2, 4, 2, 3.6, 0.235, 0.29, 0.75, 0.90},  // 64 x 128, D 3
+    {2, 2, 2, 2.7, 0.21, 0.225, 0.38, 0.46},  // 64 x 64, D 4
+};
+static double tall_cost(const TallTile& t, long tiles, int slabs) {
+    const double cus = 256;
+    auto slab = [&](double c) {
+        return c <= 1 ? t.s0 + (t.s1 - t.s0) * c : t.s1b + (t.s2 - t.s1b) * (c - 1) / (t.occ - 1);
+    };
+    const long full = tiles / (256 * t.occ), rem = tiles % (256 * t.occ);
+    const double o = t.occ == 1 ? t.o : 0;
+    return (t.occ == 1 ? 0 : t.o) + full * (o + slabs * slab(t.occ)) + (rem ? o + slabs * slab(rem / cus) : 0);
 }
 
 template <int EPI>
@@ -1092,7 +940,7 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
     const dim3 block(kGemmThreads);
     const int tile_knob = kernel_knob(EFM_KNOB_GEMM_TILE);
     const long b_rows = (EPI == GEPI_SWIGLU) ? 2L * N : (long)N;
-    const bool wide_ok = K % kPBK == 0 && offsets_fit(M, b_rows, K);
+    const bool slab_ok = K % kPBK == 0 && offsets_fit(M, b_rows, K);
     if (tile_knob == 0) {
         switch (ksplit_tile(M, N, K, EPI == GEPI_SWIGLU)) {
             case 1:
@@ -1110,53 +958,26 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
             default: break;
         }
     }
-    if (wide_ok && tile_knob != 1) {
-        // Rounds of resident workgroups times the cost of one round: 100 for 192 x 256 tiles
-        // (one per CU), 127 for 256 x 256, 106 for 512 tiles of 128 x 128 (two per CU; 96
-        // below K 1536, where the larger tiles' first loads and epilogue weigh more), 75 for
-        // a last round of one per CU. Measured on MI355X (us, 192 / 256 / 128 x 128): 4096 x
-        // 3584 -> 4608 129 / 162 / 161, 4096 x 3584 -> 3584 123 / 91 / 125, 4096 x 3584 -> 2 x
-        // 18944 909 / 855 / 1286, 1344 x 2048 -> 2 x 11008 122 / 146 / 147, 4096 x 1536 -> 2048
-        // 32.7 / 42.8 / 33.9, 1344 x 2048 -> 2560 35.3 / 48.0 / 25.2, 700 x 896 -> 2 x 4864 21.6
-        // / 26.2 / 20.4. The choice is the fastest or within 3 % of it at all 27 shapes swept
-        // (1.5B, 3B, 7B and 0.5B projections at 300 to 16384 rows).
-        const long cus = 256, t128 = tiles(128, 128);
-        const long two = K < 1536 ? 96 : 106, rem = t128 % (2 * cus);
-        const long c128 = t128 / (2 * cus) * two + (rem == 0 ? 0 : rem <= cus ? 75 : two);
-        const long c192 = (tiles(192, 256) + cus - 1) / cus * 100, c256 = (tiles(256, 256) + cus - 1) / cus * 127;
-        if (tile_knob == 3 || (tile_knob == 0 && c192 < std::min(c256, c128))) {
-            gemm_tall_launch<6, EPI>(M, N, K, A, B, bias, C, ldc, stream);
-            return check_launch("gemm_bf16");
-        }
-        if (tile_knob == 2 || c256 < c128) {
-            gemm_tall_launch<8, EPI>(M, N, K, A, B, bias, C, ldc, stream);
-            return check_launch("gemm_bf16");
-        }
-    }
-    if (K % kPBK == 0) {
-        // Tile choice from sweeps of the prefill shapes on MI355X: 128 x 128 double-
-        // buffered (two workgroups per CU) once there are >= 1.5 tiles per CU (>= 1 for
-        // SwiGLU); K >= 4096 with 129 to one-per-CU 128 x 128 tiles: those tiles over a
-        // 4-deep ring, one workgroup per CU (1344 x 11008 -> 2048 129.2 -> 106.6 us,
-        // 1024 x 18944 -> 3584 237.6 -> 182.8; at 132 tiles, 1344 x 8960 -> 1536, 80.2 ->
-        // 86.1); else 128 x 64 over a 3-deep ring (two per CU; 1024 x 1536 -> 2048 20.2 ->
-        // 18.3 against the 2-deep ring, no shape slower); else 64 x 64 (64 x 128 for
-        // SwiGLU) with shallow pipelines. Every tile shape sums each output over K in the
-        // same order: results are bit-identical whichever is chosen.
-        if constexpr (EPI != GEPI_SWIGLU) {
-            const long t = tiles(128, 128);
-            if (K / kPBK >= 64 && t > 128 && t < 384 && t <= prefill_cus()) {
-                gemm_pipe_launch<128, 128, 4, EPI>(M, N, K, A, B, bias, C, ldc, stream);
-                return check_launch("gemm_bf16");
+    if (slab_ok) {
+        // the cheapest tile (EFM_KNOB_GEMM_TILE 1: of the tiles up to 128 x 128)
+        int pick = tile_knob == 3 ? 1 : 0;
+        if (tile_knob < 2) {
+            double best = 0;
+            for (int i = tile_knob == 1 ? 3 : 0; i < (int)std::size(kTallTiles); ++i) {
+                const double c = tall_cost(kTallTiles[i], tiles(32 * kTallTiles[i].tm, 32 * kTallTiles[i].tn), K / kPBK);
+                if (best == 0 || c < best) best = c, pick = i;
             }
         }
-        if (tiles(128, 128) >= ((EPI == GEPI_SWIGLU) ? 256 : 384)) {
-            gemm_pipe_launch<128, 128, 2, EPI>(M, N, K, A, B, bias, C, ldc, stream);
-        } else if constexpr (EPI == GEPI_SWIGLU) {
-            gemm_pipe_launch<64, 128, 3, EPI>(M, N, K, A, B, bias, C, ldc, stream);
-        } else {
-            if (tiles(128, 64) >= 256) gemm_pipe_launch<128, 64, 3, EPI>(M, N, K, A, B, bias, C, ldc, stream);
-            else gemm_pipe_launch<64, 64, 4, EPI>(M, N, K, A, B, bias, C, ldc, stream);
+        switch (pick) {
+            case 0: gemm_tall_launch<8, 8, 2, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 1: gemm_tall_launch<6, 8, 2, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 2: gemm_tall_launch<6, 4, 3, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 3: gemm_tall_launch<4, 4, 4, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 4: gemm_tall_launch<4, 4, 2, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 5: gemm_tall_launch<4, 2, 4, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 6: gemm_tall_launch<4, 2, 2, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 7: gemm_tall_launch<2, 4, 3, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
+            case 8: gemm_tall_launch<2, 2, 4, EPI>(M, N, K, A, B, bias, C, ldc, stream); break;
         }
         return check_launch("gemm_bf16");
     }

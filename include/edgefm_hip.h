@@ -70,10 +70,9 @@ int efm_init(void);
  *                              4-wave (128-row) or 8-wave (256-row) workgroups; 2: the
  *                              prefill kernel runs 2-wave (64-row) workgroups (the Sage
  *                              kernel treats 2 as 4)
- *   EFM_KNOB_GEMM_TILE         prefill GEMM kernel (K % 64 == 0): 1 the two-workgroup-
- *                              per-CU 128 x 128 / 128 x 64 / 64 x 64 kernel, 2 the
- *                              one-workgroup-per-CU 256 x 256 kernel, 3 the same kernel
- *                              with 192 x 256 tiles
+ *   EFM_KNOB_GEMM_TILE         prefill GEMM kernel (K % 64 == 0): 1 the tiles up to 128 x
+ *                              128, 2 the one-workgroup-per-CU 256 x 256 tile, 3 the
+ *                              192 x 256 tile (none splits K over the waves)
  *   EFM_KNOB_FRONT_WAIT_TIMEOUT 1: efm_decode_norm_qkv_attention launches whose attention
  *                              workgroups wait for a tag that no projected word carries,
  *                              with a 64-poll limit: every wait gives up, the launch
