@@ -325,24 +325,21 @@ __global__ __launch_bounds__(256, tall_lds(TM, TN, D) <= 80 * 1024 ? 2 : 1) void
 #pragma unroll
         for (int i = 0; i < LA; ++i) {
             const int r = (i * 4 + wave) * 8 + rr;
-            va[i] = (uint32_t)((min(m0 + r, M - 1) * K + ((cs ^ pipe_swz(r)) << 3)) * 2);
+            va[i] = (uint32_t)(min(r, M - 1 - m0) * K + ((cs ^ pipe_swz(r)) << 3)) * 2;
         }
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
             const int r = (i * 4 + wave) * 8 + rr;
-            int row;
-            if (EPI == GEPI_SWIGLU) {   // 16-row blocks of up (even) and gate (odd) weights
-                const int blk = r / 16;
-                row = min(n0 + (blk / 2) * 16 + r % 16, N - 1) + (blk % 2) * N;
-            } else {
-                row = min(n0 + r, N - 1);
-            }
-            vb[i] = (uint32_t)((row * K + ((cs ^ pipe_swz(r)) << 3)) * 2);
+            // SwiGLU: 16-row blocks of up (even) and gate (odd) weights, a wave's all of one kind
+            const int row = EPI == GEPI_SWIGLU ? r / 32 * 16 + r % 16 : r;
+            vb[i] = (uint32_t)(min(row, N - 1 - n0) * K + ((cs ^ pipe_swz(r)) << 3)) * 2;
         }
     }
     const int s0 = slice * slice_slabs, nk = min(K / kPBK - s0, slice_slabs);
-    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A) + (size_t)s0 * kPRow;
-    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B) + (size_t)s0 * kPRow;
+    // 64-bit bases at the tile's first rows, 32-bit byte offsets within the tile
+    const int b0 = n0 + (EPI == GEPI_SWIGLU && (wave & 2) ? N : 0);
+    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A + (size_t)m0 * K) + (size_t)s0 * kPRow;
+    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B + (size_t)b0 * K) + (size_t)s0 * kPRow;
     // slabs past the end repeat the last one (never read, so that every step issues the same
     // loads)
     unsigned char* const base = smem + wave * 1024;
@@ -553,37 +550,31 @@ __global__ __launch_bounds__(KW * kWave, WPE) void gemm_ksplit_kernel(const bf16
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
 
-    // DMA sources: 32-bit byte offsets (the host keeps both operands under 2 GB); rows past
-    // the matrix repeat its last row (their outputs are not stored)
+    // DMA sources: 64-bit bases at the tile's first rows, 32-bit byte offsets within the
+    // tile; rows past the matrix repeat its last row (their outputs are not stored)
     uint32_t voff[LPS];
     {
         const int rr = lane >> 3, cs = lane & 7;
 #pragma unroll
         for (int i = 0; i < LPS; ++i) {
             const int r = i * 8 + rr;
-            int row;
-            if (i < LA) {
-                row = min(m0 + r, M - 1);
-            } else {
-                const int br = r - BM;
-                const int gate = EPI == GEPI_SWIGLU && br >= OC;
-                row = min(n0 + br - gate * OC, N - 1) + gate * N;
-            }
-            voff[i] = (uint32_t)((row * K + ((cs ^ pipe_swz(r)) << 3)) * 2);
+            const int row = i < LA ? min(r, M - 1 - m0) : min((r - BM) % OC, N - 1 - n0);
+            voff[i] = (uint32_t)(row * K + ((cs ^ pipe_swz(r)) << 3)) * 2;
         }
     }
     unsigned char* const ring = smem + wave * RING;
     const int s0 = slice * slice_slabs, nk = min(K / kPBK - s0, slice_slabs);
     const int k_begin = s0 + wave * nk / KW, n_slabs = s0 + (wave + 1) * nk / KW - k_begin;
-    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A) + (size_t)k_begin * kPRow;
-    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B) + (size_t)k_begin * kPRow;
+    const unsigned char* pa = reinterpret_cast<const unsigned char*>(A + (size_t)m0 * K) + (size_t)k_begin * kPRow;
+    const unsigned char* pb = reinterpret_cast<const unsigned char*>(B + (size_t)n0 * K) + (size_t)k_begin * kPRow;
+    const size_t gate = (size_t)N * K * 2;   // SwiGLU: from the up to the gate weights
     auto issue = [&](int slab) {
         const unsigned char* sa = pa + slab * kPRow;
         const unsigned char* sb = pb + slab * kPRow;
         unsigned char* dst = ring + (slab % S) * STAGE;
 #pragma unroll
         for (int i = 0; i < LPS; ++i)
-            __builtin_amdgcn_global_load_lds(static_cast<const void*>((i < LA ? sa : sb) + voff[i]),
+            __builtin_amdgcn_global_load_lds(static_cast<const void*>((i < LA ? sa : i < LA + OC / 8 ? sb : sb + gate) + voff[i]),
                                              (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, 0, 0);
     };
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)ring);
@@ -691,7 +682,7 @@ __global__ __launch_bounds__(KW * kWave, WPE) void gemm_ksplit_kernel(const bf16
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += col + e < N ? bf16_to_f32(bias[col + e]) : 0.f;
         }
-        const size_t at = (size_t)(EPI == GEPI_PARTIAL ? slice * M + row : row) * ldc + col;
+        const size_t at = (size_t)(EPI == GEPI_PARTIAL ? (size_t)slice * M + row : (size_t)row) * ldc + col;
         if (EPI == GEPI_F32 || EPI == GEPI_PARTIAL) {
             float* o = reinterpret_cast<float*>(Cout) + at;
             if (vec) {
@@ -795,12 +786,10 @@ int prefill_cus();
 // 2048 4.4 / 9.9, 19 x 896 -> 1152 4.3 / 6.7, 24 x 1536 -> 17920 14.2 / 20.0, 24 x 8960 -> 1536
 // 13.6 / 17.4 (sliced). SwiGLU only up to 32 rows: 24 x 1536 -> 8960 14.6 / 16.7, 16 x 3584 ->
 // 18944 48.1 / 67.8; 60 x 896 -> 4864 7.6 / 5.8.
-static bool offsets_fit(long M, long b_rows, long K) {   // 32-bit byte offsets into both operands
-    return M * K * 2 < 0x7fffffffL && b_rows * K * 2 < 0x7fffffffL;
-}
+constexpr int kMaxSlabK = 1 << 21;   // 32-bit byte offsets into the 256 rows of a tile
 static int ksplit_tile(int M, int N, int K, bool swiglu) {
     const int cus = prefill_cus(), nk = K / kPBK;
-    if (K % kPBK != 0 || nk < 12 || !offsets_fit(M, swiglu ? 2L * N : N, K)) return 0;
+    if (K % kPBK != 0 || nk < 12 || K > kMaxSlabK) return 0;
     if (M <= 32) return 1;
     const long mt32 = (M + 31) / 32, mt64 = (M + 63) / 64, nt32 = ((long)N + 31) / 32, nt64 = ((long)N + 63) / 64;
     if (swiglu) return 0;
@@ -834,7 +823,7 @@ struct SplitK {
 };
 static SplitK splitk_plan(int M, int N, int K) {
     SplitK p;
-    if (K % kPBK != 0 || N % 4 != 0) return p;
+    if (K % kPBK != 0 || N % 4 != 0 || K > kMaxSlabK) return p;
     const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
     const int nk = K / kPBK;
     if (tiles > 128 || nk < 64) return p;
@@ -864,7 +853,7 @@ static SplitK splitk_plan(int M, int N, int K) {
     } else {
         ks = fill_slices(tiles, 2L * cus);
     }
-    if (ks < 2 || (p.tile != 0 && !offsets_fit(M, N, K))) return SplitK{};
+    if (ks < 2) return SplitK{};
     p.kt_per = (nk + ks - 1) / ks;
     p.ksplit = (nk + p.kt_per - 1) / p.kt_per;
     return p;
@@ -939,8 +928,7 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
     };
     const dim3 block(kGemmThreads);
     const int tile_knob = kernel_knob(EFM_KNOB_GEMM_TILE);
-    const long b_rows = (EPI == GEPI_SWIGLU) ? 2L * N : (long)N;
-    const bool slab_ok = K % kPBK == 0 && offsets_fit(M, b_rows, K);
+    const bool slab_ok = K % kPBK == 0 && K <= kMaxSlabK;
     if (tile_knob == 0) {
         switch (ksplit_tile(M, N, K, EPI == GEPI_SWIGLU)) {
             case 1:

@@ -639,6 +639,38 @@ def test_gemm_tall_kernel_edges(gpu, knob, m, k, n, kind):
 
 
 @pytest.mark.parametrize("m,k,n,kind", [
+    pytest.param(20, 16384, 81921, "bf16", id="k_split"),
+    pytest.param(40, 16384, 81921, "bf16", id="slab"),
+    pytest.param(40, 98304, 16384, "bf16", id="split_k"),
+    pytest.param(20, 3584, 160000, "swiglu", id="k_split_swiglu"),
+    pytest.param(70, 3584, 160000, "swiglu", id="slab_swiglu"),
+])
+def test_gemm_operands_past_2gb(gpu, m, k, n, kind):
+    """Weights of more than 2^31 bytes: the first and last output columns of the tiled kernels
+    against fp32 products (both round an fp32 sum to bf16; the sums differ by a few ulps of
+    fp32 times sqrt(k), far below bf16's 2^-8)."""
+    nw = 2 * n if kind == "swiglu" else n
+    assert nw * k * 2 > 1 << 31
+    g = torch.Generator(device=gpu).manual_seed(m)
+    x = torch.empty(m, k, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    w = torch.empty(nw, k, dtype=torch.bfloat16, device=gpu).normal_(std=k ** -0.5, generator=g)
+    y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu)
+    if kind == "swiglu":
+        C.call("efm_fused_gate_up_swiglu", m, k, n, ptr(x), ptr(w), ptr(y), stream())
+    else:
+        ws = torch.empty(max(C.load().efm_linear_workspace_bytes(m, k, n), 256), dtype=torch.uint8, device=gpu)
+        C.call("efm_linear_ws", m, k, n, ptr(x), ptr(w), None, ptr(y), C.EFM_DTYPE_BF16, ptr(ws), ws.numel(), stream())
+    torch.cuda.synchronize()
+    for c in (slice(0, 256), slice(n // 2, n // 2 + 256), slice(n - 256, n)):
+        ref = x.float() @ w[:n][c].float().T
+        if kind == "swiglu":
+            up, gate = ref.bfloat16().float(), (x.float() @ w[n:][c].float().T).bfloat16().float()
+            ref = torch.nn.functional.silu(gate) * up
+        torch.testing.assert_close(y[:, c].float(), ref, rtol=2 ** -6, atol=2 ** -6)
+    assert not y.isnan().any()
+
+
+@pytest.mark.parametrize("m,k,n,kind", [
     pytest.param(512, 8960, 1536, "bf16", id="c2_down"),
     pytest.param(300, 18944, 3584, "bf16", id="7b_down"),
     pytest.param(300, 4096, 1000, "bias", id="ragged_bias"),
