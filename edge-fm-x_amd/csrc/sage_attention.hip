@@ -13,9 +13,13 @@
 //
 // Three launches: K column sums (float64; the attention entry point: per KV head and row
 // slice, coalesced rows; efm_sage_quantize: per KV head and 8 channels), block
-// quantisation of Q and K (one workgroup per block x head), attention (one workgroup =
-// 128 query rows of one head, 64-key tiles staged in LDS as int8 K and transposed V).
+// quantisation of Q and K (one workgroup per block x head), attention. The attention
+// kernels: keys split over waves (head_dim 64; few query blocks), shared tile stream (head_dim
+// 128), both quantising Q themselves, and the register-staged one (128 query rows of one head,
+// 64-key tiles staged in LDS as int8 K and transposed V): the others' reference in the tests
+// and the path of operands that their loads cannot take.
 #include "attn_pipe.hpp"
+#include "attn_split.hpp"
 #include "common.hpp"
 
 #include <algorithm>
@@ -24,8 +28,6 @@
 
 namespace efm {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef int int32x4_t __attribute__((ext_vector_type(4)));
 typedef int int32x16_t __attribute__((ext_vector_type(16)));
 
@@ -244,12 +246,6 @@ struct SageArgs {
     float scale_log2;
 };
 
-union Pack8 {
-    bf16x8_t v;
-    uint4 u;
-    uint32_t w[4];
-};
-
 template <int HD>
 __global__ __launch_bounds__(kSageThreads) void sage_attn_kernel(SageArgs a) {
     constexpr int KS8 = HD / 32;       // int8 MFMA k-steps
@@ -423,14 +419,6 @@ constexpr int kSPVTile = kSPKV * kSPHD * 2;      // bf16 bytes
 constexpr int kSPStage = kSPKTile + kSPVTile;
 constexpr float kSPLazy = 8.0f;
 constexpr float kMagic = 12582912.0f;   // 1.5 * 2^23: its float ulp is 1
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
-// Sum of the two bf16 halves of `w` added to acc (fp32).
-__device__ __forceinline__ float add_bf16_pair(uint32_t w, float acc) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w),
-                                           __builtin_bit_cast(bf16x2_t, 0x3f803f80u), acc, false);
-}
 
 template <int WAVES, int S>
 __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void sage_attn_pipe_kernel(SageArgs a, int nqt) {
@@ -759,8 +747,355 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void sage_attn_pipe_kernel(S
         }
 }
 
+// ---------------------------------------------------------------------------------
+// Keys split over the waves of a workgroup (attn_split.hpp's scheme on int8 K): head_dim 64,
+// and launches whose 32-row query blocks are few. One workgroup is one 32-row block of one
+// head; its KW waves take every KW-th key tile (32 keys at head_dim 128, 64 at 64: 4 KB of K
+// and 8 KB of V), each through LDS of its own, and merge their partial (max, sum, output) at
+// the end. Such a launch is bound by one wave's serial chain, not by the matrix cores.
+//  * Q is quantised here: the scale is that of the 128-row block around the 32 rows, so each
+//    wave takes the max of one 32-row quarter (an L2 read; the other quarters' workgroups
+//    read the same rows).
+//  * Score arithmetic as in the pipelined kernel above.
+//  Measured (us, whole operator, before / after; head_dim 64 ran the register-staged kernel):
+//  head_dim 64, 14/2 heads: S 100 20.5 / 13.3, 333 behind 500 60.5 / 17.4, 700 51.9 / 17.6, 4096
+//  294 / 65.5; head_dim 128: 12/2 heads S 1000 35.3 / 26.4, 37 behind 8000 173 / 55.6.
+// ---------------------------------------------------------------------------------
+template <int HD, int KW>
+__global__ __launch_bounds__(KW * 64, 2) void sage_attn_split_kernel(SageArgs a, SplitGrid sg, int nqt) {
+    typedef SplitTile<HD> T;   // V tile
+    constexpr int KT = T::kKeys, NH = KT / 32, KS8 = HD / 32, DT = HD / 32, KB = KT / 16;
+    constexpr int KBYTES = KT * HD, KLOADS = KBYTES / 1024, VLOADS = T::kLoads;
+    constexpr int KCH = HD / 16, KROWS = 64 / KCH;   // 16-byte chunks per K row, rows per wave load
+    constexpr int CPR = HD / 4;                      // float4 chunks per output row
+    constexpr int SLOT = KBYTES + T::kBytes > 32 * HD * 4 ? KBYTES + T::kBytes : 32 * HD * 4;
+    static_assert(KW % 4 == 0 && KLOADS == 4 && VLOADS == 8 && kSageBlock % KT == 0, "tile geometry");
+    __shared__ __align__(1024) unsigned char smem[KW * SLOT];
+    __shared__ float ml[2][KW][32];
+    __shared__ float s_qmax[KW];
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+    const int ql = lane % 32, hh = lane / 32;
+    int qt, head, kvh;
+    if (sg.hkv_log2 >= 0) {
+        const int x = (int)blockIdx.x;
+        kvh = x & ((1 << sg.hkv_log2) - 1);
+        head = kvh * sg.group + (x >> 3);
+        qt = nqt - 1 - (((int)blockIdx.y << (3 - sg.hkv_log2)) + ((x & 7) >> sg.hkv_log2));
+        if (qt < 0) return;
+    } else {
+        head = (int)blockIdx.x;
+        kvh = head / sg.group;
+        qt = nqt - 1 - (int)blockIdx.y;
+    }
+    const int q0 = qt * 32, qi = q0 + ql;
+    const int diag = a.L - a.S;
+    const int kv_end = a.causal ? min(a.L, min(a.S - 1, q0 + 31) + diag + 1) : a.L;
+    const int ntiles = (kv_end + KT - 1) / KT;
+
+    // this lane's row of the block and of the quarter whose max this wave takes, d = ks*32 +
+    // hh*16 + 0..15 (the int8 B-operand layout), requested first; rows past the end are 0
+    uint4 qu[KS8][2], mu[KS8][2];
+    {
+        auto load = [&](uint4 (&u)[KS8][2], int row) {
+            const bool ok = row < a.S;
+            const bf16_t* qp = a.q + (size_t)(ok ? row : 0) * a.q_sn + (size_t)head * a.q_sh + hh * 16;
+#pragma unroll
+            for (int ks = 0; ks < KS8; ++ks)
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+                    u[ks][x] = ok ? *reinterpret_cast<const uint4*>(qp + ks * 32 + x * 8) : make_uint4(0, 0, 0, 0);
+        };
+        load(qu, qi);
+        load(mu, q0 / kSageBlock * kSageBlock + (wave % 4) * 32 + ql);
+    }
+
+    const char* kbase = reinterpret_cast<const char*>(a.k8) + (size_t)kvh * HD;
+    const char* vbase = reinterpret_cast<const char*>(a.v + (size_t)kvh * a.v_sh);
+    unsigned char* const kslot = smem + wave * SLOT;
+    unsigned char* const vslot = kslot + KBYTES;
+    // 16 rows of one chunk in distinct bank groups: 128-byte rows as attn_pipe::k8_off, of
+    // 64-byte rows four fill the 256-byte bank period
+    auto k_swz = [](int row) { return HD == 128 ? (row >> 1) & 7 : (row >> 2) & 3; };
+    auto issue_k = [&](int t) {
+        const int k0 = t * KT, ksn = a.Hkv * HD;
+        const char* t0 = kbase + (size_t)k0 * ksn;
+#pragma unroll
+        for (int i = 0; i < KLOADS; ++i) {
+            const int row = i * KROWS + lane / KCH, c = (lane % KCH) ^ k_swz(row);
+            const int r = min(row, a.L - 1 - k0);   // rows past the end read the last row
+            __builtin_amdgcn_global_load_lds(static_cast<const void*>(t0 + (uint32_t)(r * ksn + c * 16)),
+                                             (__attribute__((address_space(3))) void*)(kslot + i * 1024), 16, 0, 0);
+        }
+    };
+    auto issue_v = [&](int t) {
+        const int k0 = t * KT;
+        const char* t0 = vbase + (size_t)k0 * a.v_sn * 2;
+#pragma unroll
+        for (int i = 0; i < VLOADS; ++i) {
+            const int row = i * T::kRows + lane / T::kChunks, c = (lane % T::kChunks) ^ T::v_swz(row);
+            const int r = min(row, a.L - 1 - k0);
+            __builtin_amdgcn_global_load_lds(static_cast<const void*>(t0 + (uint32_t)(r * a.v_sn + c * 8) * 2u),
+                                             (__attribute__((address_space(3))) void*)(vslot + i * 1024), 16, 0, 0);
+        }
+    };
+    if (wave < ntiles) {
+        issue_k(wave);
+        issue_v(wave);
+    }
+
+    int32x4_t qf[KS8];
+    float qscale;
+    {
+        float amax = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS8; ++ks)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                float f[8];
+                unpack8(mu[ks][x], f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(f[e]));
+            }
+        amax = wave_max(amax);
+        if (lane == 0) s_qmax[wave] = amax;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const float m = fmaxf(fmaxf(s_qmax[0], s_qmax[1]), fmaxf(s_qmax[2], s_qmax[3]));
+        const float scale = (m > 0.f) ? m / 127.0f : 1.0f;
+        qscale = (qi < a.S) ? scale : 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS8; ++ks) {
+            float f[16];
+            unpack8(qu[ks][0], &f[0]);
+            unpack8(qu[ks][1], &f[8]);
+            uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float qv = fminf(fmaxf(rintf(f[e] / scale), -127.f), 127.f);
+                w[e / 4] |= ((uint32_t)((int)qv & 0xff)) << (8 * (e % 4));
+            }
+            qf[ks] = int32x4_t{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        }
+    }
+
+    f32x16_t oacc[DT];
+#pragma unroll
+    for (int tt = 0; tt < DT; ++tt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[tt][e] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;   // -inf until the wave meets a key that the row sees
+    int32x16_t magic;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) magic[e] = __float_as_int(kMagic);
+
+    const uint32_t lk = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)kslot);
+    uint32_t ka[KS8], va[DT];
+#pragma unroll
+    for (int ks = 0; ks < KS8; ++ks) ka[ks] = lk + (uint32_t)(ql * HD + (((ks * 2 + hh) ^ k_swz(ql)) << 4));
+    {
+        // V^T operand (ds_read_b64_tr_b16, see attn_pipe.hpp)
+        const int g = lane >> 4, j = lane & 15, row = (g >> 1) * 4 + (j >> 2);
+#pragma unroll
+        for (int tt = 0; tt < DT; ++tt) {
+            const int d = tt * 32 + 16 * (g & 1) + 4 * (j & 3);
+            va[tt] = lk + (uint32_t)(KBYTES + row * T::kRow + (((d >> 3) ^ T::v_swz(row)) << 4) + ((d & 7) << 1));
+        }
+    }
+    typedef short s4_t __attribute__((ext_vector_type(4)));
+
+    for (int kt = wave; kt < ntiles; kt += KW) {
+        const bool more = kt + KW < ntiles;
+        const int kb0 = kt * KT;
+        // sk is per 128-key block; a tile lies inside one block
+        const float coef = (qscale * a.sk[(kb0 / kSageBlock) * a.Hkv + kvh]) * a.scale_log2;
+        attn_pipe::vm_wait<VLOADS>();   // K has landed; the V tile's loads may be in flight
+        asm volatile("" ::: "memory");
+        int32x4_t kf[NH][KS8];
+#pragma unroll
+        for (int ks = 0; ks < KS8; ++ks) {
+            attn_pipe::read_b128<0>(kf[0][ks], ka[ks]);
+            if constexpr (NH == 2) attn_pipe::read_b128<32 * HD>(kf[NH - 1][ks], ka[ks]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int ks = 0; ks < KS8; ++ks) asm volatile("" : "+v"(kf[h][ks]));
+        if (more) issue_k(kt + KW);
+        const float m_acc = (m_run == -INFINITY) ? 0.f : m_run;
+        const float bias = fmaf(kMagic, coef, m_acc);
+        int32x16_t acc[NH];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            acc[h] = magic;
+#pragma unroll
+            for (int ks = 0; ks < KS8; ++ks)
+                acc[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[h][ks], qf[ks], acc[h], 0, 0, 0);
+        }
+        // ---- V^T operand reads go out under the softmax
+        if (more) attn_pipe::vm_wait<KLOADS>();
+        else attn_pipe::vm_wait<0>();
+        asm volatile("" ::: "memory");
+        s4_t vf[KB][DT][2];
+#pragma unroll
+        for (int tt = 0; tt < DT; ++tt) {
+            attn_pipe::read_tr16<0>(vf[0][tt][0], va[tt]);
+            attn_pipe::read_tr16<8 * T::kRow>(vf[0][tt][1], va[tt]);
+            attn_pipe::read_tr16<16 * T::kRow>(vf[1][tt][0], va[tt]);
+            attn_pipe::read_tr16<24 * T::kRow>(vf[1][tt][1], va[tt]);
+            if constexpr (KB == 4) {
+                attn_pipe::read_tr16<32 * T::kRow>(vf[KB - 2][tt][0], va[tt]);
+                attn_pipe::read_tr16<40 * T::kRow>(vf[KB - 2][tt][1], va[tt]);
+                attn_pipe::read_tr16<48 * T::kRow>(vf[KB - 1][tt][0], va[tt]);
+                attn_pipe::read_tr16<56 * T::kRow>(vf[KB - 1][tt][1], va[tt]);
+            }
+        }
+        // s = score * coef - m_acc, in log2 units (element e of s[h]: key kb0 + 32 h + (e/4)*8 +
+        // hh*4 + e%4, row qi)
+        float s[NH][16];
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[h][e] = fmaf(__int_as_float(acc[h][e]), coef, -bias);
+        if (kb0 + KT > kv_end || (a.causal && kb0 + KT - 1 > q0 + diag)) {
+            const int lim = a.causal ? min(kv_end, qi + diag + 1) : kv_end;
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    s[h][e] = (kb0 + h * 32 + (e / 4) * 8 + hh * 4 + (e % 4) < lim) ? s[h][e] : -INFINITY;
+        }
+        float mloc = s[0][0];
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, s[h][e]);
+        {
+            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+            mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));   // tile max - m_acc
+        }
+        if (__any(m_run == -INFINITY || mloc > kSPLazy)) {
+            asm volatile("" ::: "memory");
+            // a row may see none of its wave's first tiles: its max stays -inf, its p are 0
+            const float m_new = fmaxf(m_run, mloc + m_acc);
+            const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+            const float shift = (m_new == -INFINITY) ? 0.f : m_new - m_acc;
+            l_run *= alpha;
+#pragma unroll
+            for (int tt = 0; tt < DT; ++tt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) oacc[tt][e] *= alpha;
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) s[h][e] -= shift;
+            m_run = m_new;
+        }
+        Pack8 pb[KB];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            float p[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) p[e] = __builtin_amdgcn_exp2f(s[h][e]);
+            pb[2 * h].u = pack8(&p[0]);
+            pb[2 * h + 1].u = pack8(&p[8]);
+        }
+        float psum = 0.f;
+#pragma unroll
+        for (int b = 0; b < KB; ++b) {
+            psum = add_bf16_pair(pb[b].u.x, psum);
+            psum = add_bf16_pair(pb[b].u.y, psum);
+            psum = add_bf16_pair(pb[b].u.z, psum);
+            psum = add_bf16_pair(pb[b].u.w, psum);
+        }
+        {
+            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(psum), __float_as_uint(psum), false, false);
+            l_run += __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+        }
+        // ---- O^T += V^T . P^T
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int tt = 0; tt < DT; ++tt) asm volatile("" : "+v"(vf[kb][tt][0]), "+v"(vf[kb][tt][1]));
+        if (more) issue_v(kt + KW);
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+            if (kb == 2 && kb0 + 32 >= kv_end) break;   // no row of the block sees keys 32..63
+#pragma unroll
+            for (int tt = 0; tt < DT; ++tt) {
+                union {
+                    s4_t h[2];
+                    bf16x8_t v;
+                } vv;
+                vv.h[0] = vf[kb][tt][0];
+                vv.h[1] = vf[kb][tt][1];
+                oacc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv.v, pb[kb].v, oacc[tt], 0, 0, 0);
+            }
+        }
+    }
+
+    // ---- merge through the waves' own slots (float4 chunk c of row r at c ^ (r & 15))
+    {
+        float4* part = reinterpret_cast<float4*>(kslot);
+#pragma unroll
+        for (int tt = 0; tt < DT; ++tt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                part[ql * CPR + ((tt * 8 + g * 2 + hh) ^ (ql & 15))] =
+                    make_float4(oacc[tt][g * 4], oacc[tt][g * 4 + 1], oacc[tt][g * 4 + 2], oacc[tt][g * 4 + 3]);
+        if (hh == 0) {
+            ml[0][wave][ql] = m_run;
+            ml[1][wave][ql] = l_run;
+        }
+    }
+    __syncthreads();
+    for (int idx = tid; idx < 32 * CPR; idx += KW * 64) {
+        const int r = idx / CPR, c = idx % CPR;
+        float m = ml[0][0][r];
+#pragma unroll
+        for (int w = 1; w < KW; ++w) m = fmaxf(m, ml[0][w][r]);
+        float l = 0.f;
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < KW; ++w) {
+            const float x = __builtin_amdgcn_exp2f(ml[0][w][r] - m);
+            const float4 v = reinterpret_cast<const float4*>(smem + w * SLOT)[r * CPR + (c ^ (r & 15))];
+            l += x * ml[1][w][r];
+            acc.x += x * v.x;
+            acc.y += x * v.y;
+            acc.z += x * v.z;
+            acc.w += x * v.w;
+        }
+        if (q0 + r < a.S) {
+            const float inv = (l > 0.f) ? 1.f / l : 0.f;
+            uint2 w;
+            w.x = pack_bf16x2(acc.x * inv, acc.y * inv);
+            w.y = pack_bf16x2(acc.z * inv, acc.w * inv);
+            *reinterpret_cast<uint2*>(a.o + ((size_t)(q0 + r) * a.Hq + head) * HD + c * 4) = w;
+        }
+    }
+}
+
 int prefill_cus();
 int validate_attention_ctx(const efm_attention_ctx* c, const char* who);
+
+// Whether a head_dim-128 launch splits its keys over waves or streams shared tiles (the
+// pipelined kernel). The shared stream's time is its longest chain, a row's keys, until the
+// chip is full; the split's is its work, blocks x keys, so the line is their ratio, and with
+// many blocks the stream's fewer bytes per row win. Measured on 256 CUs (us, split / shared,
+// whole operator; blocks = 32-row blocks of all heads): causal, no prefix: 64 rows, 24 blocks
+// 14.6 / 14.2; 200, 84 17.9 / 19.2; 1000, 384 26.4 / 35.3; 1344, 672 38.3 / 40.9; 2500, 1264
+// 67.1 / 68.5; 300, 280 21.5 / 20.9; 1000, 896 39.9 / 36.5; 4096, 2048 125 / 104; behind a
+// prefix: 37 + 1000, 24 23.5 / 35.7; 37 + 8000, 56 57.3 / 173.6; 700 + 500, 616 38.1 / 39.3;
+// 3000 + 3000, 1128 135.8 / 142.5; not causal: 1000 + 700, 384 38.2 / 50.5; 1300 + 500, 1148
+// 77.4 / 69.0; 4096 + 1000, 1536 181 / 151.
+static bool sage_split_wins(long blocks, long kv, bool causal, int cus) {
+    return kv >= 96 && 5 * blocks <= 3 * kv && blocks <= (causal ? 5L : 3L) * cus;
+}
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -873,9 +1208,18 @@ extern "C" int efm_attention_prefill_sage_int8(const efm_attention_ctx* ctx, con
     float* km = reinterpret_cast<float*>(p + w.q8 + w.k8 + w.sq + w.sk);
     double* kp = reinterpret_cast<double*>(p + w.q8 + w.k8 + w.sq + w.sk + w.km);
     const int hd = (int)ctx->head_dim;
-    const bool pipe = hd == kSPHD && kernel_knob(EFM_KNOB_PREFILL_REGISTER) == 0;
-    // the pipelined kernel quantises Q itself (one 128-row block per 4 waves)
-    rc = sage_quantize_impl(ctx, q, k, qo_len, kv_len, q8, sq, k8, sk, km, stream, !pipe, kp);
+    const bool fast = kernel_knob(EFM_KNOB_PREFILL_REGISTER) == 0;
+    const int shape = kernel_knob(EFM_KNOB_PREFILL_SHAPE), cus = prefill_cus();
+    const long blocks = (long)((qo_len + 31) / 32) * ctx->num_qo_heads;
+    // the split kernel's loads take 16-byte aligned rows and 32-bit offsets inside a tile,
+    // its grid 32-row blocks: anything else stays with the kernels below
+    const bool split_ok = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(v) |
+                            reinterpret_cast<uintptr_t>(workspace)) & 15u) == 0 &&
+                          ctx->kv_stride_n < (1u << 24) && blocks < (1L << 22);
+    const bool split = fast && split_ok && (hd == 64 || (shape == 0 && sage_split_wins(blocks, kv_len, causal != 0, cus)));
+    const bool pipe = fast && !split && hd == kSPHD;
+    // the split and pipelined kernels quantise Q themselves
+    rc = sage_quantize_impl(ctx, q, k, qo_len, kv_len, q8, sq, k8, sk, km, stream, !split && !pipe, kp);
     if (rc) return rc;
     SageArgs a;
     a.q = static_cast<const bf16_t*>(q);
@@ -895,11 +1239,29 @@ extern "C" int efm_attention_prefill_sage_int8(const efm_attention_ctx* ctx, con
     a.v_sh = ctx->kv_stride_h ? (int)ctx->kv_stride_h : hd;
     a.causal = causal != 0;
     a.scale_log2 = (float)(1.4426950408889634 / sqrt((double)hd));
+    if (split) {
+        const int nqt = (int)((qo_len + 31) / 32);
+        const dim3 grid = SplitGrid::dims(nqt, a.Hq, a.Hkv);
+        const SplitGrid sg = SplitGrid::of(a.Hq, a.Hkv);
+        // Waves per 32-row block: 8 (one workgroup per CU) while there is a CU for every block
+        // and the keys are worth it, else 4 (two per CU). us, 8 / 4 waves: 24 blocks x 3018
+        // keys 33.2 / 36.6, 196 x 4100 42.3 / 47.8, 156 x 8200 61.1 / 79.1; 24 x 1018 24.5 /
+        // 23.5, 384 x 8500 110.9 / 102.3; head_dim 64, 98 x 8100 37.8 / 49.0, 154 x 666 18.2 /
+        // 17.4, 308 x 8350 66.7 / 61.7.
+        const bool eight = blocks <= cus && kv_len >= 2048;
+        auto launch = [&](auto kernel, int waves) {
+            hipLaunchKernelGGL(kernel, grid, dim3(waves * kWave), 0, stream, a, sg, nqt);
+        };
+        if (hd == 128 && eight) launch(sage_attn_split_kernel<128, 8>, 8);
+        else if (hd == 128) launch(sage_attn_split_kernel<128, 4>, 4);
+        else if (eight) launch(sage_attn_split_kernel<64, 8>, 8);
+        else launch(sage_attn_split_kernel<64, 4>, 4);
+        return check_launch("sage_attention");
+    }
     if (pipe) {
-        // as the bf16 kernel: 8 waves over a 4-deep ring when those workgroups fill the
+        // 8 waves over a 4-deep ring when those workgroups fill the
         // chip, else 4 waves / two workgroups per CU (a 3-deep ring of 24 KB stages fits twice)
-        const int shape = kernel_knob(EFM_KNOB_PREFILL_SHAPE);
-        const bool small = shape != 0 ? shape <= 4 : (int)((qo_len + 255) / 256) * a.Hq < prefill_cus();
+        const bool small = shape != 0 ? shape <= 4 : (int)((qo_len + 255) / 256) * a.Hq < cus;
         if (small) {
             const int nqt = (int)((qo_len + 127) / 128);
             hipLaunchKernelGGL((sage_attn_pipe_kernel<4, 3>), dim3(nqt * a.Hq), dim3(256), 0, stream, a, nqt);

@@ -65,8 +65,8 @@ int efm_init(void);
  *                              register-staged kernel instead of the LDS-staged one
  *   EFM_KNOB_PREFILL_REGISTER  1: prefill and Sage attention run the register-staged
  *                              kernels instead of the split and pipelined ones
- *   EFM_KNOB_PREFILL_SHAPE     4 or 8: the pipelined prefill / Sage kernels run (for
- *                              prefill in place of the split kernel too) with
+ *   EFM_KNOB_PREFILL_SHAPE     4 or 8: the pipelined prefill / Sage kernels run (in
+ *                              place of the split kernels too) with
  *                              4-wave (128-row) or 8-wave (256-row) workgroups; 2: the
  *                              prefill kernel runs 2-wave (64-row) workgroups (the Sage
  *                              kernel treats 2 as 4)

@@ -1673,6 +1673,44 @@ def test_sage_attention_pipelined_matches_register_kernel(gpu, knob, shape, S, L
     assert_close_bf16(outs[0], outs[1], rtol=2e-2, atol=2e-2, what="sage pipelined vs register kernel")
 
 
+@pytest.mark.parametrize("hq,hkv,hd,S,L,causal", [
+    pytest.param(14, 2, 64, 1, 1, 1, id="hd64_one_row"),
+    pytest.param(14, 2, 64, 33, 64, 1, id="hd64_whole_tile"),
+    pytest.param(6, 3, 64, 129, 193, 1, id="hd64_three_kv_heads"),
+    pytest.param(14, 2, 64, 200, 2111, 1, id="hd64_eight_waves"),
+    pytest.param(14, 2, 64, 300, 333, 0, id="hd64_not_causal"),
+    pytest.param(12, 2, 128, 97, 97, 1, id="first_split_length"),
+    pytest.param(12, 2, 128, 5, 1025, 1, id="few_rows_one_key_past"),
+    pytest.param(6, 3, 128, 129, 255, 1, id="three_kv_heads"),
+    pytest.param(16, 16, 128, 40, 300, 0, id="sixteen_kv_heads"),
+    pytest.param(12, 2, 128, 130, 2049, 1, id="eight_waves"),
+    pytest.param(12, 2, 128, 700, 901, 0, id="not_causal"),
+])
+def test_sage_attention_split_matches_register_kernel(gpu, knob, hq, hkv, hd, S, L, causal):
+    """Launches that split their keys over waves (head_dim 64, or few query blocks), q, k and v
+    strided out of one row: against the register-staged kernel, which quantises the same. Both
+    round p to bf16 before the products; its row sums are over p before that rounding and its
+    reference point for p is the true maximum, so a p differs by 2^-8 of itself at most."""
+    g = torch.Generator(device=gpu).manual_seed(S + L)
+    rows = torch.empty(L, (hq + 2 * hkv) * hd, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+    rows[0, :hq * hd] *= 6   # one 128-row block with a larger scale than the others
+    q, k, v = (rows[:, a * hd:] for a in (0, hq, hq + hkv))
+    tot = rows.shape[1]
+    ctx = C.make_attention_ctx(hq, hkv, hd, rope=False, q_stride_n=tot, q_stride_h=hd, k_stride_n=tot, k_stride_h=hd,
+                               kv_stride_n=tot, kv_stride_h=hd)
+    ws = torch.zeros(C.load().efm_attention_prefill_sage_int8_workspace_bytes(ctx, S, L), dtype=torch.uint8, device=gpu)
+    outs = []
+    for register in (0, 1):
+        knob(C.EFM_KNOB_PREFILL_REGISTER, register)
+        o = torch.full((S + 1, hq * hd), -7.0, dtype=torch.bfloat16, device=gpu)
+        C.call("efm_attention_prefill_sage_int8", ctx, ptr(q), ptr(k), ptr(v), ptr(o), S, L, causal, ptr(ws),
+               ws.numel(), stream())
+        torch.cuda.synchronize()
+        assert (o[S] == -7.0).all() and torch.isfinite(o.float()).all()
+        outs.append(o[:S])
+    assert_close_bf16(outs[0], outs[1], rtol=2e-2, atol=2e-2, what="sage split vs register kernel")
+
+
 @pytest.mark.parametrize("hq,hkv", [(12, 2), (28, 4), (16, 2), (8, 8)])
 @pytest.mark.parametrize("kv_len,max_kv", [(1, 1), (100, 128), (767, 768), (1025, 2000), (16385, 16513)])
 def test_decode_attention_lds_kernel_matches_register_kernel(gpu, knob, hq, hkv, kv_len, max_kv):
