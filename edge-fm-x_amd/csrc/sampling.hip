@@ -14,14 +14,19 @@
 // The row is split into blocks of 1024 logits, one 256-thread workgroup each, and the
 // passes are separate launches (the launch boundary is the grid-wide barrier):
 //   1. block maxima (workgroup 0 also clears the workspace accumulators)
-//   2. m from the block maxima; total mass W and the histogram of the top exponent
-//      byte of e (device-scope integer atomics: exact and order independent)
-//   3-5. each workgroup replays the digit choice of the previous passes from the
-//      histograms (positive fp32 values order like their bit patterns), then
-//      histograms the next byte of the e_i that share the chosen prefix
-//   6. tau is fixed; every block writes its nucleus mass, and the last block to finish
+//   2. m from the block maxima; the mass histogram of the top digit of the key of e
+//      (device-scope integer atomics: exact and order independent)
+//   3-4. each workgroup replays the digit choice of the previous passes from the
+//      histograms, then histograms the next digit of the keys that share the chosen prefix
+//   5. tau is fixed; every block writes its nucleus mass, and the last block to finish
 //      scans the block masses, finds the block holding r and scans its elements.
-// With top_p >= 1 passes 3-5 are skipped (tau = 0).
+// With top_p >= 1 passes 2-4 are skipped (tau = 0).
+// The key is e's bit pattern (positive fp32 values order like theirs) less that of 2^-45: a
+// smaller e has no mass and 1 is the largest, so it has 29 bits, three digits of 10. What
+// bounds a call is its launches, 4 to 5 us each, and not the 0.6 MB of logits: with bytes as
+// digits (6 launches) and a pass for the total mass (the first histogram's sum) 151936 logits
+// took 31.0 us with top_p 0.9 and 14.1 without, now 25.3 and 10.1; 8192 25.0 / 11.1, now 20.7
+// / 8.4 (graph replay).
 #include "common.hpp"
 
 namespace efm {
@@ -31,13 +36,15 @@ constexpr int kSamplePer = 4;                                  // logits per thr
 constexpr int kSampleBlock = kSampleThreads * kSamplePer;      // logits per workgroup
 constexpr int kSampleMaxVocab = 1 << 20;
 constexpr int kSampleMaxBlocks = kSampleMaxVocab / kSampleBlock;
+constexpr int kSampleDigits = 3, kSampleDigitBits = 10, kSampleBins = 1 << kSampleDigitBits;
+constexpr uint32_t kSampleKey0 = (127u - 45u) << 23;           // bits of 2^-45
+static_assert(kSampleBins == 4 * kSampleThreads, "a thread scans 4 bins");
 
 // Device workspace of one sampler call (efm_sampler_top_p_workspace_bytes).
 struct SampleWs {
     float bmax[kSampleMaxBlocks];
     unsigned long long bmass[kSampleMaxBlocks];
-    unsigned long long hist[4][256];
-    unsigned long long W;
+    unsigned long long hist[kSampleDigits][kSampleBins];   // mass by digit
     uint32_t counter;
 };
 
@@ -153,53 +160,49 @@ __device__ __forceinline__ float global_max(const SampleArgs& a, float* red) {
     return block_max_f(m, red);
 }
 
-// Replays the radix choices of passes [0, npass): returns the chosen key prefix and
-// the mass still needed inside it. Every workgroup computes the same values.
-__device__ uint32_t select_prefix(const SampleArgs& a, int npass, unsigned long long* s_sel) {
-    const int lane = threadIdx.x % kWave;
-    if (threadIdx.x < kWave) {
-        const uint64_t W = a.ws->W;
-        uint64_t need = (uint64_t)ceil((double)a.top_p * (double)W);
-        if (need < 1) need = 1;
-        if (need > W) need = W;
-        uint64_t rem = need;
-        uint32_t prefix = 0u;
-        for (int p = 0; p < npass; ++p) {
-            const int shift = 24 - 8 * p;
-            // lane j owns digits 255-4j .. 252-4j (descending)
-            uint64_t h[4], own = 0;
+// Replays the digit choices of passes [0, npass): returns the chosen key prefix. Every
+// workgroup computes the same values. Thread t owns the bins 1023-4t .. 1020-4t (descending).
+__device__ uint32_t select_prefix(const SampleArgs& a, int npass, unsigned long long* red, unsigned long long* s_sel) {
+    uint64_t h[kSampleDigits][4];
+#pragma unroll
+    for (int p = 0; p < kSampleDigits; ++p)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            h[p][k] = p < npass ? a.ws->hist[p][kSampleBins - 1 - 4 * (int)threadIdx.x - k] : 0ull;
+    if (threadIdx.x < 2) s_sel[threadIdx.x] = 0ull;
+    uint64_t rem = 0;
+    uint32_t prefix = 0u;
+#pragma unroll
+    for (int p = 0; p < kSampleDigits; ++p) {
+        if (p >= npass) break;
+        const uint64_t own = h[p][0] + h[p][1] + h[p][2] + h[p][3];
+        uint64_t W;
+        const uint64_t excl = block_scan_u64(own, red, &W);
+        if (p == 0) {   // the first histogram holds all of the mass
+            rem = (uint64_t)ceil((double)a.top_p * (double)W);
+            if (rem < 1) rem = 1;
+            if (rem > W) rem = W;
+        }
+        // exactly one thread's bins hold the rem-th unit of mass
+        if (excl < rem && rem <= excl + own) {
+            uint64_t acc = excl;
+            bool found = false;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                h[k] = a.ws->hist[p][255 - 4 * lane - k];
-                own += h[k];
-            }
-            const uint64_t incl = wave_scan_u64(own, lane);
-            const uint64_t excl = incl - own;
-            // exactly one lane's digit range holds the rem-th unit of mass
-            const bool owns = excl < rem && rem <= incl;
-            uint32_t digit = 0u;
-            uint64_t left = 0ull;
-            if (owns) {
-                uint64_t acc = excl;
-                bool found = false;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (!found && rem <= acc + h[k]) {
-                        digit = (uint32_t)(255 - 4 * lane - k);
-                        left = rem - acc;
-                        found = true;
-                    }
-                    acc += h[k];
+                if (!found && rem <= acc + h[p][k]) {
+                    s_sel[0] = (unsigned long long)(kSampleBins - 1 - 4 * (int)threadIdx.x - k);
+                    s_sel[1] = rem - acc;
+                    found = true;
                 }
+                acc += h[p][k];
             }
-            const int src = __ffsll((unsigned long long)__ballot(owns)) - 1;
-            prefix |= (uint32_t)__shfl((int)digit, src, kWave) << shift;
-            rem = (uint64_t)__shfl((unsigned long long)left, src, kWave);
         }
-        if (lane == 0) s_sel[0] = prefix;
+        __syncthreads();
+        prefix |= (uint32_t)s_sel[0] << (kSampleDigitBits * (kSampleDigits - 1 - p));
+        rem = s_sel[1];
+        __syncthreads();
     }
-    __syncthreads();
-    return (uint32_t)s_sel[0];
+    return prefix;
 }
 
 // pass 1: block maxima; workgroup 0 clears the accumulators the later passes add into
@@ -215,59 +218,51 @@ __global__ void __launch_bounds__(kSampleThreads) sample_max_kernel(SampleArgs a
     if (threadIdx.x == 0) a.ws->bmax[blockIdx.x] = m;
     if (blockIdx.x == 0) {
         unsigned long long* h = &a.ws->hist[0][0];
-        for (int i = threadIdx.x; i < 4 * 256; i += kSampleThreads) h[i] = 0ull;
-        if (threadIdx.x == 0) {
-            a.ws->W = 0ull;
-            a.ws->counter = 0u;
-        }
+        for (int i = threadIdx.x; i < kSampleDigits * kSampleBins; i += kSampleThreads) h[i] = 0ull;
+        if (threadIdx.x == 0) a.ws->counter = 0u;
     }
 }
 
-// passes 2-5: pass 2 adds the total mass W; every pass histograms the next byte
-// (shift 24 - 8 * npass) of the e_i under the prefix chosen so far.
-__global__ void __launch_bounds__(kSampleThreads) sample_hist_kernel(SampleArgs a, int npass, int want_hist) {
+// passes 2-4: histograms digit npass of the keys under the prefix chosen so far.
+__global__ void __launch_bounds__(kSampleThreads) sample_hist_kernel(SampleArgs a, int npass) {
     __shared__ float red[kSampleThreads / kWave];
     __shared__ unsigned long long redu[kSampleThreads / kWave];
-    __shared__ unsigned long long s_hist[256];
-    __shared__ unsigned long long s_sel[1];
+    __shared__ unsigned long long s_hist[kSampleBins];
+    __shared__ unsigned long long s_sel[2];
     float l[kSamplePer];
     bool ok[kSamplePer];
     load_block(a, l, ok);
-    s_hist[threadIdx.x] = 0ull;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s_hist[threadIdx.x + k * kSampleThreads] = 0ull;
     const float m = global_max(a, red);
     const float T = a.temperature;
-    uint32_t prefix = 0u;
-    if (npass > 0) prefix = select_prefix(a, npass, s_sel);
-    const int shift = 24 - 8 * npass;
-    const uint32_t mask = (npass == 0) ? 0u : (0xffffffffu << (shift + 8));
-    uint64_t tot = 0;
+    const uint32_t prefix = npass > 0 ? select_prefix(a, npass, redu, s_sel) : 0u;
+    const int shift = kSampleDigitBits * (kSampleDigits - 1 - npass);
+    const uint32_t mask = 0xffffffffu << (shift + kSampleDigitBits);
+    __syncthreads();   // s_hist is clear
 #pragma unroll
     for (int k = 0; k < kSamplePer; ++k) {
         if (!ok[k]) continue;
         const float e = sample_e(l[k], m, T);
         const uint64_t w = sample_w(e);
-        tot += w;
-        const uint32_t key = __float_as_uint(e);
-        if (want_hist && w != 0 && (key & mask) == prefix)
-            atomicAdd(&s_hist[(key >> shift) & 255u], (unsigned long long)w);
+        const uint32_t key = __float_as_uint(e) - kSampleKey0;
+        if (w != 0 && (npass == 0 || (key & mask) == prefix))
+            atomicAdd(&s_hist[(key >> shift) & (kSampleBins - 1)], (unsigned long long)w);
     }
-    if (npass == 0) {
-        tot = block_sum_u64(tot, redu);
-        if (threadIdx.x == 0) __hip_atomic_fetch_add(&a.ws->W, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (want_hist) {
-        __syncthreads();
-        const unsigned long long hv = s_hist[threadIdx.x];
-        if (hv != 0ull)
-            __hip_atomic_fetch_add(&a.ws->hist[npass][threadIdx.x], hv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int d = threadIdx.x + k * kSampleThreads;
+        const unsigned long long hv = s_hist[d];
+        if (hv != 0ull) __hip_atomic_fetch_add(&a.ws->hist[npass][d], hv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
-// pass 6: nucleus mass per block; the last block to finish locates r.
+// pass 5: nucleus mass per block; the last block to finish locates r.
 __global__ void __launch_bounds__(kSampleThreads) sample_locate_kernel(SampleArgs a) {
     __shared__ float red[kSampleThreads / kWave];
     __shared__ unsigned long long redu[kSampleThreads / kWave];
-    __shared__ unsigned long long s_sel[1];
+    __shared__ unsigned long long s_sel[2];
     __shared__ uint32_t s_last;
     __shared__ int s_block;
     __shared__ unsigned long long s_base;
@@ -276,7 +271,7 @@ __global__ void __launch_bounds__(kSampleThreads) sample_locate_kernel(SampleArg
     load_block(a, l, ok);
     const float m = global_max(a, red);
     const float T = a.temperature;
-    const uint32_t tau_key = (a.top_p < 1.0f) ? select_prefix(a, 4, s_sel) : 0u;
+    const uint32_t tau_key = (a.top_p < 1.0f) ? kSampleKey0 + select_prefix(a, kSampleDigits, redu, s_sel) : 0u;
     uint64_t own = 0;
 #pragma unroll
     for (int k = 0; k < kSamplePer; ++k) {
@@ -294,6 +289,8 @@ __global__ void __launch_bounds__(kSampleThreads) sample_locate_kernel(SampleArg
         asm volatile("s_waitcnt vmcnt(0)" : : "v"(old) : "memory");
         const uint32_t prev = __hip_atomic_fetch_add(&a.ws->counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s_last = (prev == (uint32_t)a.nblocks - 1) ? 1u : 0u;
+        s_block = 0;   // no block holds r where the logits have no mass (NaN)
+        s_base = 0ull;
     }
     __syncthreads();
     if (!s_last) return;
@@ -386,9 +383,8 @@ extern "C" int efm_sampler_top_p(int64_t vocab, const float* logits, float tempe
     SampleArgs a{logits, (int)vocab, temperature, top_p, seed, offset, d_offset, token_out,
                  static_cast<SampleWs*>(workspace), nb};
     hipLaunchKernelGGL(sample_max_kernel, dim3(nb), dim3(kSampleThreads), 0, stream, a);
-    const int passes = (top_p < 1.0f) ? 4 : 1;
-    for (int p = 0; p < passes; ++p)
-        hipLaunchKernelGGL(sample_hist_kernel, dim3(nb), dim3(kSampleThreads), 0, stream, a, p, top_p < 1.0f ? 1 : 0);
+    for (int p = 0; top_p < 1.0f && p < kSampleDigits; ++p)
+        hipLaunchKernelGGL(sample_hist_kernel, dim3(nb), dim3(kSampleThreads), 0, stream, a, p);
     hipLaunchKernelGGL(sample_locate_kernel, dim3(nb), dim3(kSampleThreads), 0, stream, a);
     return check_launch("sampler_top_p");
 }

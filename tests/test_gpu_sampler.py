@@ -117,6 +117,22 @@ def test_sampler_top_p_device_offset_and_seed_words(gpu):
     assert a == want or O.sample_margin(logits, 1.0, 0.95, (3 << 40) | 5, 117) < MARGIN
 
 
+@pytest.mark.parametrize("vocab", [1023, 1025, 152064])
+@pytest.mark.parametrize("p", [1e-7, 0.5, 0.999999, 1.0 - 2.0 ** -24])
+def test_sampler_top_p_threshold_digits(gpu, vocab, p):
+    """The threshold's key is chosen digit by digit: masses from the largest down to the
+    smallest that counts (e = 2^-45 has none, 2^-44.5 has one unit), runs of neighbouring
+    keys that differ in the last digit only, -inf logits, and nuclei of one and of nearly all."""
+    rng = np.random.default_rng(vocab)
+    logits = (-rng.uniform(0, 45 * np.log(2.0), vocab)).astype(np.float32)
+    logits[rng.integers(0, vocab, vocab // 3)] = -np.inf
+    near = rng.integers(0, vocab, vocab // 4)
+    logits[near] = np.float32(-3.0) + np.arange(near.size, dtype=np.float32) * np.float32(2.0 ** -22)
+    logits[vocab // 2] = 0.0
+    for off in range(4):
+        _check(gpu, logits, 1.0, p, seed=77, offset=off)
+
+
 def test_sampler_top_p_deterministic(gpu):
     rng = np.random.default_rng(3)
     logits = rng.standard_normal(151936).astype(np.float32) * 3
