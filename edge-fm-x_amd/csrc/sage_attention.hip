@@ -137,7 +137,9 @@ __global__ __launch_bounds__(kSageThreads) void sage_kpart_kernel(const bf16_t* 
 // ---- block quantisation: grid (blocks, H), 256 threads --------------------------
 // dst [T][H][hd] int8 (contiguous), scales [blocks][H]. KM = 0: Q (no shift); 1: K with
 // its mean from kmean (sage_kmean_kernel); 2: K with its mean added up here from the
-// kKSlices row-slice sums in kpart (sage_kpart_kernel; block 0 stores it in kmean_out).
+// kKSlices row-slice sums in kpart (sage_kpart_kernel; block 0 stores it in kmean_out); 3: K
+// with its mean summed here over every row (float64: exact, the same bits), which saves the
+// slices' launch while the rows are few (sage_few_rows).
 // Every load is issued up front and branch-free (rows past the block's end are buffer
 // loads past the resource: zeros, no memory access), so one round trip covers them all.
 template <int KM>
@@ -145,7 +147,8 @@ __global__ __launch_bounds__(kSageThreads) void sage_quant_kernel(const bf16_t* 
                                                                   int hd, const float* kmean, const double* kpart,
                                                                   float* kmean_out, int8_t* dst, float* scales) {
     __shared__ float red[kSageThreads / kWave];
-    __shared__ float kms[KM == 2 ? 128 : 1];
+    __shared__ float kms[KM >= 2 ? 128 : 1];
+    __shared__ double sums[KM == 3 ? kSageThreads : 1][8];
     const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     const int t0 = b * kSageBlock;
     const int rows = min(kSageBlock, T - t0);
@@ -178,11 +181,41 @@ __global__ __launch_bounds__(kSageThreads) void sage_quant_kernel(const bf16_t* 
 #pragma unroll
         for (int sl = 0; sl < kKSlices; ++sl) kv[sl] = kpart[((size_t)sl * H + h) * hd + tid % hd];
     }
-    float km[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-    if constexpr (KM == 2) {
-        double sum = 0.0;
+    double sum = 0.0;   // KM >= 2: of channel tid % hd over the T rows
+    if constexpr (KM == 3) {
+        constexpr int kDeep = 16;   // rows in flight per thread
+        const int r0 = tid / cpr, rstep = kSageThreads / cpr;
+        const bf16_t* base = src + (size_t)h * sh + d0;
+        double s[8];
 #pragma unroll
-        for (int sl = 0; sl < kKSlices; ++sl) sum += kv[sl];
+        for (int e = 0; e < 8; ++e) s[e] = 0.0;
+        for (int j = r0; j < T; j += kDeep * rstep) {
+            uint4 u[kDeep];
+#pragma unroll
+            for (int r = 0; r < kDeep; ++r) {
+                const int row = j + r * rstep;
+                u[r] = row < T ? *reinterpret_cast<const uint4*>(base + (size_t)row * sn) : make_uint4(0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < kDeep; ++r) {
+                float f[8];
+                unpack8(u[r], f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s[e] += (double)f[e];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sums[tid][e] = s[e];
+        __syncthreads();
+        const int ch = tid % hd;
+        for (int r = 0; r < rstep; ++r) sum += sums[r * cpr + ch / 8][ch % 8];
+    }
+    float km[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+    if constexpr (KM >= 2) {
+        if constexpr (KM == 2) {
+#pragma unroll
+            for (int sl = 0; sl < kKSlices; ++sl) sum += kv[sl];
+        }
         const float mean = (float)(sum / (double)T);
         if (tid < hd) {
             kms[tid] = mean;
@@ -1116,6 +1149,12 @@ static SageWs sage_ws(const efm_attention_ctx* c, uint32_t S, uint32_t L) {
     return w;
 }
 
+// Rows few enough (128 KB) that every 128-row block sums them all itself, 16 rows of a thread
+// in flight: a launch less, against reading every row once per block. us, whole operator,
+// slices / here: head_dim 64 (14/2 heads) 64 rows 12.3 / 11.1, 300 14.5 / 13.3, 1000 18.9 /
+// 18.9; head_dim 128 64 rows 14.2 / 13.0, 200 17.4 / 16.2, 400 19.2 / 19.0, 512 20.1 / 19.9.
+static bool sage_few_rows(uint32_t L, int hd) { return (size_t)L * hd <= 512 * 128; }
+
 // kpart == nullptr (efm_sage_quantize): the K mean from one workgroup per (KV head, 8
 // channels); else (the attention entry point, whose workspace holds kpart) from row-slice
 // sums added up by the quantisation kernel, which also stores the mean in kmean.
@@ -1127,10 +1166,11 @@ static int sage_quantize_impl(const efm_attention_ctx* c, const void* q, const v
     const int q_sh = c->q_stride_h ? (int)c->q_stride_h : hd;
     const int k_sn = c->k_stride_n ? (int)c->k_stride_n : (int)(c->num_kv_heads * hd);
     const int k_sh = c->k_stride_h ? (int)c->k_stride_h : hd;
-    if (kpart != nullptr) {
+    const bool few = kpart != nullptr && sage_few_rows(L, hd);
+    if (kpart != nullptr && !few) {
         hipLaunchKernelGGL(sage_kpart_kernel, dim3(c->num_kv_heads, kKSlices), dim3(kSageThreads), 0, stream,
                            static_cast<const bf16_t*>(k), (int)L, k_sn, k_sh, hd, kpart);
-    } else {
+    } else if (kpart == nullptr) {
         hipLaunchKernelGGL(sage_kmean_kernel, dim3(c->num_kv_heads, hd / 8), dim3(kKmeanThreads), 0, stream,
                            static_cast<const bf16_t*>(k), (int)L, k_sn, k_sh, hd, kmean);
     }
@@ -1145,7 +1185,11 @@ static int sage_quantize_impl(const efm_attention_ctx* c, const void* q, const v
         if (rc) return rc;
     }
     const dim3 kgrid((L + kSageBlock - 1) / kSageBlock, c->num_kv_heads);
-    if (kpart != nullptr)
+    if (few)
+        hipLaunchKernelGGL(sage_quant_kernel<3>, kgrid, dim3(kSageThreads), 0, stream, static_cast<const bf16_t*>(k),
+                           (int)L, (int)c->num_kv_heads, k_sn, k_sh, hd, (const float*)nullptr, (const double*)nullptr,
+                           kmean, k8, sk);
+    else if (kpart != nullptr)
         hipLaunchKernelGGL(sage_quant_kernel<2>, kgrid, dim3(kSageThreads), 0, stream, static_cast<const bf16_t*>(k),
                            (int)L, (int)c->num_kv_heads, k_sn, k_sh, hd, (const float*)nullptr, (const double*)kpart,
                            kmean, k8, sk);
