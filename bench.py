@@ -310,7 +310,7 @@ def kernel_only(torch, C, S, shape, seed):
 def gemm_only(torch, C, reps=3):
     """Prefill GEMM counter workload: the C5 (7B, 16384-token prefill) gate/up projection
     with its SwiGLU epilogue, [16384, 3584] x [2 x 18944, 3584]^T, reps launches through
-    efm_fused_gate_up_swiglu (the library's own kernel choice: the 256 x 256 wide kernel),
+    efm_fused_gate_up_swiglu (the library's own kernel choice: the slab kernel's 256 x 256 tile),
     after one untimed launch; average time from HIP events on the launch stream."""
     dev = torch.device("cuda:0")
     torch.cuda.set_device(dev)
