@@ -789,7 +789,11 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void sage_attn_pipe_kernel(S
 //  * Q is quantised here: the scale is that of the 128-row block around the 32 rows, so each
 //    wave takes the max of one 32-row quarter (an L2 read; the other quarters' workgroups
 //    read the same rows).
-//  * Score arithmetic as in the pipelined kernel above.
+//  * Scores enter the softmax as exact integers (converted, then one FMA with the scale and the
+//    running max). The pipelined kernel's fold of 1.5 * 2^23 * coef into the FMA's addend rounds
+//    that addend once per tile, an offset common to the tile of up to 0.75 coef in log2 units:
+//    1e-4 of a tile's weight where q and k have unit variance, 3 % at 16 times that. The
+//    conversion takes the place of the move that sets the accumulator's start value.
 //  Measured (us, whole operator, before / after; head_dim 64 ran the register-staged kernel):
 //  head_dim 64, 14/2 heads: S 100 20.5 / 13.3, 333 behind 500 60.5 / 17.4, 700 51.9 / 17.6, 4096
 //  294 / 65.5; head_dim 128: 12/2 heads S 1000 35.3 / 26.4, 37 behind 8000 173 / 55.6.
@@ -920,9 +924,6 @@ __global__ __launch_bounds__(KW * 64, 2) void sage_attn_split_kernel(SageArgs a,
 #pragma unroll
         for (int e = 0; e < 16; ++e) oacc[tt][e] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;   // -inf until the wave meets a key that the row sees
-    int32x16_t magic;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) magic[e] = __float_as_int(kMagic);
 
     const uint32_t lk = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)kslot);
     uint32_t ka[KS8], va[DT];
@@ -959,11 +960,11 @@ __global__ __launch_bounds__(KW * 64, 2) void sage_attn_split_kernel(SageArgs a,
             for (int ks = 0; ks < KS8; ++ks) asm volatile("" : "+v"(kf[h][ks]));
         if (more) issue_k(kt + KW);
         const float m_acc = (m_run == -INFINITY) ? 0.f : m_run;
-        const float bias = fmaf(kMagic, coef, m_acc);
         int32x16_t acc[NH];
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
-            acc[h] = magic;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[h][e] = 0;
 #pragma unroll
             for (int ks = 0; ks < KS8; ++ks)
                 acc[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[h][ks], qf[ks], acc[h], 0, 0, 0);
@@ -992,7 +993,7 @@ __global__ __launch_bounds__(KW * 64, 2) void sage_attn_split_kernel(SageArgs a,
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) s[h][e] = fmaf(__int_as_float(acc[h][e]), coef, -bias);
+            for (int e = 0; e < 16; ++e) s[h][e] = fmaf((float)acc[h][e], coef, -m_acc);
         if (kb0 + KT > kv_end || (a.causal && kb0 + KT - 1 > q0 + diag)) {
             const int lim = a.causal ? min(kv_end, qi + diag + 1) : kv_end;
 #pragma unroll

@@ -1711,6 +1711,44 @@ def test_sage_attention_split_matches_register_kernel(gpu, knob, hq, hkv, hd, S,
     assert_close_bf16(outs[0], outs[1], rtol=2e-2, atol=2e-2, what="sage split vs register kernel")
 
 
+@pytest.mark.parametrize("amp", [1.0, 8.0, 16.0, 64.0])
+def test_sage_head_dim_64_scores_are_exact(gpu, amp):
+    """The int8 scores of head_dim 64 enter the softmax as exact integers times the scale, at
+    any amplitude of q and k: against float64 over the quantised operands. Queries are one
+    quantum in one channel, so that the scores of a row stay within a few octaves, and V is
+    +-1 per 64-key tile, so that an offset common to a tile shows. Bound: a p is rounded to
+    bf16 (2^-9 of it, in the weights and in their sum at most), the output too."""
+    g = torch.Generator(device=gpu).manual_seed(int(amp))
+    hq, hkv, hd, S, L = 14, 2, 64, 300, 1500
+    q = torch.zeros(S, hq, hd, device=gpu)
+    ch = torch.randint(0, hd, (S, hq, 1), device=gpu, generator=g)
+    q.scatter_(2, ch, amp * 4.0 / 127)
+    q[torch.arange(0, S, 128)] = amp * 4.0   # one row of every 128-row block sets its scale
+    q = q.bfloat16()
+    blk = torch.arange(L, device=gpu) // 128
+    k = (torch.empty(L, hkv, hd, device=gpu).normal_(generator=g) * (amp * (1 + 0.13 * blk))[:, None, None]).bfloat16()
+    v = (torch.randint(0, 2, ((L + 63) // 64, hkv, hd), device=gpu, generator=g) * 2 - 1)[torch.arange(L, device=gpu) // 64].bfloat16()
+    ctx = C.make_attention_ctx(hq, hkv, hd, rope=False)
+    q8, k8 = torch.empty(q.shape, dtype=torch.int8, device=gpu), torch.empty(k.shape, dtype=torch.int8, device=gpu)
+    sq, sk = torch.empty((S + 127) // 128, hq, device=gpu), torch.empty((L + 127) // 128, hkv, device=gpu)
+    km = torch.empty(hkv, hd, device=gpu)
+    C.call("efm_sage_quantize", ctx, ptr(q), ptr(k), S, L, ptr(q8), ptr(sq), ptr(k8), ptr(sk), ptr(km), stream())
+    ws = torch.zeros(C.load().efm_attention_prefill_sage_int8_workspace_bytes(ctx, S, L), dtype=torch.uint8, device=gpu)
+    o = torch.empty(S, hq, hd, dtype=torch.bfloat16, device=gpu)
+    C.call("efm_attention_prefill_sage_int8", ctx, ptr(q), ptr(k), ptr(v), ptr(o), S, L, 0, ptr(ws), ws.numel(), stream())
+    torch.cuda.synchronize()
+    rows = torch.arange(S, device=gpu)
+    qd = q8.double() * sq.double()[rows // 128][..., None]
+    kd = (k8.double() * sk.double()[blk][..., None]).repeat_interleave(hq // hkv, 1)
+    worst = 0.0
+    for h in range(hq):
+        w = torch.softmax(qd[:, h] @ kd[:, h].T.contiguous() / 8.0, -1)
+        ref = w @ v[:, h // (hq // hkv)].double()
+        err = (o[:, h].double() - ref).abs() - (2.0 ** -8 + 2.0 ** -9 * ref.abs() + 1e-4)
+        worst = max(worst, float(err.max()))
+    assert worst <= 0, worst
+
+
 @pytest.mark.parametrize("hq,hkv", [(12, 2), (28, 4), (16, 2), (8, 8)])
 @pytest.mark.parametrize("kv_len,max_kv", [(1, 1), (100, 128), (767, 768), (1025, 2000), (16385, 16513)])
 def test_decode_attention_lds_kernel_matches_register_kernel(gpu, knob, hq, hkv, kv_len, max_kv):
