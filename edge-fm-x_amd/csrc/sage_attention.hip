@@ -794,6 +794,8 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void sage_attn_pipe_kernel(S
 //    that addend once per tile, an offset common to the tile of up to 0.75 coef in log2 units:
 //    1e-4 of a tile's weight where q and k have unit variance, 3 % at 16 times that. The
 //    conversion takes the place of the move that sets the accumulator's start value.
+//  * At head_dim 64 every new max raises the running max, at 128 (calls that with more blocks
+//    run the pipelined kernel) one past 2^8: attn_split.hpp has the reason and the cost.
 //  Measured (us, whole operator, before / after; head_dim 64 ran the register-staged kernel):
 //  head_dim 64, 14/2 heads: S 100 20.5 / 13.3, 333 behind 500 60.5 / 17.4, 700 51.9 / 17.6, 4096
 //  294 / 65.5; head_dim 128: 12/2 heads S 1000 35.3 / 26.4, 37 behind 8000 173 / 55.6.
@@ -810,6 +812,8 @@ __global__ __launch_bounds__(KW * 64, 2) void sage_attn_split_kernel(SageArgs a,
     __shared__ __align__(1024) unsigned char smem[KW * SLOT];
     __shared__ float ml[2][KW][32];
     __shared__ float s_qmax[KW];
+
+    constexpr float lazy = HD == 64 ? 0.f : kSPLazy;   // as in attn_split.hpp
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -1011,7 +1015,7 @@ __global__ __launch_bounds__(KW * 64, 2) void sage_attn_split_kernel(SageArgs a,
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
             mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));   // tile max - m_acc
         }
-        if (__any(m_run == -INFINITY || mloc > kSPLazy)) {
+        if (__any(m_run == -INFINITY || mloc > lazy)) {
             asm volatile("" ::: "memory");
             // a row may see none of its wave's first tiles: its max stays -inf, its p are 0
             const float m_new = fmaxf(m_run, mloc + m_acc);
