@@ -624,10 +624,12 @@ static bool prefill_split_wins(const PrefillArgs& a, int cus) {
 
 // Waves per 32-row block: 8 (one workgroup per CU) while there is a CU for every block and
 // the keys are worth it, else 4 (two per CU), and 2 for many blocks where the chain is short
-// (head_dim 128, rotated keys). Measured (us, 8 / 4 / 2 waves): 24 blocks x 2018 keys 15.8 /
-// 19.2 / 33.5; 224 x 8128 50.8 / 65.8 / 124; 192 x 256 9.3 / 8.9 / 11.8; 384 x 512 16.1 /
-// 14.0 / 19.9; 1316 x 750 51.5 / 36.0 / 33.6; head_dim 64, 308 x 350 9.5 / 7.4 / 9.8;
-// RoPE inside, 384 x 524 29.3 / 25.2 / 36.4, 2632 x 5000 730 / 626 / 660.
+// (head_dim 128, no RoPE inside: where Q is rotated, 1900 rows of 28 heads behind 100 take
+// 58.8 us on 2 waves, which share that among fewer, 57.5 on 4). Measured (us, 8 / 4 / 2
+// waves): 24 blocks x 2018 keys 15.8 / 19.2 / 33.5; 224 x 8128 50.8 / 65.8 / 124; 192 x 256
+// 9.3 / 8.9 / 11.8; 384 x 512 16.1 / 14.0 / 19.9; 1316 x 750 51.5 / 36.0 / 33.6; head_dim 64,
+// 308 x 350 9.5 / 7.4 / 9.8; RoPE inside, 384 x 524 29.3 / 25.2 / 36.4, 2632 x 5000 730 / 626 /
+// 660.
 static void prefill_split_launch(const PrefillArgs& a, int hd, int cus, hipStream_t stream) {
     const int nqt = (a.S + 31) / 32;
     const long blocks = (long)nqt * a.Hq;
@@ -642,7 +644,7 @@ static void prefill_split_launch(const PrefillArgs& a, int hd, int cus, hipStrea
         else launch(prefill_attn_split_kernel<128, 4, true>, 4);
     } else if (hd == 128) {
         if (eight) launch(prefill_attn_split_kernel<128, 8, false>, 8);
-        else if (blocks <= 5L * cus) launch(prefill_attn_split_kernel<128, 4, false>, 4);
+        else if (blocks <= 5L * cus || a.rope_q) launch(prefill_attn_split_kernel<128, 4, false>, 4);
         else launch(prefill_attn_split_kernel<128, 2, false>, 2);
     } else if (a.rope_k) {
         if (eight) launch(prefill_attn_split_kernel<64, 8, true>, 8);

@@ -37,6 +37,7 @@
 #include "common.hpp"
 
 #include <type_traits>
+#include <utility>
 
 namespace efm {
 
@@ -116,10 +117,14 @@ __global__ __launch_bounds__(KW * 64, 2) void prefill_attn_split_kernel(PrefillA
     const float sc = SCALE_Q ? 1.f : a.sm_scale_log2;             // scores to log2 units
     constexpr float lazy = SCALE_Q ? kP2Lazy : 0.f;
     constexpr int CPR = HD / 4;                      // float4 chunks per output row
-    static_assert(KW >= 2 && NL == 8 && 32 * HD * 4 <= SLOT, "tile geometry");
+    static_assert(KW >= (ROTK ? 4 : 2) && NL == 8 && 32 * HD * 4 <= SLOT, "tile geometry");
     __shared__ __align__(1024) unsigned char smem[KW * SLOT];
     __shared__ float ml[2][KW][32];
-    __shared__ __align__(16) float sfreq[ROTK ? HD / 2 : 4];
+    // frequencies and rotated Q fragments; KW 2 takes no RoPE, so that four workgroups fit a CU
+    constexpr bool ROPE = KW >= 4;
+    const bool rope_q = ROPE && (ROTK || a.rope_q);
+    __shared__ __align__(16) float sfreq[ROPE ? HD / 2 : 4];
+    __shared__ __align__(16) unsigned char qrot[ROPE ? KS * 1024 : 16];
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -164,50 +169,82 @@ __global__ __launch_bounds__(KW * 64, 2) void prefill_attn_split_kernel(PrefillA
     auto issue_k = [&](int t) { issue(kbase, a.k_sn, t * KT, kslot, std::false_type{}); };
     auto issue_v = [&](int t) { issue(vbase, a.v_sn, t * KT, vslot, std::true_type{}); };
 
-    // ---- Q (B operand) of this lane's row, d = ks*16 + hh*8 + e, requested first
+    // ---- Q (B operand) of this lane's row, d = ks*16 + hh*8 + e, requested first. Where Q is
+    // rotated, the sines and cosines (sincosf, some 60 instructions a pair) are shared out: a
+    // wave rotates RE of a lane's 8 pairs in one pair of fragments (ks, ks + KS / 2), and the
+    // waves exchange the bf16 fragments through LDS (12/2 heads, 1000 rows behind 24, RoPE
+    // inside: 27.8 us where each wave rotates all of them, 24.4 shared).
+    constexpr int RE = ROPE ? KS * 4 / KW : 8;
+    typedef uint32_t rot_t __attribute__((ext_vector_type(RE / 2)));
+    const int rk = wave * RE / 8, re = wave * RE % 8, rd = rk * 16 + hh * 8 + re;
     uint4 qraw[KS];
+    rot_t r0{}, r1{};
+    float freq = 0.f;
     {
         const bool qv = qi < a.S;
         const bf16_t* qp = a.q + (size_t)(qv ? qi : 0) * a.q_sn + (size_t)head * a.q_sh;
+        if (rope_q) {
+            if (tid < HD / 2) freq = a.rope.inv_freq[tid];
+            if (qv) {
+                r0 = *reinterpret_cast<const rot_t*>(qp + rd);
+                r1 = *reinterpret_cast<const rot_t*>(qp + rd + HD / 2);
+            }
+        } else {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-            qraw[ks] = qv ? *reinterpret_cast<const uint4*>(qp + ks * 16 + hh * 8) : make_uint4(0, 0, 0, 0);
+            for (int ks = 0; ks < KS; ++ks)
+                qraw[ks] = qv ? *reinterpret_cast<const uint4*>(qp + ks * 16 + hh * 8) : make_uint4(0, 0, 0, 0);
+        }
     }
     if (wave < ntiles) {
         issue_k(wave);
         issue_v(wave);
     }
-    if constexpr (ROTK) {
-        if (tid < HD / 2) sfreq[tid] = a.rope.inv_freq[tid];
+    bf16x8_t qf[KS];
+    if (rope_q) {
+        if (tid < HD / 2) sfreq[tid] = freq;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-    }
-    bf16x8_t qf[KS];
-    {
-        float x[KS][8];
+        auto rotate = [&](float& x0, float& x1, int d) {
+            float sn, cs;
+            sincosf((float)(qi + a.q_pos_off) * sfreq[d], &sn, &cs);
+            const float y0 = x0 * cs - x1 * sn, y1 = x1 * cs + x0 * sn;
+            x0 = SCALE_Q ? y0 * a.sm_scale_log2 : y0;
+            x1 = SCALE_Q ? y1 * a.sm_scale_log2 : y1;
+        };
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) unpack8(qraw[ks], x[ks]);
-        if (a.rope_q) {
-            const float pos = (float)(qi + a.q_pos_off);
-#pragma unroll
-            for (int ks = 0; ks < KS / 2; ++ks)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int d = ks * 16 + hh * 8 + e;
-                    float sn, cs;
-                    sincos_reduced(pos * (ROTK ? sfreq[d] : a.rope.inv_freq[d]), &sn, &cs);
-                    const float x0 = x[ks][e], x1 = x[ks + KS / 2][e];
-                    x[ks][e] = x0 * cs - x1 * sn;
-                    x[ks + KS / 2][e] = x1 * cs + x0 * sn;
-                }
+        for (int e = 0; e < RE; e += 2) {
+            float x0 = __uint_as_float(r0[e / 2] << 16), x1 = __uint_as_float(r0[e / 2] & 0xffff0000u);
+            float y0 = __uint_as_float(r1[e / 2] << 16), y1 = __uint_as_float(r1[e / 2] & 0xffff0000u);
+            rotate(x0, y0, rd + e);
+            rotate(x1, y1, rd + e + 1);
+            r0[e / 2] = pack_bf16x2(x0, x1);
+            r1[e / 2] = pack_bf16x2(y0, y1);
         }
+        // fragment ks of lane l at 16 (64 ks + l)
+        unsigned char* const dst = qrot + rk * 1024 + lane * 16 + re * 2;
+        *reinterpret_cast<rot_t*>(dst) = r0;
+        *reinterpret_cast<rot_t*>(dst + KS * 512) = r1;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const uint32_t ra =
+            (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)qrot) + lane * 16;
+        [&]<int... I>(std::integer_sequence<int, I...>) {
+            (attn_pipe::read_b128<I * 1024>(qf[I], ra), ...);
+        }(std::make_integer_sequence<int, KS>{});
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+    } else {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
+            float x[8];
+            unpack8(qraw[ks], x);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[ks][e] *= SCALE_Q ? a.sm_scale_log2 : 1.f;
+            for (int e = 0; e < 8; ++e) x[e] *= SCALE_Q ? a.sm_scale_log2 : 1.f;
             Pack8 pk;
-            pk.u = pack8(x[ks]);
+            pk.u = pack8(x);
             qf[ks] = pk.v;
         }
     }

@@ -5,6 +5,7 @@ Mirrors tests/operators/test_attention_decode.py, test_norm_sampler.py,
 test_decode_linear.py and test_fused_gate_up_activation.py of the reference."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -1390,6 +1391,59 @@ def test_attention_split_error_against_64_bits(gpu, knob, op, hq, hkv, hd, S, L,
         torch.cuda.synchronize()
         errs.append(float((o.double() - ref).norm() / ref.norm()))
     assert errs[0] <= 1.005 * errs[1], errs
+
+
+@pytest.mark.parametrize("hd,mode,off", [
+    pytest.param(128, "prerot", 3, id="hd128_prerotated"),
+    pytest.param(128, "read", 3, id="hd128_rope"),
+    pytest.param(64, "read", 70000, id="hd64_rope_far"),
+    pytest.param(64, "prerot", 3, id="hd64_prerotated"),
+])
+def test_attention_prefill_split_query_rotation(gpu, knob, hd, mode, off):
+    """The query's sine and cosine in the split kernel are those of fp32 (sincosf), once per row.
+    Row i holds one pair (x0, x1) of bf16 values whose rotated x0 nearly cancels (1 to 3e-5 of
+    the pair), so that an error e of the sine or cosine is one of e / 2e-5 in its score; key 0 is
+    that channel alone, the other keys are zero, and the output is key 0's weight. Bound on the
+    rotated value: sine and cosine within an ulp (2^-24) and one product rounded to fp32, 2 x
+    2^-24 of the pair in all, and 2^-9 of itself where it is rounded to bf16; the weight's slope
+    in the score is p (1 - p), and it is rounded to bf16 twice. (Hardware sine and cosine: 1.6 to
+    1.9 times the bound.)"""
+    S, d, half = 512, 1, hd // 2
+    freq = np.float32(math.exp(-2.0 * d / hd * math.log(1.0e6)))
+    ang = (np.arange(S, dtype=np.float32) + np.float32(off)) * freq
+    c, s = np.cos(ang.astype(np.float64)), np.sin(ang.astype(np.float64))
+    pair, y0 = np.zeros((S, 2)), np.zeros(S)
+    x0 = np.arange(128, 256) / 128.0   # bf16 mantissas, and the largest bf16 x1 of no more than x0 |c / s|
+    for i in range(S):
+        x1 = x0 * abs(c[i] / s[i])
+        ulp = 2.0 ** (np.floor(np.log2(x1)) - 7)
+        x1 = np.floor(x1 / ulp) * ulp
+        y = x0 * abs(c[i]) - x1 * abs(s[i])
+        j = np.argmin(np.abs(y / np.hypot(x0, x1) - 2e-5))
+        pair[i], y0[i] = (x0[j] * np.sign(c[i]), x1[j] * np.sign(s[i])), y[j]
+    scale = 2.0 ** np.round(np.log2(4.1 * math.sqrt(hd) / y0) - 8)   # times key 0's 2^8
+    pair, y0 = pair * scale[:, None], y0 * scale
+    q = torch.zeros(S, 1, hd, dtype=torch.float64)
+    q[:, 0, d], q[:, 0, d + half] = torch.from_numpy(pair[:, 0]), torch.from_numpy(pair[:, 1])
+    assert torch.equal(q.bfloat16().double(), q)
+    k, v = torch.zeros(S, 1, hd), torch.zeros(S, 1, hd)
+    k[0, 0, d], v[0] = 256.0, 1.0
+    sc = y0 * 256.0 / math.sqrt(hd)
+    ref = np.exp(sc) / (np.exp(sc) + S - 1)
+    use = (y0 / np.hypot(*pair.T) > 1e-5) & (y0 / np.hypot(*pair.T) < 3e-5)
+    assert use.sum() > 100
+    err_s = 256.0 / math.sqrt(hd) * (2 * 2.0 ** -24 * np.hypot(*pair.T) + 2.0 ** -9 * y0)
+    bound = ref * (1 - ref) * err_s * 1.1 + 2.0 ** -8 * ref
+    qg, kg, vg = (t.to(torch.bfloat16).to(gpu) for t in (q, k, v))
+    ctx = C.make_attention_ctx(1, 1, hd, rope=True, q_rope_pos_offset=off, k_already_prerotated=mode == "prerot")
+    for register in (1, 0):
+        knob(C.EFM_KNOB_PREFILL_REGISTER, register)
+        o = torch.empty_like(qg)
+        C.call("efm_attention_prefill", ctx, ptr(qg), ptr(kg), ptr(vg), ptr(o), S, S, 0, stream())
+        torch.cuda.synchronize()
+        got = o[:, 0, 0].double().cpu().numpy()
+        over = np.abs(got - ref)[use] / bound[use]
+        assert over.max() <= 1, (register, float(over.max()))
 
 
 def test_attention_prefill_unaligned_rows(gpu):
