@@ -1100,7 +1100,9 @@ __global__ __launch_bounds__(KW * 64, 2) void sage_attn_split_kernel(SageArgs a,
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < KW; ++w) {
-            const float x = __builtin_amdgcn_exp2f(ml[0][w][r] - m);
+            // a row whose visible scores are all -inf has no weight in any wave (head_dim 128
+            // calls with more rows run the pipelined kernel, which makes such rows NaN)
+            const float x = HD == 64 && m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0][w][r] - m);
             const float4 v = reinterpret_cast<const float4*>(smem + w * SLOT)[r * CPR + (c ^ (r & 15))];
             l += x * ml[1][w][r];
             acc.x += x * v.x;

@@ -1446,6 +1446,42 @@ def test_attention_prefill_split_query_rotation(gpu, knob, hd, mode, off):
         assert over.max() <= 1, (register, float(over.max()))
 
 
+@pytest.mark.parametrize("op,hq,hkv,hd,L,mode", [
+    pytest.param("bf16", 14, 2, 64, 200, "none", id="hd64"),
+    pytest.param("bf16", 14, 2, 64, 1100, "read", id="hd64_rope_eight_waves"),
+    pytest.param("bf16", 12, 2, 128, 200, "read", id="rope"),
+    pytest.param("sage", 14, 2, 64, 200, "none", id="sage_hd64"),
+    pytest.param("sage", 14, 2, 64, 2100, "none", id="sage_hd64_eight_waves"),
+])
+def test_attention_split_rows_without_weight(gpu, knob, op, hq, hkv, hd, L, mode):
+    """Rows whose visible scores all overflow to -inf are 0, as in the register-staged kernel;
+    rows that also see a key of finite score (bf16: key L / 2 and later are 0) are its value."""
+    q, k = torch.zeros(L, hq, hd), torch.zeros(L, hkv, hd)
+    q[:, :, hd // 2 - 1] = 2.0 ** 100   # the pair of the lowest frequency
+    k[: L // 2, :, hd // 2 - 1] = -(2.0 ** 100)
+    if op == "sage":   # K less its mean: both signs, so only the first half of the rows is finite
+        k[L // 2:, :, hd // 2 - 1] = 2.0 ** 100
+    v = torch.randn(L, hkv, hd, generator=torch.Generator().manual_seed(L))
+    qg, kg, vg = (t.to(torch.bfloat16).to(gpu) for t in (q, k, v))
+    ctx = C.make_attention_ctx(hq, hkv, hd, rope=mode == "read")
+    ws = torch.zeros(C.load().efm_attention_prefill_sage_int8_workspace_bytes(ctx, L, L), dtype=torch.uint8, device=gpu)
+    for register in (1, 0):
+        knob(C.EFM_KNOB_PREFILL_REGISTER, register)
+        o = torch.full_like(qg, -7.0)
+        args = (ctx, ptr(qg), ptr(kg), ptr(vg), ptr(o), L, L, 1)
+        if op == "sage":
+            C.call("efm_attention_prefill_sage_int8", *args, ptr(ws), ws.numel(), stream())
+        else:
+            C.call("efm_attention_prefill", *args, stream())
+        torch.cuda.synchronize()
+        assert (o[: L // 2] == 0).all(), register
+        if op == "bf16":
+            h = torch.arange(hq, device=gpu) * hkv // hq
+            assert torch.equal(o[L // 2], vg[L // 2, h]), register
+            ref = (vg[L // 2:, h].double().cumsum(0) / torch.arange(1, L - L // 2 + 1, device=gpu)[:, None, None])
+            assert_close_bf16(o[L // 2:], ref.to(torch.bfloat16), rtol=2e-2, atol=2e-2)
+
+
 def test_attention_prefill_unaligned_rows(gpu):
     """head_dim 64 rows at an 8-byte (not 16-byte) aligned address: accepted as before."""
     torch.manual_seed(5)
