@@ -698,18 +698,20 @@ extern "C" int efm_attention_prefill(const efm_attention_ctx* ctx, const void* q
     a.sm_scale_log2 = 1.4426950408889634f / sqrtf((float)hd);
     const int cus = prefill_cus();
     const int knob = kernel_knob(EFM_KNOB_PREFILL_SHAPE);
-    const bool pipe_ok = hd == kP2HD && !a.rope_k;
-    // the split kernel's tile loads take 16-byte aligned rows and 32-bit offsets inside a
-    // tile, its grid 32-row blocks: anything else stays with the kernels below
-    const bool split_ok = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
-                            reinterpret_cast<uintptr_t>(v)) & 15u) == 0 &&
-                          std::max(ctx->k_stride_n, ctx->kv_stride_n) < (1u << 24) &&
-                          (long)((qo_len + 31) / 32) * a.Hq < (1L << 22);
-    if (prefill_pipe_enabled() && split_ok && (pipe_ok ? knob == 0 && prefill_split_wins(a, cus) : true)) {
+    // the tile loads of the split and pipelined kernels take 16-byte aligned rows and 32-bit
+    // offsets inside a tile; other operands stay with the register-staged kernel
+    const bool dma_ok = prefill_pipe_enabled() &&
+                        ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                          reinterpret_cast<uintptr_t>(v)) & 15u) == 0 &&
+                        std::max(ctx->k_stride_n, ctx->kv_stride_n) < (1u << 24);
+    const bool pipe_ok = dma_ok && hd == kP2HD && !a.rope_k;
+    // the split kernel's grid counts 32-row blocks
+    const bool split_ok = dma_ok && (long)((qo_len + 31) / 32) * a.Hq < (1L << 22);
+    if (split_ok && (pipe_ok ? knob == 0 && prefill_split_wins(a, cus) : true)) {
         prefill_split_launch(a, hd, cus, stream);
         return check_launch("attention_prefill");
     }
-    if (pipe_ok && prefill_pipe_enabled()) {
+    if (pipe_ok) {
         // 8 waves (256 rows, 4-deep ring, one workgroup per CU) when those workgroups fill
         // the chip; fewer rows (behind a long prefix; without one the split kernel takes
         // them): 4 waves (128 rows) over a 2-deep ring, two workgroups per CU. 28/4 heads,

@@ -1259,16 +1259,18 @@ extern "C" int efm_attention_prefill_sage_int8(const efm_attention_ctx* ctx, con
     float* km = reinterpret_cast<float*>(p + w.q8 + w.k8 + w.sq + w.sk);
     double* kp = reinterpret_cast<double*>(p + w.q8 + w.k8 + w.sq + w.sk + w.km);
     const int hd = (int)ctx->head_dim;
-    const bool fast = kernel_knob(EFM_KNOB_PREFILL_REGISTER) == 0;
     const int shape = kernel_knob(EFM_KNOB_PREFILL_SHAPE), cus = prefill_cus();
     const long blocks = (long)((qo_len + 31) / 32) * ctx->num_qo_heads;
-    // the split kernel's loads take 16-byte aligned rows and 32-bit offsets inside a tile,
-    // its grid 32-row blocks: anything else stays with the kernels below
-    const bool split_ok = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(v) |
-                            reinterpret_cast<uintptr_t>(workspace)) & 15u) == 0 &&
-                          ctx->kv_stride_n < (1u << 24) && blocks < (1L << 22);
-    const bool split = fast && split_ok && (hd == 64 || (shape == 0 && sage_split_wins(blocks, kv_len, causal != 0, cus)));
-    const bool pipe = fast && !split && hd == kSPHD;
+    // the tile loads of the split and pipelined kernels take 16-byte aligned rows and 32-bit
+    // offsets inside a tile; other operands stay with the register-staged kernel
+    const bool dma_ok = kernel_knob(EFM_KNOB_PREFILL_REGISTER) == 0 &&
+                        ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(v) |
+                          reinterpret_cast<uintptr_t>(workspace)) & 15u) == 0 &&
+                        ctx->kv_stride_n < (1u << 24);
+    // the split kernel's grid counts 32-row blocks
+    const bool split = dma_ok && blocks < (1L << 22) &&
+                       (hd == 64 || (shape == 0 && sage_split_wins(blocks, kv_len, causal != 0, cus)));
+    const bool pipe = dma_ok && !split && hd == kSPHD;
     // the split and pipelined kernels quantise Q themselves
     rc = sage_quantize_impl(ctx, q, k, qo_len, kv_len, q8, sq, k8, sk, km, stream, !split && !pipe, kp);
     if (rc) return rc;

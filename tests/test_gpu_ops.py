@@ -1498,6 +1498,51 @@ def test_attention_prefill_unaligned_rows(gpu):
     assert_close_bf16(o.reshape(S, hq, hd), ref, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("S", [70, 1500])
+@pytest.mark.parametrize("op,rope", [("bf16", False), ("bf16", True), ("sage", False)])
+@pytest.mark.parametrize("how", ["offset", "stride"])
+def test_attention_prefill_operands_without_dma(gpu, knob, op, rope, how, S):
+    """head_dim 128 operands that the tile loads cannot take (rows 8 bytes off a 16-byte
+    boundary; rows so far apart that a tile spans more than 32-bit offsets) run the
+    register-staged kernel, at row counts where aligned ones run the split and the pipelined
+    kernel: the same bits as the same rows through that kernel, packed."""
+    hq, hkv, hd = 28, 4, 128
+    L = 66 if how == "stride" else S
+    S = min(S, L)
+    g = torch.Generator(device=gpu).manual_seed(S)
+    q, k, v = (torch.empty(n, h, hd, dtype=torch.bfloat16, device=gpu).normal_(generator=g)
+               for n, h in ((S, hq), (L, hkv), (L, hkv)))
+    moved, kw = [q, k, v], {}
+    only_v = op == "sage"   # its q and k are quantised by another kernel
+    if how == "offset":
+        for i in (2,) if only_v else (0, 1, 2):
+            t = moved[i]
+            moved[i] = torch.zeros(t.numel() + 4, dtype=torch.bfloat16, device=gpu)[4:].view_as(t).copy_(t)
+            assert moved[i].data_ptr() % 16 == 8
+    else:   # one buffer of L rows, K and V side by side in each
+        sn = 1 << 25
+        rows = torch.empty(L, sn, dtype=torch.bfloat16, device=gpu)
+        kw = dict(kv_stride_n=sn, kv_stride_h=hd)
+        moved[2] = rows[:, hkv * hd:2 * hkv * hd].copy_(v.reshape(L, -1))
+        if not only_v:
+            kw.update(k_stride_n=sn, k_stride_h=hd)
+            moved[1] = rows[:, :hkv * hd].copy_(k.reshape(L, -1))
+    outs = []
+    for register, ts, c in ((1, (q, k, v), {}), (0, moved, kw)):
+        knob(C.EFM_KNOB_PREFILL_REGISTER, register)
+        ctx = C.make_attention_ctx(hq, hkv, hd, rope=rope, k_already_prerotated=rope, **c)
+        ws = torch.zeros(C.load().efm_attention_prefill_sage_int8_workspace_bytes(ctx, S, L), dtype=torch.uint8, device=gpu)
+        o = torch.empty_like(q)
+        args = (ctx, *(ptr(t) for t in ts), ptr(o), S, L, 1)
+        if op == "sage":
+            C.call("efm_attention_prefill_sage_int8", *args, ptr(ws), ws.numel(), stream())
+        else:
+            C.call("efm_attention_prefill", *args, stream())
+        torch.cuda.synchronize()
+        outs.append(o)
+    assert torch.equal(*outs)
+
+
 def test_attention_prefill_last_row_equals_decode(gpu):
     """The last prefill row equals single-query decode over the same cache (the
     reference's prefill/decode consistency)."""
