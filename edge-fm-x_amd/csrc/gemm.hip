@@ -885,8 +885,8 @@ static void gemm_splitk_launch(int M, int N, int K, const bf16_t* A, const bf16_
 }
 
 // Tiles of the slab kernel and what a launch of them takes, fitted to sweeps on MI355X over
-// weights that rotate through the memory-side cache (us). A launch is rounds of 256 x occ
-// resident workgroups. A round of c tiles per CU takes s us a 64-key slab: s0 at one tile on
+// weights that rotate through the memory-side cache (us, 256 CUs). A launch is rounds of occ
+// resident workgroups per CU. A round of c tiles per CU takes s us a 64-key slab: s0 at one tile on
 // few CUs rising to s1 at one on each (the same work draws more power, and the clock drops),
 // and from s1b just above one per CU to s2 at occ per CU; plus o us before the first and
 // after the last slab, which a next round hides where two workgroups share a CU. The deep
@@ -909,13 +909,13 @@ constexpr TallTile kTallTiles[] = {
     {2, 2, 2, 2.7, 0.21, 0.225, 0.38, 0.46},  // 64 x 64, D 4
 };
 static double tall_cost(const TallTile& t, long tiles, int slabs) {
-    const double cus = 256;
+    const int cus = prefill_cus();
     auto slab = [&](double c) {
         return c <= 1 ? t.s0 + (t.s1 - t.s0) * c : t.s1b + (t.s2 - t.s1b) * (c - 1) / (t.occ - 1);
     };
-    const long full = tiles / (256 * t.occ), rem = tiles % (256 * t.occ);
+    const long full = tiles / (cus * t.occ), rem = tiles % (cus * t.occ);
     const double o = t.occ == 1 ? t.o : 0;
-    return (t.occ == 1 ? 0 : t.o) + full * (o + slabs * slab(t.occ)) + (rem ? o + slabs * slab(rem / cus) : 0);
+    return (t.occ == 1 ? 0 : t.o) + full * (o + slabs * slab(t.occ)) + (rem ? o + slabs * slab((double)rem / cus) : 0);
 }
 
 template <int EPI>
