@@ -211,21 +211,7 @@ __device__ __forceinline__ void vm_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Waits until at most `slabs` slabs of LPW loads are in flight (the counter holds 63: past
-// that the wait is for fewer).
-constexpr int vm_count(int loads) { return loads < 63 ? loads : 63; }
-template <int LPW>
-__device__ __forceinline__ void vm_wait_slabs(int slabs) {
-    switch (slabs) {
-        case 0: vm_wait<0>(); break;
-        case 1: vm_wait<vm_count(1 * LPW)>(); break;
-        case 2: vm_wait<vm_count(2 * LPW)>(); break;
-        case 3: vm_wait<vm_count(3 * LPW)>(); break;
-        case 4: vm_wait<vm_count(4 * LPW)>(); break;
-        case 5: vm_wait<vm_count(5 * LPW)>(); break;
-        default: vm_wait<vm_count(6 * LPW)>(); break;
-    }
-}
+constexpr int vm_count(int loads) { return loads < 63 ? loads : 63; }   // the counter holds 63
 
 template <int OFF>
 __device__ __forceinline__ bf16x8_t ds_read16(uint32_t addr) {
@@ -510,32 +496,35 @@ __global__ __launch_bounds__(256, tall_lds(TM, TN, D) <= 80 * 1024 ? 2 : 1) void
 // ---------------------------------------------------------------------------------
 // K split over the waves of a workgroup: for launches whose tiles are too few to keep the
 // CUs busy by themselves. The slab kernel's four waves share every slab and meet at a barrier
-// for each. Here each of KW waves owns a contiguous range of the slabs and the whole 32 TM x
-// 32 TN tile, with an S-deep LDS ring of its own: no barrier until the partial tiles are
-// summed through LDS, in wave order.
+// for each. Here each of four waves owns a contiguous range of the slabs and the whole 32 TM
+// x 32 TN tile, with a ring of two slabs in LDS of its own: no barrier until the partial tiles
+// are summed through LDS, in wave order.
 //  * A slab's operand reads are all issued one slab ahead of their MFMAs (two register
 //    sets); its LDS slot is refilled as soon as they have landed.
 //  * The weight rows are the MFMA's first operand, so a lane ends with four consecutive
 //    columns of one row: float4 partials, 16-byte output stores.
 //  * SwiGLU: the tile's first half of weight rows is up, the second gate.
 // ---------------------------------------------------------------------------------
+constexpr int kKsplitWaves = 4, kKsplitRing = 2;
+
 template <int TM, int TN>
 struct KsplitFrags {
     bf16x8_t a[kPBK / 16][TM], b[kPBK / 16][TN];
 };
 
-template <int TM, int TN, int KW, int S, int EPI, int WPE>
-__global__ __launch_bounds__(KW * kWave, WPE) void gemm_ksplit_kernel(const bf16_t* __restrict__ A,
+template <int TM, int TN, int EPI, int WPE>
+__global__ __launch_bounds__(kKsplitWaves * kWave, WPE) void gemm_ksplit_kernel(const bf16_t* __restrict__ A,
                                                                  const bf16_t* __restrict__ B,
                                                                  const bf16_t* __restrict__ bias,
                                                                  void* __restrict__ Cout, int M, int N, int K, int ldc,
                                                                  int mt, int nt, int vec, int kslices, int slice_slabs) {
+    constexpr int KW = kKsplitWaves, S = kKsplitRing;
     constexpr int BM = 32 * TM, BN = 32 * TN, KSN = kPBK / 16;
     constexpr int OC = EPI == GEPI_SWIGLU ? BN / 2 : BN;   // output columns per tile
     constexpr int STAGE = (BM + BN) * kPRow, RING = S * STAGE;
     constexpr int LA = BM / 8, LPS = (BM + BN) / 8;        // 1 KB wave loads per slab
     constexpr int CH = BN / 4;                             // float4 chunks per partial row
-    static_assert(S >= 2 && S * LPS <= 63 && BM * BN * 4 <= RING, "bad K-split shape");
+    static_assert(S == 2 && BM * BN * 4 <= RING, "bad K-split shape");
     __shared__ __align__(1024) unsigned char smem[KW * RING];
 
     // GEPI_PARTIAL: work unit t covers slice t / (mt * nt) of the slabs
@@ -616,7 +605,8 @@ __global__ __launch_bounds__(KW * kWave, WPE) void gemm_ksplit_kernel(const bf16
         }
         if (i + S < n_slabs) issue(i + S);
         if (i + 1 < n_slabs) {
-            vm_wait_slabs<LPS>(min(S - 1, n_slabs - 2 - i));
+            if (i + 2 < n_slabs) vm_wait<LPS>();   // slab i + 2 may be in flight
+            else vm_wait<0>();
             asm volatile("" ::: "memory");
             read(g, i + 1);
         }
@@ -630,7 +620,8 @@ __global__ __launch_bounds__(KW * kWave, WPE) void gemm_ksplit_kernel(const bf16
     };
     if (n_slabs > 0) {
         for (int p = 0; p < min(S, n_slabs); ++p) issue(p);
-        vm_wait_slabs<LPS>(min(S, n_slabs) - 1);
+        if (n_slabs > 1) vm_wait<LPS>();
+        else vm_wait<0>();
         asm volatile("" ::: "memory");
         Frags f, g;
         read(f, 0);
@@ -761,15 +752,15 @@ static void gemm_tall_launch(int M, int N, int K, const bf16_t* A, const bf16_t*
                        vec, kslices, slice_slabs);
 }
 
-template <int TM, int TN, int KW, int S, int EPI, int WPE>
+template <int TM, int TN, int EPI, int WPE>
 static void gemm_ksplit_launch(int M, int N, int K, const bf16_t* A, const bf16_t* B, const bf16_t* bias, void* C,
                                int ldc, hipStream_t stream, int kslices = 1, int slice_slabs = 1 << 30) {
     const int oc = (EPI == GEPI_SWIGLU) ? 16 * TN : 32 * TN;
     const int mt = (M + 32 * TM - 1) / (32 * TM), nt = (N + oc - 1) / oc;
     const int grid = 8 * ((mt * nt * kslices + 7) / 8);
     const int vec = N % 4 == 0 && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
-    hipLaunchKernelGGL((gemm_ksplit_kernel<TM, TN, KW, S, EPI, WPE>), dim3(grid), dim3(KW * kWave), 0, stream, A, B, bias,
-                       C, M, N, K, ldc, mt, nt, vec, kslices, slice_slabs);
+    hipLaunchKernelGGL((gemm_ksplit_kernel<TM, TN, EPI, WPE>), dim3(grid), dim3(kKsplitWaves * kWave), 0, stream, A, B,
+                       bias, C, M, N, K, ldc, mt, nt, vec, kslices, slice_slabs);
 }
 
 int prefill_cus();
@@ -869,11 +860,11 @@ static void gemm_splitk_launch(int M, int N, int K, const bf16_t* A, const bf16_
                                bool f32out, float* part, const SplitK& p, hipStream_t stream) {
     const int mt = (M + 127) / 128, nt = (N + 127) / 128;
     if (p.tile == 1)
-        gemm_ksplit_launch<1, 1, 4, 2, GEPI_PARTIAL, 2>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
+        gemm_ksplit_launch<1, 1, GEPI_PARTIAL, 2>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     else if (p.tile == 2)
-        gemm_ksplit_launch<2, 1, 4, 2, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
+        gemm_ksplit_launch<2, 1, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     else if (p.tile == 3)
-        gemm_ksplit_launch<2, 2, 4, 2, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
+        gemm_ksplit_launch<2, 2, GEPI_PARTIAL, 1>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     else if (mt * nt * p.ksplit <= prefill_cus())
         gemm_tall_launch<4, 4, 4, GEPI_PARTIAL>(M, N, K, A, B, nullptr, part, N, stream, p.ksplit, p.kt_per);
     else
@@ -932,17 +923,20 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
     if (tile_knob == 0) {
         switch (ksplit_tile(M, N, K, EPI == GEPI_SWIGLU)) {
             case 1:
-                gemm_ksplit_launch<1, 1, 4, 2, EPI, 2>(M, N, K, A, B, bias, C, ldc, stream);
+                gemm_ksplit_launch<1, 1, EPI, 2>(M, N, K, A, B, bias, C, ldc, stream);
                 return check_launch("gemm_bf16");
             case 2:
                 if constexpr (EPI != GEPI_SWIGLU) {
-                    gemm_ksplit_launch<2, 1, 4, 2, EPI, 1>(M, N, K, A, B, bias, C, ldc, stream);
+                    gemm_ksplit_launch<2, 1, EPI, 1>(M, N, K, A, B, bias, C, ldc, stream);
                     return check_launch("gemm_bf16");
                 }
                 break;
             case 3:
-                gemm_ksplit_launch<2, 2, 4, 2, EPI, 1>(M, N, K, A, B, bias, C, ldc, stream);
-                return check_launch("gemm_bf16");
+                if constexpr (EPI != GEPI_SWIGLU) {
+                    gemm_ksplit_launch<2, 2, EPI, 1>(M, N, K, A, B, bias, C, ldc, stream);
+                    return check_launch("gemm_bf16");
+                }
+                break;
             default: break;
         }
     }
