@@ -888,7 +888,7 @@ struct TallTile {
     int tm, tn, occ;
     double o, s0, s1, s1b, s2;
 };
-constexpr TallTile kTallTiles[] = {
+constexpr TallTile kTallTiles[] = {   // EFM_KNOB_GEMM_TILE 10, 11, ...
     {8, 8, 1, 8.0, 1.05, 1.42, 0, 0},         // 256 x 256, D 2
     {6, 8, 1, 7.4, 0.72, 1.06, 0, 0},         // 192 x 256, D 2
     {6, 4, 1, 4.7, 0.47, 0.56, 0, 0},         // 192 x 128, D 3
@@ -941,8 +941,8 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
         }
     }
     if (slab_ok) {
-        // the cheapest tile (EFM_KNOB_GEMM_TILE 1: of the tiles up to 128 x 128)
-        int pick = tile_knob == 3 ? 1 : 0;
+        // the cheapest tile (EFM_KNOB_GEMM_TILE 1: of the tiles up to 128 x 128), or the knob's
+        int pick = tile_knob >= 10 ? tile_knob - 10 : tile_knob == 3 ? 1 : 0;
         if (tile_knob < 2) {
             double best = 0;
             for (int i = tile_knob == 1 ? 3 : 0; i < (int)std::size(kTallTiles); ++i) {

@@ -72,7 +72,10 @@ int efm_init(void);
  *                              kernel treats 2 as 4)
  *   EFM_KNOB_GEMM_TILE         prefill GEMM kernel (K % 64 == 0): 1 the tiles up to 128 x
  *                              128, 2 the one-workgroup-per-CU 256 x 256 tile, 3 the
- *                              192 x 256 tile (none splits K over the waves)
+ *                              192 x 256 tile; 10 to 18 one tile and ring each: 256 x
+ *                              256, 192 x 256, 192 x 128, 128 x 128 (rings of 4 and 2
+ *                              slabs), 128 x 64 (4, 2), 64 x 128, 64 x 64 (none splits K
+ *                              over the waves)
  *   EFM_KNOB_FRONT_WAIT_TIMEOUT 1: efm_decode_norm_qkv_attention launches whose attention
  *                              workgroups wait for a tag that no projected word carries,
  *                              with a 64-poll limit: every wait gives up, the launch
