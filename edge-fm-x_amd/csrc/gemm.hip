@@ -253,6 +253,30 @@ __device__ __forceinline__ void lgkm_wait() {
 // ---------------------------------------------------------------------------------
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
+// N consecutive columns of an output row, `left` of them inside the matrix. Whole segments go
+// as 16-byte (bf16 of four: 8-byte) stores whatever their alignment, which the hardware takes:
+// rows of a ragged N start anywhere (3052 x 64 -> 36014: 191 us with a store per column).
+template <int N, typename T>
+__device__ __forceinline__ void store_cols(T* o, const float* v, int left) {
+    if (left >= N) {
+        if constexpr (sizeof(T) == 4) {
+            __builtin_memcpy(o, v, N * 4);
+        } else {
+            uint32_t w[N / 2];
+#pragma unroll
+            for (int e = 0; e < N; e += 2) w[e / 2] = pack_bf16x2(v[e], v[e + 1]);
+            __builtin_memcpy(o, w, N * 2);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+            if (e < left) {
+                if constexpr (sizeof(T) == 4) o[e] = v[e];
+                else o[e] = (bf16_t)f32_to_bf16(v[e]);
+            }
+    }
+}
+
 __device__ __forceinline__ void tall_load(const unsigned char* src, uint32_t off, unsigned char* dst) {
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(src), (short)0, 0x7fffffff, 0x00020000);
@@ -280,7 +304,7 @@ constexpr int tall_lds(int tm, int tn, int d) { return 32 * kPRow * ((d + 1) * t
 template <int TM, int TN, int D, int EPI>
 __global__ __launch_bounds__(256, tall_lds(TM, TN, D) <= 80 * 1024 ? 2 : 1) void gemm_tall_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                            const bf16_t* __restrict__ bias, void* __restrict__ Cout,
-                                                           int M, int N, int K, int ldc, int mt, int nt, int vec,
+                                                           int M, int N, int K, int ldc, int mt, int nt,
                                                            int kslices, int slice_slabs) {
     constexpr int BM = 32 * TM, BN = 32 * TN;       // a wave: TM x TN tiles of 16 x 16
     constexpr int ASZ = BM * kPRow, BSZ = BN * kPRow;   // an operand slab (64 keys)
@@ -430,10 +454,11 @@ __global__ __launch_bounds__(256, tall_lds(TM, TN, D) <= 80 * 1024 ? 2 : 1) void
     // theirs), so that the stores are whole row segments, LPR lanes to a row.
     constexpr int SLOT = (B0 + D * BSZ) / 4 / 1024 * 1024;
     constexpr int H = TM / 2, CPR = TN * 4, LPR = TN * 2, RPP = kWave / LPR;
+    constexpr int NV = EPI == GEPI_SWIGLU ? 4 : 8;   // columns a lane stores
     static_assert(H * 16 * CPR * 16 <= SLOT, "half a wave's tile fits a slot");
     float4* const part = reinterpret_cast<float4*>(smem + wave * SLOT);
     const int seg = lane % LPR;
-    const int col = n0 + wn * (EPI == GEPI_SWIGLU ? BN / 4 : BN / 2) + seg * (EPI == GEPI_SWIGLU ? 4 : 8);
+    const int col = n0 + wn * (LPR * NV) + seg * NV;
     float bv[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e)
@@ -451,7 +476,6 @@ __global__ __launch_bounds__(256, tall_lds(TM, TN, D) <= 80 * 1024 ? 2 : 1) void
         for (int q = 0; q < H * 16 / RPP; ++q) {
             const int r = q * RPP + lane / LPR;
             const int row = m0 + wm * (BM / 2) + i0 * 16 + r, sw = (r & 15) % CPR;
-            constexpr int NV = EPI == GEPI_SWIGLU ? 4 : 8;
             const int c0 = EPI == GEPI_SWIGLU ? (seg >> 2) * 8 + (seg & 3) : seg * 2;
             const float4 x = part[r * CPR + (c0 ^ sw)], y = part[r * CPR + ((c0 + (EPI == GEPI_SWIGLU ? 4 : 1)) ^ sw)];
             float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
@@ -462,31 +486,8 @@ __global__ __launch_bounds__(256, tall_lds(TM, TN, D) <= 80 * 1024 ? 2 : 1) void
             }
             if (row >= M) continue;
             const size_t at = (size_t)(EPI == GEPI_PARTIAL ? (size_t)slice * M + row : (size_t)row) * ldc + col;
-            if constexpr (EPI == GEPI_F32 || EPI == GEPI_PARTIAL) {
-                float* o = reinterpret_cast<float*>(Cout) + at;
-                if (vec) {
-                    if (col < N) {
-                        *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
-                        *reinterpret_cast<float4*>(o + 4) = make_float4(v[4], v[5], v[6], v[7]);
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < NV; ++e)
-                        if (col + e < N) o[e] = v[e];
-                }
-            } else {
-                bf16_t* o = reinterpret_cast<bf16_t*>(Cout) + at;
-                if (vec) {
-                    if (col < N) {
-                        if constexpr (NV == 8) *reinterpret_cast<uint4*>(o) = pack8(v);
-                        else *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < NV; ++e)
-                        if (col + e < N) o[e] = (bf16_t)f32_to_bf16(v[e]);
-                }
-            }
+            if constexpr (EPI == GEPI_F32 || EPI == GEPI_PARTIAL) store_cols<8>(reinterpret_cast<float*>(Cout) + at, v, N - col);
+            else store_cols<NV>(reinterpret_cast<bf16_t*>(Cout) + at, v, N - col);
         }
     };
     half(std::integral_constant<int, 0>{});
@@ -517,7 +518,7 @@ __global__ __launch_bounds__(kKsplitWaves * kWave, WPE) void gemm_ksplit_kernel(
                                                                  const bf16_t* __restrict__ B,
                                                                  const bf16_t* __restrict__ bias,
                                                                  void* __restrict__ Cout, int M, int N, int K, int ldc,
-                                                                 int mt, int nt, int vec, int kslices, int slice_slabs) {
+                                                                 int mt, int nt, int kslices, int slice_slabs) {
     constexpr int KW = kKsplitWaves, S = kKsplitRing;
     constexpr int BM = 32 * TM, BN = 32 * TN, KSN = kPBK / 16;
     constexpr int OC = EPI == GEPI_SWIGLU ? BN / 2 : BN;   // output columns per tile
@@ -674,28 +675,8 @@ __global__ __launch_bounds__(kKsplitWaves * kWave, WPE) void gemm_ksplit_kernel(
             for (int e = 0; e < 4; ++e) v[e] += col + e < N ? bf16_to_f32(bias[col + e]) : 0.f;
         }
         const size_t at = (size_t)(EPI == GEPI_PARTIAL ? (size_t)slice * M + row : (size_t)row) * ldc + col;
-        if (EPI == GEPI_F32 || EPI == GEPI_PARTIAL) {
-            float* o = reinterpret_cast<float*>(Cout) + at;
-            if (vec) {
-                *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (col + e < N) o[e] = v[e];
-            }
-        } else {
-            bf16_t* o = reinterpret_cast<bf16_t*>(Cout) + at;
-            if (vec) {
-                uint2 w;
-                w.x = pack_bf16x2(v[0], v[1]);
-                w.y = pack_bf16x2(v[2], v[3]);
-                *reinterpret_cast<uint2*>(o) = w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (col + e < N) o[e] = (bf16_t)f32_to_bf16(v[e]);
-            }
-        }
+        if constexpr (EPI == GEPI_F32 || EPI == GEPI_PARTIAL) store_cols<4>(reinterpret_cast<float*>(Cout) + at, v, N - col);
+        else store_cols<4>(reinterpret_cast<bf16_t*>(Cout) + at, v, N - col);
     }
 }
 
@@ -747,9 +728,8 @@ static void gemm_tall_launch(int M, int N, int K, const bf16_t* A, const bf16_t*
     const int ocols = (EPI == GEPI_SWIGLU) ? 16 * TN : 32 * TN;
     const int mt = (M + 32 * TM - 1) / (32 * TM), nt = (N + ocols - 1) / ocols;
     const int grid = 8 * ((mt * nt * kslices + 7) / 8);
-    const int vec = N % 8 == 0 && ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
     hipLaunchKernelGGL((gemm_tall_kernel<TM, TN, D, EPI>), dim3(grid), dim3(256), 0, stream, A, B, bias, C, M, N, K, ldc, mt, nt,
-                       vec, kslices, slice_slabs);
+                       kslices, slice_slabs);
 }
 
 template <int TM, int TN, int EPI, int WPE>
@@ -758,9 +738,8 @@ static void gemm_ksplit_launch(int M, int N, int K, const bf16_t* A, const bf16_
     const int oc = (EPI == GEPI_SWIGLU) ? 16 * TN : 32 * TN;
     const int mt = (M + 32 * TM - 1) / (32 * TM), nt = (N + oc - 1) / oc;
     const int grid = 8 * ((mt * nt * kslices + 7) / 8);
-    const int vec = N % 4 == 0 && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
     hipLaunchKernelGGL((gemm_ksplit_kernel<TM, TN, EPI, WPE>), dim3(grid), dim3(kKsplitWaves * kWave), 0, stream, A, B,
-                       bias, C, M, N, K, ldc, mt, nt, vec, kslices, slice_slabs);
+                       bias, C, M, N, K, ldc, mt, nt, kslices, slice_slabs);
 }
 
 int prefill_cus();

@@ -919,6 +919,29 @@ def test_linear_unaligned_output(gpu):
     assert_close_bf16(aligned[:3], O.linear(x[:3].cpu(), w.cpu()))
 
 
+@pytest.mark.parametrize("m,k,n,kind", [
+    pytest.param(300, 256, 1000, "bias", id="slab"),
+    pytest.param(300, 256, 1000, "f32", id="slab_f32"),
+    pytest.param(70, 192, 200, "swiglu", id="slab_swiglu"),
+    pytest.param(20, 1536, 1000, "bias", id="k_split"),
+    pytest.param(20, 1536, 1000, "f32", id="k_split_f32"),
+    pytest.param(20, 896, 200, "swiglu", id="k_split_swiglu"),
+])
+def test_gemm_output_one_element_off(gpu, m, k, n, kind):
+    """Every epilogue stores whole segments at any alignment: an output one element behind a
+    16-byte boundary holds the aligned call's bits, and its neighbours are untouched."""
+    torch.manual_seed(m + n)
+    x = torch.randn(m, k, dtype=torch.bfloat16, device=gpu)
+    w = (torch.randn((2 if kind == "swiglu" else 1) * n, k, device=gpu) * 0.05).to(torch.bfloat16)
+    b = (torch.randn(n, device=gpu) * 0.05).to(torch.bfloat16) if kind == "bias" else None
+    buf = [torch.full((m * n + 16,), -7.0, dtype=torch.float32 if kind == "f32" else torch.bfloat16, device=gpu)
+           for _ in range(2)]
+    for t, at in zip(buf, (8, 1)):
+        _gemm_call(kind, m, k, n, x, w, b, t[at:])
+        assert (t[:at] == -7.0).all() and (t[at + m * n:] == -7.0).all()
+    assert torch.equal(buf[0][8:8 + m * n], buf[1][1:1 + m * n])
+
+
 def test_linear_under_graph_capture(gpu):
     """A prefill GEMM captured into a HIP graph: every replay equals the eager call bit for
     bit, with eager calls between replays."""
