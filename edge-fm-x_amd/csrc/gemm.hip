@@ -755,12 +755,18 @@ int prefill_cus();
 // 9.8 / 8.0, 256 x 2048 -> 2560 10.2 / 8.7. Against the kernels before either: 37 x 1536 ->
 // 2048 4.4 / 9.9, 19 x 896 -> 1152 4.3 / 6.7, 24 x 1536 -> 17920 14.2 / 20.0, 24 x 8960 -> 1536
 // 13.6 / 17.4 (sliced). SwiGLU only up to 32 rows: 24 x 1536 -> 8960 14.6 / 16.7, 16 x 3584 ->
-// 18944 48.1 / 67.8; 60 x 896 -> 4864 7.6 / 5.8.
+// 18944 48.1 / 67.8; 60 x 896 -> 4864 7.6 / 5.8; and not where its second round of two tiles per
+// CU is nearly full, which the slab kernel's 64 x 64 tiles cover in one: 5 x 896 -> 2 x 15872
+// 13.7 / 12.6, up to 15 % over 70 shapes with K of 1280 to 3584, save K of 2048 and 4096, where
+// this kernel stays up to 15 % ahead.
 constexpr int kMaxSlabK = 1 << 21;   // 32-bit byte offsets into the 256 rows of a tile
 static int ksplit_tile(int M, int N, int K, bool swiglu) {
     const int cus = prefill_cus(), nk = K / kPBK;
     if (K % kPBK != 0 || nk < 12 || K > kMaxSlabK) return 0;
-    if (M <= 32) return 1;
+    if (M <= 32) {
+        const long t = swiglu ? ((long)N + 15) / 16 : 0;
+        return t > 3 * cus && t <= 4 * cus && nk % 32 != 0 ? 0 : 1;
+    }
     const long mt32 = (M + 31) / 32, mt64 = (M + 63) / 64, nt32 = ((long)N + 31) / 32, nt64 = ((long)N + 63) / 64;
     if (swiglu) return 0;
     if (M > 64 && nk >= 128) return 0;
