@@ -783,10 +783,12 @@ static int ksplit_tile(int M, int N, int K, bool swiglu) {
 //    (one) workgroups per CU: 24 x 8960 -> 1536 17.4 -> 8.9, 19 x 4864 -> 896 17.6 -> 7.3,
 //    60 x 11008 -> 2048 22.3 -> 16.6, 24 x 18944 -> 3584 35.2 -> 31.2 (128 x 128 tiles
 //    before); 64 x 18944 -> 3584 stays (36.7 against 40.4);
-//  * more rows, half the CUs in 64 x 64 tiles at most and at most 64 MB of weights: the
-//    K-split kernel's 64 x 64 tiles, one workgroup per CU: 300 x 8960 -> 1536 24.0 -> 19.9,
-//    128 x 8960 -> 1536 20.1 -> 13.4, 300 x 4864 -> 896 20.7 -> 12.9; 128 x 18944 -> 3584
-//    stays (39.5 against 49.1);
+//  * more rows, a third of the CUs in 64 x 64 tiles at most and at most 64 MB of weights: the
+//    K-split kernel's 64 x 64 tiles, one workgroup per CU: 128 x 8960 -> 1536 20.1 -> 13.4,
+//    300 x 4864 -> 896 20.7 -> 12.9. 128 x 18944 -> 3584 stays (39.5 against 49.1), and so do
+//    launches with room for two slices only (118 shapes 11 % slower than 128 x 128 tiles at
+//    the geometric mean, 59 with three slices 3 % faster: 188 x 11008 -> 2048 29.7 against
+//    24.5, 104 x 8960 -> 1536, five slices, 15.2 against 19.2);
 //  * K < 8192 and a 64 x 64 tile (or fewer rows: a 32 x 32 tile) for every CU: unsliced
 //    (ksplit_tile): 700 x 4864 -> 896 24.2 -> 18.6;
 //  * else 128 x 128 tiles of the slab kernel, slices chosen the same way over two workgroups
@@ -821,7 +823,7 @@ static SplitK splitk_plan(int M, int N, int K) {
         ks = fill_slices(t, slots);
     } else if (nk < 128 && mt32 * nt32 <= cus) {
         return p;
-    } else if (2 * mt64 * nt64 <= cus && small_w) {
+    } else if (3 * mt64 * nt64 <= cus && small_w) {
         p.tile = 3;
         ks = (int)std::min<long>(most, cus / (mt64 * nt64));
     } else if (nk < 128 && mt64 * nt64 <= cus) {
