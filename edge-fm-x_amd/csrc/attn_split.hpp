@@ -120,11 +120,12 @@ __global__ __launch_bounds__(KW * 64, 2) void prefill_attn_split_kernel(PrefillA
     static_assert(KW >= (ROTK ? 4 : 2) && NL == 8 && 32 * HD * 4 <= SLOT, "tile geometry");
     __shared__ __align__(1024) unsigned char smem[KW * SLOT];
     __shared__ float ml[2][KW][32];
-    // frequencies and rotated Q fragments; KW 2 takes no RoPE, so that four workgroups fit a CU
-    constexpr bool ROPE = KW >= 4;
-    const bool rope_q = ROPE && (ROTK || a.rope_q);
-    __shared__ __align__(16) float sfreq[ROPE ? HD / 2 : 4];
-    __shared__ __align__(16) unsigned char qrot[ROPE ? KS * 1024 : 16];
+    // frequencies and Q fragments; KW 2 takes no RoPE and shares no Q, so that four workgroups
+    // fit a CU
+    constexpr bool SHARE = KW >= 4;
+    const bool rope_q = ROTK || a.rope_q;
+    __shared__ __align__(16) float sfreq[SHARE ? HD / 2 : 4];
+    __shared__ __align__(16) unsigned char qfrag[SHARE ? KS * 1024 : 16];
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -169,12 +170,12 @@ __global__ __launch_bounds__(KW * 64, 2) void prefill_attn_split_kernel(PrefillA
     auto issue_k = [&](int t) { issue(kbase, a.k_sn, t * KT, kslot, std::false_type{}); };
     auto issue_v = [&](int t) { issue(vbase, a.v_sn, t * KT, vslot, std::true_type{}); };
 
-    // ---- Q (B operand) of this lane's row, d = ks*16 + hh*8 + e, requested first. Where Q is
-    // rotated, the sines and cosines (sincosf, some 60 instructions a pair) are shared out: a
-    // wave rotates RE of a lane's 8 pairs in one pair of fragments (ks, ks + KS / 2), and the
-    // waves exchange the bf16 fragments through LDS (12/2 heads, 1000 rows behind 24, RoPE
-    // inside: 27.8 us where each wave rotates all of them, 24.4 shared).
-    constexpr int RE = ROPE ? KS * 4 / KW : 8;
+    // ---- Q (B operand) of this lane's row, d = ks*16 + hh*8 + e, requested first. A wave loads,
+    // rotates and rounds RE of a lane's 8 values in each of one pair of fragments (ks, ks + KS /
+    // 2), and the waves exchange the fragments through LDS: the loads, and with RoPE the sines
+    // and cosines (sincosf, some 60 instructions a pair), are shared out (12/2 heads, 1000 rows
+    // behind 24, RoPE inside: 27.8 us where each wave rotates all of them, 24.4 shared).
+    constexpr int RE = SHARE ? KS * 4 / KW : 8;
     typedef uint32_t rot_t __attribute__((ext_vector_type(RE / 2)));
     const int rk = wave * RE / 8, re = wave * RE % 8, rd = rk * 16 + hh * 8 + re;
     uint4 qraw[KS];
@@ -183,8 +184,8 @@ __global__ __launch_bounds__(KW * 64, 2) void prefill_attn_split_kernel(PrefillA
     {
         const bool qv = qi < a.S;
         const bf16_t* qp = a.q + (size_t)(qv ? qi : 0) * a.q_sn + (size_t)head * a.q_sh;
-        if (rope_q) {
-            if (tid < HD / 2) freq = a.rope.inv_freq[tid];
+        if constexpr (SHARE) {
+            if (rope_q && tid < HD / 2) freq = a.rope.inv_freq[tid];
             if (qv) {
                 r0 = *reinterpret_cast<const rot_t*>(qp + rd);
                 r1 = *reinterpret_cast<const rot_t*>(qp + rd + HD / 2);
@@ -200,36 +201,44 @@ __global__ __launch_bounds__(KW * 64, 2) void prefill_attn_split_kernel(PrefillA
         issue_v(wave);
     }
     bf16x8_t qf[KS];
-    if (rope_q) {
-        if (tid < HD / 2) sfreq[tid] = freq;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        auto rotate = [&](float& x0, float& x1, int d) {
-            float sn, cs;
-            sincosf((float)(qi + a.q_pos_off) * sfreq[d], &sn, &cs);
-            const float y0 = x0 * cs - x1 * sn, y1 = x1 * cs + x0 * sn;
-            x0 = SCALE_Q ? y0 * a.sm_scale_log2 : y0;
-            x1 = SCALE_Q ? y1 * a.sm_scale_log2 : y1;
+    if constexpr (SHARE) {
+        if (rope_q) {
+            if (tid < HD / 2) sfreq[tid] = freq;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+        auto prepare = [&](float& x0, float& x1, int d) {
+            if (rope_q) {
+                float sn, cs;
+                sincosf((float)(qi + a.q_pos_off) * sfreq[d], &sn, &cs);
+                const float y0 = x0 * cs - x1 * sn;
+                x1 = x1 * cs + x0 * sn;
+                x0 = y0;
+            }
+            if constexpr (SCALE_Q) {
+                x0 *= a.sm_scale_log2;
+                x1 *= a.sm_scale_log2;
+            }
         };
 #pragma unroll
         for (int e = 0; e < RE; e += 2) {
             float x0 = __uint_as_float(r0[e / 2] << 16), x1 = __uint_as_float(r0[e / 2] & 0xffff0000u);
             float y0 = __uint_as_float(r1[e / 2] << 16), y1 = __uint_as_float(r1[e / 2] & 0xffff0000u);
-            rotate(x0, y0, rd + e);
-            rotate(x1, y1, rd + e + 1);
+            prepare(x0, y0, rd + e);
+            prepare(x1, y1, rd + e + 1);
             r0[e / 2] = pack_bf16x2(x0, x1);
             r1[e / 2] = pack_bf16x2(y0, y1);
         }
         // fragment ks of lane l at 16 (64 ks + l)
-        unsigned char* const dst = qrot + rk * 1024 + lane * 16 + re * 2;
+        unsigned char* const dst = qfrag + rk * 1024 + lane * 16 + re * 2;
         *reinterpret_cast<rot_t*>(dst) = r0;
         *reinterpret_cast<rot_t*>(dst + KS * 512) = r1;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const uint32_t ra =
-            (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)qrot) + lane * 16;
+            (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)qfrag) + lane * 16;
         [&]<int... I>(std::integer_sequence<int, I...>) {
             (attn_pipe::read_b128<I * 1024>(qf[I], ra), ...);
         }(std::make_integer_sequence<int, KS>{});
