@@ -868,9 +868,11 @@ static void gemm_splitk_launch(int M, int N, int K, const bf16_t* A, const bf16_
 // few CUs rising to s1 at one on each (the same work draws more power, and the clock drops),
 // and from s1b just above one per CU to s2 at occ per CU; plus o us before the first and
 // after the last slab, which the other workgroup of a CU hides where two share it and their
-// slabs take as long; the silu of a short SwiGLU launch is as long as its slabs. (Of 680 shapes
-// with K of 64 to 1024 the tile picked is 0.7 % slower than the best one at the geometric mean.
-// With o hidden always 1.6 %, and up to 1.8 times: 1045 x 64 -> 2 x 4864 16.8 us on 64 x 64
+// slabs take as long. SwiGLU: the silu of a short launch is as long as its slabs; in longer
+// ones the tiles that share a CU take 15 % more than the fit (1230 x 896 -> 2 x 4864 33.5 us on
+// 128 x 128 tiles, 29.6 on 256 x 256). Of 680 shapes with K of 64 to 1024 the tile picked is
+// 0.5 % slower than the best one at the geometric mean, of 420 of the models' dimensions 0.4 %.
+// (With o hidden always 1.6 %, and up to 1.8 times: 1045 x 64 -> 2 x 4864 16.8 us on 64 x 64
 // tiles, 10.6 on 192 x 128; 2871 x 64 -> 2 x 10208 52 on 256 x 256, 41 on 128 x 128.) The deep
 // rings (D 3 and 4) carry launches of at most a tile per CU over the latency of the
 // memory-side cache (300 x 3584 -> 4608: 128 x 64 tiles 36.9 us over 2 slabs, 20.1 over 4);
@@ -892,8 +894,9 @@ constexpr TallTile kTallTiles[] = {   // EFM_KNOB_GEMM_TILE 10, 11, ...
 };
 static double tall_cost(const TallTile& t, long tiles, int slabs, bool swiglu) {
     const int cus = prefill_cus();
+    const double sw = swiglu && slabs > 8 && t.occ == 2 ? 1.15 : 1;
     auto slab = [&](double c) {
-        return c <= 1 ? t.s0 + (t.s1 - t.s0) * c : t.s1b + (t.s2 - t.s1b) * (c - 1) / (t.occ - 1);
+        return sw * (c <= 1 ? t.s0 + (t.s1 - t.s0) * c : t.s1b + (t.s2 - t.s1b) * (c - 1) / (t.occ - 1));
     };
     const long rounds = (tiles + cus * t.occ - 1) / (cus * t.occ), last = tiles - (rounds - 1) * cus * t.occ;
     const double o = t.o + (swiglu && slabs <= 8 ? t.tm * t.tn / 32 : 0);
