@@ -535,10 +535,9 @@ def test_lm_head_top1_negative_scores_edges_and_clean_workspace(gpu):
 
 @pytest.mark.parametrize("kind", ["bf16", "swiglu"])
 def test_gemm_tile_shapes_agree_bit_exact(gpu, kind):
-    """The kernel and tile shape follow M: 100 rows run 64 x 64 (SwiGLU 64 x 128), 300
-    rows 128 x 64 (SwiGLU 128 x 128), 1344 rows 128 x 128 (many tiles per XCD: the
-    grouped tile order) and 6144 rows the 256 x 256 wide kernel. Every kernel sums each
-    output over K in the same order, so the first 100 rows must agree bit for bit across
+    """The slab kernel's tile follows M (bf16: 64 x 64 at 100 rows, 128 x 128 at 300, 192 x 256
+    at 1344, 256 x 256 at 6144, with many tiles per XCD in the grouped order). Every tile sums
+    each output over K in the same order, so the first 100 rows must agree bit for bit across
     all launches (and with the oracle on a sample)."""
     torch.manual_seed(17)
     k, n = 1024, 8192
@@ -573,10 +572,9 @@ def test_gemm_tile_shapes_agree_bit_exact(gpu, kind):
     pytest.param(512, 1536, 8960, "swiglu", id="c2_gate_up"),
 ])
 def test_gemm_wide_kernel_matches_narrow_bit_exact(gpu, knob, m, k, n, kind):
-    """The 256 x 256 wide kernel (EFM_KNOB_GEMM_TILE 2) and its 192 x 256 tiles (knob 3:
-    12 A and 16 B blocks per stage over 8 waves) against the 128 x 128 family (knob 1) on
-    aligned and ragged shapes and every epilogue: bit-identical outputs (all sum keys 16
-    at a time in increasing order), and a row sample against the oracle."""
+    """The slab kernel's 256 x 256 (EFM_KNOB_GEMM_TILE 2) and 192 x 256 tiles (knob 3) against
+    its tiles up to 128 x 128 (knob 1) on aligned and ragged shapes and every epilogue:
+    bit-identical outputs, and a row sample against the oracle."""
     torch.manual_seed(m + n)
     x = torch.randn(m, k, dtype=torch.bfloat16, device=gpu)
     nw = 2 * n if kind == "swiglu" else n
@@ -595,8 +593,8 @@ def test_gemm_wide_kernel_matches_narrow_bit_exact(gpu, knob, m, k, n, kind):
         torch.cuda.synchronize()
         outs.append(y)
     for path, y in zip((2, 3), outs[1:]):
-        assert not torch.isnan(y).any(), f"wide kernel (knob {path}) left outputs unwritten"
-        assert torch.equal(outs[0], y), f"{kind}: wide (knob {path}) and narrow kernels differ"
+        assert not torch.isnan(y).any(), f"tile of knob {path} left outputs unwritten"
+        assert torch.equal(outs[0], y), f"{kind}: tiles of knobs {path} and 1 differ"
     rows = torch.tensor([0, m // 2, m - 1])
     xs = x[rows].cpu()
     if kind == "swiglu":
@@ -813,10 +811,9 @@ def test_gemm_k_split_over_waves(gpu, knob, m, k, n, kind, split):
 
 
 def test_gemm_long_k_tiles_agree_bit_exact(gpu):
-    """K = 11008 (the VL-3B down projection) at three M: 100 rows run 64 x 64 tiles, 1344
-    rows (176 tiles of 128 x 128, at most one per CU) 128 x 128 tiles over a 4-deep ring
-    with one workgroup per CU, 2300 rows 128 x 64 tiles over a 3-deep ring. All sum each
-    output over K in the same order: the first 100 rows agree bit for bit, and a row
+    """K = 11008 (the VL-3B down projection) at three M: 64 x 64 tiles at 100 rows, 128 x 128
+    ones over rings of four slabs at 1344 (at most one per CU), 192 x 128 ones at 2300. All sum
+    each output over K in the same order: the first 100 rows agree bit for bit, and a row
     sample of each launch matches the oracle."""
     torch.manual_seed(29)
     k, n = 11008, 2048
@@ -1346,20 +1343,31 @@ def test_attention_prefill_pipelined_matches_register_kernel_c4(gpu, knob, shape
 
 SPLIT_CASES = [
     # hq, hkv, hd, S, L, causal, rope: tile and block edges, one key, one row behind a prefix,
-    # every wave count (8, 4, 2), grids by XCD (1, 2, 4, 8 KV heads) and plain (3)
-    pytest.param(12, 2, 128, 1, 1, 1, "none", id="one_key"),
-    pytest.param(12, 2, 128, 32, 32, 1, "none", id="one_block"),
-    pytest.param(12, 2, 128, 33, 2050, 1, "read", id="eight_waves_rope"),
-    pytest.param(28, 4, 128, 1, 8193, 1, "prerot", id="row_behind_8k"),
-    pytest.param(6, 3, 128, 65, 161, 1, "none", id="plain_grid"),
-    pytest.param(8, 8, 128, 900, 900, 1, "read", id="four_waves_8_kv_heads"),
-    pytest.param(28, 4, 128, 1472, 1475, 1, "prerot", id="two_waves"),
-    pytest.param(12, 2, 128, 130, 97 + 130, 0, "read", id="noncausal_rope"),
-    pytest.param(14, 2, 64, 1, 1, 1, "read", id="hd64_one_key"),
-    pytest.param(14, 2, 64, 31, 95, 1, "none", id="hd64_half_tile"),
-    pytest.param(14, 2, 64, 19, 1531, 1, "prerot", id="hd64_eight_waves"),
-    pytest.param(7, 1, 64, 1200, 1200, 1, "read", id="hd64_four_waves_rope"),
-    pytest.param(16, 8, 64, 97, 128, 0, "none", id="hd64_noncausal"),
+    # grids by XCD (1, 2, 4, 8 KV heads) and plain (3); w8 / w4 / w2: waves per block at 256 CUs
+    # (8 up to half a block per CU, or a block per CU and 1024 keys; 2 past 5 blocks per CU where
+    # nothing is rotated inside)
+    pytest.param(12, 2, 128, 1, 1, 1, "none", id="w8_one_key"),
+    pytest.param(12, 2, 128, 32, 32, 1, "none", id="w8_one_block"),
+    pytest.param(12, 2, 128, 33, 2050, 1, "read", id="w8_rope"),
+    pytest.param(28, 4, 128, 1, 8193, 1, "prerot", id="w8_row_behind_8k"),
+    pytest.param(6, 3, 128, 65, 161, 1, "none", id="w8_plain_grid"),
+    pytest.param(8, 8, 128, 900, 900, 1, "read", id="w4_rope_8_kv_heads"),
+    pytest.param(28, 4, 128, 1472, 1475, 1, "prerot", id="w4_prerot_many_blocks"),
+    pytest.param(28, 4, 128, 1472, 1475, 1, "none", id="w2"),
+    pytest.param(28, 4, 128, 1489, 1600, 0, "none", id="w2_noncausal"),
+    pytest.param(12, 2, 128, 130, 97 + 130, 0, "read", id="w8_noncausal_rope"),
+    pytest.param(12, 2, 128, 509, 509, 1, "none", id="w4"),
+    pytest.param(16, 2, 128, 1343, 1345, 1, "none", id="w4_two_behind"),
+    pytest.param(9, 3, 128, 451, 613, 0, "none", id="w4_plain_grid_noncausal"),
+    pytest.param(12, 2, 128, 400, 613, 0, "prerot", id="w4_noncausal_prerot"),
+    pytest.param(14, 2, 64, 1, 1, 1, "read", id="hd64_w8_one_key"),
+    pytest.param(14, 2, 64, 31, 95, 1, "none", id="hd64_w8_half_tile"),
+    pytest.param(14, 2, 64, 19, 1531, 1, "prerot", id="hd64_w8"),
+    pytest.param(7, 1, 64, 1200, 1200, 1, "read", id="hd64_w4_rope"),
+    pytest.param(16, 8, 64, 97, 128, 0, "none", id="hd64_w8_noncausal"),
+    pytest.param(14, 2, 64, 700, 700, 1, "none", id="hd64_w4"),
+    pytest.param(14, 2, 64, 613, 650, 0, "none", id="hd64_w4_noncausal"),
+    pytest.param(14, 2, 64, 320, 1001, 1, "prerot", id="hd64_w4_behind_prefix"),
 ]
 
 
