@@ -611,8 +611,8 @@ int prefill_cus() {
 // or streams shared tiles. The shared stream reads each K / V byte once per 128 or 256 rows
 // and is the faster one once the chip is full; the split pays while 32-row blocks are few.
 // Measured on 256 CUs (us, split / shared; blocks = 32-row blocks of all heads, keys = mean
-// keys a row sees): 24 blocks x 2018 keys 15.8 / 43.1; 192 x 256 8.9 / 15.6; 672 x 672
-// 22.0 / 30.6; 1020 x 1350 43.8 / 58.0; 752 x 3500 70.0 / 75.1; 896 x 8500 183.9 / 181.6;
+// keys a row sees): 24 blocks x 2018 keys 15.0 / 42.9; 28 x 16 5.1 / 5.1; 192 x 256 8.9 / 15.6; 672 x 672
+// 20.1 / 30.6; 1020 x 1350 43.8 / 58.0; 752 x 3500 70.0 / 75.1; 896 x 8500 183.9 / 181.6;
 // 1536 x 2048 80.6 / 95.5; 1764 x 1000 51.0 / 53.8; 3584 x 2048 170 / 128.
 static bool prefill_split_wins(const PrefillArgs& a, int cus) {
     const long blocks = (long)((a.S + 31) / 32) * a.Hq;
@@ -625,8 +625,8 @@ static bool prefill_split_wins(const PrefillArgs& a, int cus) {
 // Waves per 32-row block: 8 (one workgroup per CU) while there is a CU for every block and
 // the keys are worth it, else 4 (two per CU), and 2 for many blocks where the chain is short
 // (head_dim 128, no RoPE inside: where Q is rotated, 1900 rows of 28 heads behind 100 take
-// 58.8 us on 2 waves, which share that among fewer, 57.5 on 4). Measured (us, 8 / 4 / 2
-// waves): 24 blocks x 2018 keys 15.8 / 19.2 / 33.5; 224 x 8128 50.8 / 65.8 / 124; 192 x 256
+// 58.8 us on 2 waves, which share that among fewer, 57.5 on 4). Measured while every wave still
+// loaded all of Q (us, 8 / 4 / 2 waves): 24 blocks x 2018 keys 15.8 / 19.2 / 33.5; 224 x 8128 50.8 / 65.8 / 124; 192 x 256
 // 9.3 / 8.9 / 11.8; 384 x 512 16.1 / 14.0 / 19.9; 1316 x 750 51.5 / 36.0 / 33.6; head_dim 64,
 // 308 x 350 9.5 / 7.4 / 9.8; RoPE inside, 384 x 524 29.3 / 25.2 / 36.4, 2632 x 5000 730 / 626 /
 // 660.

@@ -13,11 +13,11 @@
 //        quarter of K each over 32 x 32 to 64 x 64 tiles.
 //  * Other K: a register-staged kernel with a padded LDS row pitch (40 bf16).
 //  * Epilogues: bf16 (+bias, the cuBLASLt BIAS epilogue), fp32, and SwiGLU, where the
-//    B tile interleaves 32-row blocks of up and gate weights so that each lane holds u
-//    and g of the same output element: out = bf16(silu(bf16(g)) * bf16(u)).
-//  * Every kernel sums each output's keys 16 at a time in increasing order, so results
-//    are bit-identical across kernels and tile shapes (K-split and split-K aside, which add
-//    the sums of contiguous ranges of K in order).
+//    B tile holds blocks of up and of gate weights so that a lane meets u and g of the same
+//    output element: out = bf16(silu(bf16(g)) * bf16(u)).
+//  * Every kernel sums each output's keys in the same order (the 16 x 16 x 32 MFMA as two of
+//    the 32 x 32 x 16 one), so results are bit-identical across kernels and tile shapes
+//    (K-split and split-K aside, which add the sums of contiguous ranges of K in order).
 #include "common.hpp"
 
 #include <algorithm>

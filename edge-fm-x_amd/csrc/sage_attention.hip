@@ -91,7 +91,8 @@ __global__ __launch_bounds__(kKmeanThreads) void sage_kmean_kernel(const bf16_t*
 // The attention entry point's K mean: workgroup (h, sl) sums rows [sl * per, (sl + 1) *
 // per) of KV head h over every channel, 16 lanes (hd 128) per row, so a wave's 16-byte
 // loads cover four whole 256-byte rows; the quantisation kernel adds the slices (float64:
-// exact, so the mean equals sage_kmean_kernel's bit for bit).
+// exact, so the mean equals sage_kmean_kernel's bit for bit, while the values of a channel
+// span no more than 45 - log2(L) powers of two; beyond, to float64 rounding).
 constexpr int kKSlices = 16;
 __global__ __launch_bounds__(kSageThreads) void sage_kpart_kernel(const bf16_t* k, int L, int k_sn, int k_sh, int hd,
                                                                   double* part) {
@@ -138,8 +139,9 @@ __global__ __launch_bounds__(kSageThreads) void sage_kpart_kernel(const bf16_t* 
 // dst [T][H][hd] int8 (contiguous), scales [blocks][H]. KM = 0: Q (no shift); 1: K with
 // its mean from kmean (sage_kmean_kernel); 2: K with its mean added up here from the
 // kKSlices row-slice sums in kpart (sage_kpart_kernel; block 0 stores it in kmean_out); 3: K
-// with its mean summed here over every row (float64: exact, the same bits), which saves the
-// slices' launch while the rows are few (sage_few_rows).
+// with its mean summed here over every row (float64: the same bits as far as those sums are
+// exact, see sage_kpart_kernel), which saves the slices' launch while the rows are few
+// (sage_few_rows).
 // Every load is issued up front and branch-free (rows past the block's end are buffer
 // loads past the resource: zeros, no memory access), so one round trip covers them all.
 template <int KM>
