@@ -892,8 +892,7 @@ constexpr TallTile kTallTiles[] = {   // EFM_KNOB_GEMM_TILE 10, 11, ...
     {2, 4, 2, 3.6, 0.235, 0.29, 0.75, 0.90},  // 64 x 128, D 3
     {2, 2, 2, 2.7, 0.21, 0.225, 0.38, 0.46},  // 64 x 64, D 4
 };
-static double tall_cost(const TallTile& t, long tiles, int slabs, bool swiglu) {
-    const int cus = prefill_cus();
+static double tall_cost(const TallTile& t, long tiles, int slabs, bool swiglu, int cus) {
     const double sw = swiglu && slabs > 8 && t.occ == 2 ? 1.15 : 1;
     auto slab = [&](double c) {
         return sw * (c <= 1 ? t.s0 + (t.s1 - t.s0) * c : t.s1b + (t.s2 - t.s1b) * (c - 1) / (t.occ - 1));
@@ -939,10 +938,11 @@ static int gemm_dispatch(int M, int N, int K, const bf16_t* A, const bf16_t* B, 
         // the cheapest tile (EFM_KNOB_GEMM_TILE 1: of the tiles up to 128 x 128), or the knob's
         int pick = tile_knob >= 10 ? tile_knob - 10 : tile_knob == 3 ? 1 : 0;
         if (tile_knob < 2) {
+            const int cus = prefill_cus();
             double best = 0;
             for (int i = tile_knob == 1 ? 3 : 0; i < (int)std::size(kTallTiles); ++i) {
                 const double c = tall_cost(kTallTiles[i], tiles(32 * kTallTiles[i].tm, 32 * kTallTiles[i].tn), K / kPBK,
-                                          EPI == GEPI_SWIGLU);
+                                          EPI == GEPI_SWIGLU, cus);
                 if (best == 0 || c < best) best = c, pick = i;
             }
         }
